@@ -204,7 +204,7 @@ OVFQ_API int ovfq_project_dev(ovfq_ctx* ctx, const ovfq_weight* w, const float* 
 
 /* ovfq_project_dev that allocates nothing. No counterpart in the reference: it is for callers that cannot
  * allocate device memory (code under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc).
- * Same arguments, kernels and bit-identical outputs as ovfq_project_dev; where that entry point quantises the
+ * Same arguments and bit-identical outputs as ovfq_project_dev; where that entry point quantises the
  * activation into the context's growable scratch, this one uses a fixed device array of 2.5 MiB that the
  * library holds on every GPU it runs on until the process ends. rows * input_size is limited to 2^21
  * (OVFQ_NOALLOC_MAX_ELEMS; e.g. 512 rows of 4096); larger calls return OVFQ_ERR_SIZE. Every call on one GPU

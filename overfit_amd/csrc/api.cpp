@@ -230,7 +230,8 @@ int weight_create(ovfq_ctx* ctx, int type, const void* blocks, size_t nbytes, co
     w->type = type;
     w->in = in;
     w->out = out;
-    hipError_t e = hipMalloc(&w->blocks, expected);
+    // whole 256-byte pieces: kernels that fetch 16 bytes at a time read up to the end of the last one
+    hipError_t e = hipMalloc(&w->blocks, (expected + 255) & ~size_t(255));
     if (e != hipSuccess) {
         delete w;
         return fail(OVFQ_ERR_HIP, "hipMalloc(%zu) failed: %s", expected, hipGetErrorString(e));
@@ -256,9 +257,21 @@ int weight_create(ovfq_ctx* ctx, int type, const void* blocks, size_t nbytes, co
 }
 
 // Quantises `rows` activation rows of length `in` for weight type `type` into the context scratch.
-int quantize_into_scratch(ovfq_ctx* c, int type, const float* x_dev, int rows, int in, ovfq::ActQ* act) {
+int quantize_into_scratch(ovfq_ctx* c, int type, const float* x_dev, int rows, int in, ovfq::ActQ* act,
+                          bool tiled = false) {
     const size_t n = (size_t)rows * in;
-    int rc = ensure(c, c->act_q, n);
+    int rc;
+    if (tiled) {
+        const size_t recs = (size_t)ovfq::tiled_subs(rows) * (size_t)(in / OVFQ_QK);
+        if ((rc = ensure(c, c->act_q, recs * ovfq::kTiledQ)) || (rc = ensure(c, c->act_s, recs * ovfq::kTiledS)) ||
+            (rc = ensure(c, c->act_b, recs * ovfq::kTiledB)))
+            return rc;
+        *act = ovfq::ActQ{(const int8_t*)c->act_q.p, (const float*)c->act_s.p, nullptr, (const uint16_t*)c->act_b.p, true};
+        HIP_TRY(ovfq::launch_quantize_q8k_tiled(type, x_dev, rows, in, (int8_t*)c->act_q.p, (float*)c->act_s.p,
+                                                (uint16_t*)c->act_b.p, c->stream));
+        return OVFQ_OK;
+    }
+    rc = ensure(c, c->act_q, n);
     if (rc) return rc;
     if (type == OVFQ_TYPE_Q8_0) {
         rc = ensure(c, c->act_s, n / 32 * sizeof(float));
@@ -340,6 +353,27 @@ bool use_gemv_rows(const ovfq_ctx* c, int type, int in, int rows, int count, int
     return rows <= 4 || count >= 3;
 }
 
+// The split-contraction MFMA kernel (mfma_split.hip): batches that the multi-row decode kernel does not take, by the shape
+// rule of split_preferred. It reads operand-ordered activation planes, so the choice is made where the activation is
+// quantised (the callers that quantise here; a caller's own quantised activation keeps the other kernels).
+bool use_split(const ovfq_ctx* c, int in, int rows, const ovfq_weight* const* ws, int count) {
+    const int type = ws[0]->type;
+    if ((type != OVFQ_TYPE_Q4_K && type != OVFQ_TYPE_Q6_K) || rows < 2 || !small_mfma_enabled(3) ||
+        c->batched_kernel != OVFQ_BATCHED_AUTO)
+        return false;
+    const int pair_out = count == 2 && ws[0]->out == ws[1]->out ? ws[0]->out : 0;
+    // The multi-row decode kernel works through a row in items of 16 super-blocks; where the last item is mostly empty
+    // (5120 inputs: 20 of 32) this kernel takes over at 3 rows, and for three or more weights at 2 (MI355X, us, multi-row /
+    // this kernel: 5120x5120 2 rows 9.5 / 10.6, 3 rows 11.2 / 10.7, q/k/v of 5120 inputs 2 rows 13.9 / 12.6, 6 rows 22.4 /
+    // 12.8; q/k/v of 4096 inputs, no empty part, 5 rows 10.2 / 10.8).
+    const int spr = in / OVFQ_QK;
+    const bool short_item = spr > 16 && 2 * ((spr + 15) / 16 * 16) >= 3 * spr;
+    if (use_gemv_rows(c, type, in, rows, count, pair_out) && !(short_item && (rows >= 3 || count >= 3))) return false;
+    long tiles = 0;
+    for (int i = 0; i < count; i++) tiles += (ws[i]->out + 15) / 16;
+    return ovfq::split_preferred(type, in, rows, tiles);
+}
+
 // Whether the projection launch quantises its fp32 input itself instead of a separate Q8_K / Q8_0 launch: one row on
 // a decode kernel (K <= 8192), or up to 64 super-blocks of rows on the multi-row decode kernel.
 bool quantize_in_launch(const ovfq_ctx* c, int type, int in, int rows, int count, int pair_out = 0) {
@@ -368,7 +402,9 @@ int launch_projection(ovfq_ctx* c, const ovfq_weight* const* ws, int count, cons
         return fail(OVFQ_ERR_SIZE, "in-launch quantisation of %d rows needs the multi-row decode kernel", rows);
     // Every kernel below reads either the fp32 input (decode kernels that quantise it) or the quantised activation.
     if (!x && (!act.q || !act.s)) return fail(OVFQ_ERR_NULL, "projection launch without a quantised activation");
-    if (type == OVFQ_TYPE_Q8_0) {
+    if (act.tiled) {
+        HIP_TRY(ovfq::launch_project_split(type, jobs, count, in, rows, act, c->stream));
+    } else if (type == OVFQ_TYPE_Q8_0) {
         // The int8-MFMA kernel from 8 rows; for inputs up to 8192 from 6 rows, and from 4 rows for 8192 outputs or
         // more. Its time is flat up to 16 rows (one 16-row tile, one-wave workgroups of 16 outputs), the row
         // kernel's grows by a pass over the weights per row (MI355X, graph replay, us, row kernel / MFMA kernel):
@@ -974,14 +1010,15 @@ static int project_impl(ovfq_ctx* ctx, int count, const ovfq_weight* const* ws, 
             bd[i] = biases ? biases[i] : nullptr;
         }
     }
-    if (quantize_in_launch(ctx, ws[0]->type, in, rows, count,
-                           count == 2 && ws[0]->out == ws[1]->out ? ws[0]->out : 0)) {
+    const bool split = use_split(ctx, in, rows, ws, count);
+    if (!split && quantize_in_launch(ctx, ws[0]->type, in, rows, count,
+                                     count == 2 && ws[0]->out == ws[1]->out ? ws[0]->out : 0)) {
         // Decode: the Q8_K quantisation happens inside the projection launch.
         if ((rc = launch_projection(ctx, ws, count, bd, yd, rows, ovfq::ActQ{nullptr, nullptr, nullptr}, xd)))
             return rc;
     } else {
         ovfq::ActQ act;
-        if ((rc = quantize_into_scratch(ctx, ws[0]->type, xd, rows, in, &act))) return rc;
+        if ((rc = quantize_into_scratch(ctx, ws[0]->type, xd, rows, in, &act, split))) return rc;
         if ((rc = launch_projection(ctx, ws, count, bd, yd, rows, act))) return rc;
     }
     if (host) {
@@ -1523,12 +1560,16 @@ static int ffn_impl(ovfq_ctx* ctx, const ovfq_weight* gate, const ovfq_weight* u
     std::lock_guard<std::mutex> lk(ctx->mu);
     HIP_TRY(hipSetDevice(ctx->device));
     const size_t R = (size_t)rows;
+    const ovfq_weight* dw[1] = {down};
+    // the intermediate in the order that the down projection's kernel reads
+    const bool down_split = use_split(ctx, dff, rows, dw, 1);
+    const size_t recs = (size_t)ovfq::tiled_subs(rows) * (size_t)(dff / OVFQ_QK);
     auto carve = [&](Carver& c, float** g, float** u, int8_t** iq, float** is, int16_t** ib, float** hx, float** hy) {
         *g = c.take<float>(R * dff * 4);
         *u = c.take<float>(R * dff * 4);
-        *iq = c.take<int8_t>(R * dff);
-        *is = c.take<float>(R * (dff / OVFQ_QK) * 4);
-        *ib = c.take<int16_t>(R * (dff / 16) * 2);
+        *iq = c.take<int8_t>(down_split ? recs * ovfq::kTiledQ : R * dff);
+        *is = c.take<float>(down_split ? recs * ovfq::kTiledS : R * (dff / OVFQ_QK) * 4);
+        *ib = c.take<int16_t>(down_split ? recs * ovfq::kTiledB : R * (dff / 16) * 2);
         if (host) {
             *hx = c.take<float>(R * dmodel * 4);
             *hy = c.take<float>(R * dmodel * 4);
@@ -1558,15 +1599,16 @@ static int ffn_impl(ovfq_ctx* ctx, const ovfq_weight* gate, const ovfq_weight* u
             return rc;
     } else {
         ovfq::ActQ act;
-        if ((rc = quantize_into_scratch(ctx, gate->type, xd, rows, dmodel, &act))) return rc;
+        if ((rc = quantize_into_scratch(ctx, gate->type, xd, rows, dmodel, &act, use_split(ctx, dmodel, rows, gu, 2))))
+            return rc;
         if ((rc = launch_projection(ctx, gu, 2, nullptr, gu_out, rows, act))) return rc;
     }
     // act(gate) * up, quantised to Q8_K for the down projection
     HIP_TRY(ovfq::launch_gate_up_q8k(g, u, nullptr, 0, rows, dff, activation == OVFQ_FFN_GEGLU, iq, is, ib,
-                                     ctx->stream));
-    const ovfq_weight* dw[1] = {down};
+                                     ctx->stream, ovfq::MoeFold{}, down_split ? down->type : 0, (uint16_t*)ib));
     float* dy[1] = {yd};
-    if ((rc = launch_projection(ctx, dw, 1, nullptr, dy, rows, ovfq::ActQ{iq, is, ib}))) return rc;
+    const ovfq::ActQ mid = down_split ? ovfq::ActQ{iq, is, nullptr, (const uint16_t*)ib, true} : ovfq::ActQ{iq, is, ib};
+    if ((rc = launch_projection(ctx, dw, 1, nullptr, dy, rows, mid))) return rc;
     if (host && ((rc = io.down(y, yd, R * dmodel * 4)) || (rc = io.finish()))) return rc;
     return ok();
 }

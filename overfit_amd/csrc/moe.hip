@@ -335,7 +335,7 @@ __global__ __launch_bounds__(256) void gate_up_q8k_kernel(const float* __restric
                                                          const int* __restrict__ expert_off, int n_experts,
                                                          int max_pairs, int spr, int8_t* __restrict__ q,
                                                          float* __restrict__ s, int16_t* __restrict__ bs,
-                                                         const MoeFold fold) {
+                                                         uint16_t* __restrict__ bh, int tiled, const MoeFold fold) {
     {
         const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
         for (int64_t j = i * 4; j < fold.y_len && j < i * 4 + 4; j++) fold.y[j] = 0.0f;
@@ -372,6 +372,18 @@ __global__ __launch_bounds__(256) void gate_up_q8k_kernel(const float* __restric
     }
     const Q8KLane r = q8k_quantize_wave(v[0], v[1], v[2], v[3]);
     if (!live) return;
+    if (tiled) {  // operand-ordered planes for a down weight of type `tiled` (quantize_q8k_tiled_kernel's layout)
+        const int64_t row = blk / spr;
+        const size_t rec = (size_t)(row >> 4) * spr + (size_t)(blk - row * spr);
+        const int r16 = (int)(row & 15), p = lane >> 2;
+        const int slot = tiled_slot(p, tiled == 14);
+        *reinterpret_cast<uint32_t*>(q + rec * kTiledQ + slot * 256 + r16 * 16 + (lane & 3) * 4) = r.packed;
+        if (tiled == 12 && (lane & 3) == 0)
+            bh[(rec * kTiledB + (p >> 2) * 128 + r16 * 8) / 2 + (p & 3)] =
+                __builtin_bit_cast(uint16_t, (_Float16)r.group_sum);
+        if (lane == 0) s[rec * (kTiledS / 4) + r16] = r.scale;
+        return;
+    }
     reinterpret_cast<uint32_t*>(q + blk * kQK)[lane] = r.packed;
     if ((lane & 3) == 0) bs[blk * 16 + (lane >> 2)] = (int16_t)r.group_sum;
     if (lane == 0) s[blk] = r.scale;
@@ -479,17 +491,17 @@ hipError_t launch_moe_plan(const int* idx, int rows, int k, int n_experts, int* 
 
 hipError_t launch_gate_up_q8k(const float* gate, const float* up, const int* expert_off, int n_experts, int max_pairs,
                               int dff, bool gelu, int8_t* q, float* s, int16_t* b, hipStream_t st,
-                              const MoeFold& fold) {
+                              const MoeFold& fold, int tiled, uint16_t* bh) {
     const int spr = dff / kQK;
     const int64_t waves = (int64_t)max_pairs * spr;
     const int64_t fold_threads = std::max<int64_t>((fold.y_len + 3) / 4, fold.slots);
     const dim3 grid((unsigned)std::max((waves + 3) / 4, (fold_threads + 255) / 256)), block(256);
     if (gelu)
         hipLaunchKernelGGL(gate_up_q8k_kernel<true>, grid, block, 0, st, gate, up, expert_off, n_experts, max_pairs, spr,
-                           q, s, b, fold);
+                           q, s, b, bh, tiled, fold);
     else
         hipLaunchKernelGGL(gate_up_q8k_kernel<false>, grid, block, 0, st, gate, up, expert_off, n_experts, max_pairs,
-                           spr, q, s, b, fold);
+                           spr, q, s, b, bh, tiled, fold);
     return hipGetLastError();
 }
 

@@ -220,4 +220,12 @@ __device__ __forceinline__ Q8KRow q8k_quantize_row16(const float (&x)[16]) {
     return r;
 }
 
+// Slot 4 t + g of the operand-ordered activation that holds 16-byte piece p of a super-block: the inverse of
+// Q4KMfma::src_piece (p has bits [t & 1, g >> 1, t >> 1, g & 1]) and Q6KMfma::src_piece ([g >> 1, t, t, g & 1]).
+__device__ __forceinline__ int tiled_slot(int p, bool q6) {
+    const int t = q6 ? (p >> 1) & 3 : (p >> 3) | (p & 2);
+    const int g = q6 ? ((p >> 2) & 2) | (p & 1) : ((p >> 1) & 2) | (p & 1);
+    return 4 * t + g;
+}
+
 }  // namespace ovfq

@@ -25,11 +25,19 @@ struct ActQ {
     const float* s;
     const int16_t* b;
     const uint16_t* bh = nullptr;  // the bsums again as fp16 (the quantiser's optional second plane), or NULL
+    bool tiled = false;            // operand-ordered planes (launch_quantize_q8k_tiled): q, s and bh, no b
 };
 
 // bh != NULL: the bsums are also written as fp16 (exact: |bsum| <= 16 * 127), the tiled Q4_K kernels' min-term operand.
 hipError_t launch_quantize_q8k(const float* x, int64_t n_blocks, int8_t* q, float* s, int16_t* b, hipStream_t st,
                                uint16_t* bh = nullptr);
+// Q8_K quantisation into the operand-ordered planes that launch_project_split reads for weights of `type` (12 or 14):
+// for every 16 rows and super-block, kTiledQ bytes of quants, kTiledB bytes of fp16 bsums and kTiledS bytes of scales.
+// Planes cover 16 * tiled_subs(rows) rows; the rows past `rows` are not written.
+constexpr size_t kTiledQ = 4096, kTiledB = 512, kTiledS = 64;
+inline int64_t tiled_subs(int64_t rows) { return (rows + 15) / 16; }
+hipError_t launch_quantize_q8k_tiled(int type, const float* x, int rows, int in, int8_t* q, float* s, uint16_t* bh,
+                                     hipStream_t st);
 hipError_t launch_quantize_q8_0(const float* x, int64_t n_blocks, int8_t* q, float* s, hipStream_t st);
 
 // type: 12 (Q4_K) or 14 (Q6_K). `in` % 256 == 0. rows = activation rows (M).
@@ -58,6 +66,12 @@ bool mfma_tiled_preferred(int type, int rows, int o_tiles, long out_rows);
 constexpr int kMfmaMinRows = 32;
 hipError_t launch_project_mfma(int type, const ProjJob* jobs, int njobs, int in, int rows, ActQ act,
                                hipStream_t st);
+// Batched K-quant projection with the contraction split over the waves of a workgroup (mfma_split.hip), any rows and K,
+// from operand-ordered planes (act.tiled); bit-identical to launch_project_kquant. split_preferred: the automatic choice of
+// that kernel for `rows` activation rows against weights of `tiles` 16-row tiles in all.
+bool split_preferred(int type, int in, int rows, long tiles);
+hipError_t launch_project_split(int type, const ProjJob* jobs, int njobs, int in, int rows, ActQ act,
+                                hipStream_t st);
 // Small-batch / grouped-expert K-quant projection. One or two matrices per expert (gate, up) of equal shape;
 // expert_off/pair_row (device arrays) select each expert's activation rows, or NULL for a single expert over
 // activation rows 0..rows-1 (outputs row-major [pairs][n_rows]).
@@ -125,10 +139,12 @@ struct MoeFold {
     int slots = 0;
     float* pw = nullptr;
 };
-// act(gate) * up (act: SiLU, or GELU with the tanh approximation), quantised to Q8_K for the down projection.
+// act(gate) * up (act: SiLU, or GELU with the tanh approximation), quantised to Q8_K for the down projection: row-major
+// planes, or, tiled = 12 / 14, the operand-ordered planes of launch_project_split for a down weight of that type (q, s,
+// bh; not with expert_off).
 hipError_t launch_gate_up_q8k(const float* gate, const float* up, const int* expert_off, int n_experts, int max_pairs,
                               int dff, bool gelu, int8_t* q, float* s, int16_t* b, hipStream_t st,
-                              const MoeFold& fold = MoeFold{});
+                              const MoeFold& fold = MoeFold{}, int tiled = 0, uint16_t* bh = nullptr);
 hipError_t launch_moe_combine(const float* out, const int* pair_of, const float* w, int rows, int k, int dmodel,
                               float* y, hipStream_t st);
 

@@ -44,6 +44,42 @@ __global__ __launch_bounds__(256) void quantize_q8k_kernel(const float* __restri
     }
 }
 
+// The same quantisation into operand-ordered planes (launch_quantize_q8k_tiled): the 16-byte piece that lane (g, r16) of
+// MFMA t reads goes to byte 1024 t + 256 g + 16 r16 of its (16 rows, super-block) record, so that a wave loads an A operand
+// as one contiguous KiB. Piece p of a super-block (elements 16 p ..) belongs to the (t, g) with src_piece(4 t + g) == p of
+// the weight format's operand order (Q4KMfma / Q6KMfma). Lane (g, r16) of the min MFMA reads bsums 4 g .. 4 g + 3.
+__global__ __launch_bounds__(256) void quantize_q8k_tiled_kernel(const float* __restrict__ x, int64_t n_blocks, int spr,
+                                                                 int q6, uint8_t* __restrict__ q,
+                                                                 uint8_t* __restrict__ s, uint8_t* __restrict__ bh) {
+    const int64_t blk0 = ((int64_t)blockIdx.x * 4 + wave_id()) * 4;
+    if (blk0 >= n_blocks) return;
+    const int lane = threadIdx.x & 63, p = lane & 15;
+    const int64_t blk = blk0 + (lane >> 4);
+    const __amdgpu_buffer_rsrc_t xr =
+        make_rsrc(x + blk0 * kQK, rsrc_bytes((uint64_t)n_blocks * kQK * 4, (uint64_t)blk0 * kQK * 4));
+    float v[16];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const u32x4 t = ld4(xr, (uint32_t)lane * 64u + (uint32_t)i * 16u);
+        v[4 * i] = as_float(t.x);
+        v[4 * i + 1] = as_float(t.y);
+        v[4 * i + 2] = as_float(t.z);
+        v[4 * i + 3] = as_float(t.w);
+    }
+    const Q8KRow r = q8k_quantize_row16(v);
+    if (blk < n_blocks) {
+        const int64_t row = blk / spr;
+        const size_t rec = (size_t)(row >> 4) * spr + (size_t)(blk - row * spr);
+        const int r16 = (int)(row & 15);
+        const int slot = tiled_slot(p, q6 != 0);  // 4 t + g
+        *reinterpret_cast<u32x4*>(q + rec * kTiledQ + slot * 256 + r16 * 16) = r.packed;
+        if (bh)
+            *reinterpret_cast<_Float16*>(bh + rec * kTiledB + (p >> 2) * 128 + r16 * 8 + (p & 3) * 2) =
+                (_Float16)r.group_sum;
+        if (p == 0) *reinterpret_cast<float*>(s + rec * kTiledS + r16 * 4) = r.scale;
+    }
+}
+
 // ------------------------------------------------------------------------------------------ Q8_0 activation
 // Q8DotKernel.Quantize (RT/Q8DotKernel.cs:42-91): 32-element blocks, eight lanes per block.
 __global__ __launch_bounds__(256) void quantize_q8_0_kernel(const float* __restrict__ x, int64_t n_blocks,
@@ -346,6 +382,15 @@ hipError_t launch_quantize_q8k(const float* x, int64_t n_blocks, int8_t* q, floa
     if (n_blocks <= 0) return hipSuccess;
     const int64_t grid = (n_blocks + 15) / 16;
     hipLaunchKernelGGL(quantize_q8k_kernel, dim3((unsigned)grid), dim3(256), 0, st, x, n_blocks, q, s, b, bh);
+    return hipGetLastError();
+}
+
+hipError_t launch_quantize_q8k_tiled(int type, const float* x, int rows, int in, int8_t* q, float* s, uint16_t* bh,
+                                     hipStream_t st) {
+    const int64_t n_blocks = (int64_t)rows * (in / kQK);
+    hipLaunchKernelGGL(quantize_q8k_tiled_kernel, dim3((unsigned)((n_blocks + 15) / 16)), dim3(256), 0, st, x, n_blocks,
+                       in / kQK, type == 14 ? 1 : 0, reinterpret_cast<uint8_t*>(q), reinterpret_cast<uint8_t*>(s),
+                       type == 12 ? reinterpret_cast<uint8_t*>(bh) : nullptr);
     return hipGetLastError();
 }
 

@@ -1,0 +1,104 @@
+"""The split-contraction MFMA kernel (mfma_split.hip) against the oracle, bit for bit: every output is an exact integer
+dot per super-block and the reference's fp32 sum over the row (RT/Q4KDotKernel.cs:944-951, RT/Q6KDotKernel.cs:114-115).
+
+It takes batches whose activation is quantised by the call, by a rule on rows and shapes; the shapes here lie on both
+sides of its tile edges: 3 .. 130 rows around multiples of 16 and 64, output counts off the 16-row tiles, one
+super-block to one more than the small-M kernel takes, four and eight waves, odd Q6_K super-block counts (rows that start
+2, 4, .. 14 bytes past a 16-byte boundary), a last block that ends inside a 16-byte piece.
+"""
+import sys
+
+import numpy as np
+import pytest
+
+from qdata import normal, random_q4k_blocks, random_q6k_blocks, set_subnormal_scales
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+ov = pytest.importorskip("overfit_amd")
+
+DEV = "cuda:0"
+
+
+def case(*what):
+    print("[case]", *what, flush=True, file=sys.stderr)
+
+
+def t(a):
+    return torch.from_numpy(np.ascontiguousarray(a)).to(DEV)
+
+
+def _weight(rng, fmt, n, k):
+    nb = n * (k // 256)
+    if fmt == "q4k":
+        blocks = set_subnormal_scales(random_q4k_blocks(rng, nb))
+        return blocks, ov.Q4KWeight(blocks.reshape(-1), k, n)
+    blocks = set_subnormal_scales(random_q6k_blocks(rng, nb), q6=True)
+    return blocks, ov.Q6KWeight(blocks.reshape(-1), k, n)
+
+
+def _check(y, ref, what):
+    y = y.cpu().numpy().reshape(ref.shape)
+    bad = int(np.count_nonzero(y.view(np.uint32) != ref.view(np.uint32)))
+    assert bad == 0, f"{what}: {bad}/{y.size} outputs differ from the oracle"
+
+
+def _ref(orc, fmt, x, rows, blocks, k, n, bias):
+    return (orc.q4k_project_batched if fmt == "q4k" else orc.q6k_project_batched)(x, rows, blocks, k, n, bias)
+
+
+@pytest.mark.parametrize("fmt", ["q4k", "q6k"])
+@pytest.mark.parametrize("rows,k,n", [
+    (9, 256, 33),      # one super-block: three of four waves idle
+    (3, 16640, 17),    # past the small-M kernel's inputs, from 3 rows; an incomplete last round of eight waves
+    (5, 4352, 250),    # 17 super-blocks
+    (16, 2048, 48),    # exactly one tile, one round of eight waves
+    (17, 1792, 65),    # two tiles, four waves
+    (33, 2304, 97),    # three tiles, two rounds
+    (64, 2560, 16),    # four tiles
+    (65, 3328, 31),    # two workgroups of three tiles, the last rows of the second absent
+    (130, 768, 1000),  # nine tiles over three workgroups, four waves with one idle
+])
+def test_split_projection_bit_exact(orc, fmt, rows, k, n):
+    case("split", fmt, rows, k, n)
+    rng = np.random.default_rng(rows * 7919 + k + n)
+    blocks, w = _weight(rng, fmt, n, k)
+    x, bias = normal(rng, (rows, k)), normal(rng, n)
+    _check(ov.project(w, t(x), t(bias), rows=rows), _ref(orc, fmt, x, rows, blocks, k, n, bias), "bias")
+    _check(ov.project(w, t(x), rows=rows), _ref(orc, fmt, x, rows, blocks, k, n, None), "no bias")
+
+
+@pytest.mark.parametrize("rows,k,shapes", [(2, 4352, [128, 48, 50]), (40, 1024, [256, 64, 70, 16])])
+def test_split_fused_projections_bit_exact(orc, rows, k, shapes):
+    """Several weights in one launch, none a multiple of the tile (2 rows of 17 super-blocks: the launch that the multi-row
+    decode kernel's mostly empty last item would slow down)."""
+    case("split fused", rows, k, shapes)
+    rng = np.random.default_rng(rows + k)
+    made = [_weight(rng, "q4k", n, k) for n in shapes]
+    x = normal(rng, (rows, k))
+    bias = normal(rng, shapes[1])
+    ys = ov.project_multi([w for _, w in made], t(x), rows=rows,
+                          biases=[t(bias) if i == 1 else None for i in range(len(shapes))])
+    for i, (y, (blocks, _)) in enumerate(zip(ys, made)):
+        _check(y, _ref(orc, "q4k", x, rows, blocks, k, shapes[i], bias if i == 1 else None), f"job {i}")
+
+
+@pytest.mark.parametrize("down", ["q4k", "q6k"])
+def test_split_ffn_intermediate_matches_separate_calls(down):
+    """The FFN's intermediate, quantised in the down kernel's operand order, against the same FFN with another kernel
+    forced, which reads it row by row: the same quants, so the same bits (35 rows, 9 super-blocks)."""
+    case("split ffn", down)
+    rng = np.random.default_rng(5)
+    d, ff, rows = 512, 2304, 35
+    gate, up = _weight(rng, "q4k", ff, d)[1], _weight(rng, "q4k", ff, d)[1]
+    w = _weight(rng, down, d, ff)[1]
+    x = t(normal(rng, (rows, d), 0.02))
+    y = ov.ffn_swiglu(gate, up, w, x, rows)
+    ctx = ov.default_context()
+    ctx.set_batched_kernel("tiled")
+    try:
+        ref = ov.ffn_swiglu(gate, up, w, x, rows)
+    finally:
+        ctx.set_batched_kernel("auto")
+    assert torch.equal(y.view(torch.int32), ref.view(torch.int32))
