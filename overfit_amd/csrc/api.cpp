@@ -353,25 +353,28 @@ bool use_gemv_rows(const ovfq_ctx* c, int type, int in, int rows, int count, int
     return rows <= 4 || count >= 3;
 }
 
-// The split-contraction MFMA kernel (mfma_split.hip): batches that the multi-row decode kernel does not take, by the shape
-// rule of split_preferred. It reads operand-ordered activation planes, so the choice is made where the activation is
+// The split or the panel kernel (mfma_split.hip) for batches that the multi-row decode kernel does not take, by the shape
+// rule of mid_kernel. They read operand-ordered activation planes, so the choice is made where the activation is
 // quantised (the callers that quantise here; a caller's own quantised activation keeps the other kernels).
-bool use_split(const ovfq_ctx* c, int in, int rows, const ovfq_weight* const* ws, int count) {
+ovfq::MidKernel use_mid(const ovfq_ctx* c, int in, int rows, const ovfq_weight* const* ws, int count) {
     const int type = ws[0]->type;
     if ((type != OVFQ_TYPE_Q4_K && type != OVFQ_TYPE_Q6_K) || rows < 2 || !small_mfma_enabled(3) ||
         c->batched_kernel != OVFQ_BATCHED_AUTO)
-        return false;
+        return ovfq::MidKernel::kNone;
     const int pair_out = count == 2 && ws[0]->out == ws[1]->out ? ws[0]->out : 0;
-    // The multi-row decode kernel works through a row in items of 16 super-blocks; where the last item is mostly empty
-    // (5120 inputs: 20 of 32) this kernel takes over at 3 rows, and for three or more weights at 2 (MI355X, us, multi-row /
-    // this kernel: 5120x5120 2 rows 9.5 / 10.6, 3 rows 11.2 / 10.7, q/k/v of 5120 inputs 2 rows 13.9 / 12.6, 6 rows 22.4 /
-    // 12.8; q/k/v of 4096 inputs, no empty part, 5 rows 10.2 / 10.8).
-    const int spr = in / OVFQ_QK;
-    const bool short_item = spr > 16 && 2 * ((spr + 15) / 16 * 16) >= 3 * spr;
-    if (use_gemv_rows(c, type, in, rows, count, pair_out) && !(short_item && (rows >= 3 || count >= 3))) return false;
     long tiles = 0;
     for (int i = 0; i < count; i++) tiles += (ws[i]->out + 15) / 16;
-    return ovfq::split_preferred(type, in, rows, tiles);
+    // The multi-row decode kernel works through a row in items of 16 super-blocks; where the last item is mostly empty
+    // (5120 inputs: 20 of 32) these kernels take over at 3 rows, and for three or more weights at 2 (MI355X, us, multi-row /
+    // split kernel: 5120x5120 2 rows 9.5 / 10.6, 3 rows 11.2 / 10.7, q/k/v of 5120 inputs 2 rows 13.9 / 12.6, 6 rows 22.4 /
+    // 12.8; q/k/v of 4096 inputs, no empty part, 5 rows 10.2 / 10.8). It also loses on one very tall matrix (128256x2048 at 3
+    // rows 64.9, panel kernel 39.1).
+    const int spr = in / OVFQ_QK;
+    const bool short_item = spr > 16 && 2 * ((spr + 15) / 16 * 16) >= 3 * spr;
+    if (use_gemv_rows(c, type, in, rows, count, pair_out) && !(short_item && (rows >= 3 || count >= 3)) &&
+        !(rows >= 3 && count == 1 && tiles >= 1536))
+        return ovfq::MidKernel::kNone;
+    return ovfq::mid_kernel(type, in, rows, tiles, count);
 }
 
 // Whether the projection launch quantises its fp32 input itself instead of a separate Q8_K / Q8_0 launch: one row on
@@ -403,7 +406,10 @@ int launch_projection(ovfq_ctx* c, const ovfq_weight* const* ws, int count, cons
     // Every kernel below reads either the fp32 input (decode kernels that quantise it) or the quantised activation.
     if (!x && (!act.q || !act.s)) return fail(OVFQ_ERR_NULL, "projection launch without a quantised activation");
     if (act.tiled) {
-        HIP_TRY(ovfq::launch_project_split(type, jobs, count, in, rows, act, c->stream));
+        if (use_mid(c, in, rows, ws, count) == ovfq::MidKernel::kPanel)
+            HIP_TRY(ovfq::launch_project_panel(type, jobs, count, in, rows, act, c->stream));
+        else
+            HIP_TRY(ovfq::launch_project_split(type, jobs, count, in, rows, act, c->stream));
     } else if (type == OVFQ_TYPE_Q8_0) {
         // The int8-MFMA kernel from 8 rows; for inputs up to 8192 from 6 rows, and from 4 rows for 8192 outputs or
         // more. Its time is flat up to 16 rows (one 16-row tile, one-wave workgroups of 16 outputs), the row
@@ -1010,15 +1016,15 @@ static int project_impl(ovfq_ctx* ctx, int count, const ovfq_weight* const* ws, 
             bd[i] = biases ? biases[i] : nullptr;
         }
     }
-    const bool split = use_split(ctx, in, rows, ws, count);
-    if (!split && quantize_in_launch(ctx, ws[0]->type, in, rows, count,
+    const bool tiled = use_mid(ctx, in, rows, ws, count) != ovfq::MidKernel::kNone;
+    if (!tiled && quantize_in_launch(ctx, ws[0]->type, in, rows, count,
                                      count == 2 && ws[0]->out == ws[1]->out ? ws[0]->out : 0)) {
         // Decode: the Q8_K quantisation happens inside the projection launch.
         if ((rc = launch_projection(ctx, ws, count, bd, yd, rows, ovfq::ActQ{nullptr, nullptr, nullptr}, xd)))
             return rc;
     } else {
         ovfq::ActQ act;
-        if ((rc = quantize_into_scratch(ctx, ws[0]->type, xd, rows, in, &act, split))) return rc;
+        if ((rc = quantize_into_scratch(ctx, ws[0]->type, xd, rows, in, &act, tiled))) return rc;
         if ((rc = launch_projection(ctx, ws, count, bd, yd, rows, act))) return rc;
     }
     if (host) {
@@ -1384,31 +1390,34 @@ static int moe_impl(ovfq_ctx* ctx, int E, const ovfq_weight* const* gate, const 
     std::lock_guard<std::mutex> lk(ctx->mu);
     HIP_TRY(hipSetDevice(ctx->device));
     // scratch layout (sizes first, then the pointers into one buffer)
-    // Many pairs per expert: the batched int8-MFMA kernel over expert groups (64-row tiles, operand build amortised
-    // over the tile); few: the small-M kernel (16-row tiles, super-block-parallel waves). Measured on MI355X with 8
-    // Mixtral-shaped experts, top-2: small-M wins at 8 pairs per expert on average (304 vs 352 us), the grouped
-    // kernel from 12 (354 vs 365 us; 64 tokens 362 vs 469 us).
+    // Many pairs per expert: the panel kernel over expert groups (each weight read once per 64 pairs); few: the
+    // expert-stream or small-M kernel (once per 16). Measured on MI355X, us, top-2 of 8 experts, stream / panel: 4096x14336
+    // experts with 12 pairs each on average 204 / 239, 16 pairs 276 / 256; 2048x4096 experts with Q6_K down 12 pairs 58 /
+    // 70, 16 pairs 82 / 76 (some experts then have more than 16, and the stream reads their weights twice).
     static const int grouped_min = [] {
         const char* v = getenv("OVFQ_MOE_GROUPED_MIN_PAIRS");
-        return v && *v ? atoi(v) : 12;
+        return v && *v ? atoi(v) : 16;
     }();
     // the small-M kernel keeps a row's block values in LDS (d_model, d_ff <= 16384); past that, always grouped
     const bool small_ok = ovfq::mfma_small_supported(gt, dmodel) && ovfq::mfma_small_supported(dt, dff);
     const bool grouped_big = !small_ok || ctx->batched_kernel == OVFQ_BATCHED_TILED ||
                              (ctx->batched_kernel == OVFQ_BATCHED_AUTO && P >= (size_t)grouped_min * E);
     const int max_tiles = (int)((P + ovfq::kGroupedTileRows - 1) / ovfq::kGroupedTileRows) + E;
-    auto carve = [&](Carver& c, int** off, int** prow, int** pof, float** pw, float** g, float** u, int8_t** iq,
+    // grouped_big: the intermediate in operand-ordered planes, every expert's pairs from a 16-row tile of their own on
+    const size_t i_recs = (size_t)ovfq::grouped_subs((int)P, E) * (size_t)(dff / OVFQ_QK);
+    auto carve = [&](Carver& c, int** off, int** prow, int** pof, int** pdst, float** pw, float** g, float** u, int8_t** iq,
                      float** is, int16_t** ib, float** out, float** hx, int** hidx, float** hw, float** hy,
                      float** hl) {
         *off = c.take<int>((size_t)(E + 2 + max_tiles) * 4);  // expert_off[E + 1], tile count, tile list
         *prow = c.take<int>(P * 4);
         *pof = c.take<int>(P * 4);
+        *pdst = c.take<int>(grouped_big ? P * 4 : 0);
         *pw = c.take<float>(P * 4);
         *g = c.take<float>(P * dff * 4);
         *u = c.take<float>(P * dff * 4);
-        *iq = c.take<int8_t>(P * dff);
-        *is = c.take<float>(P * (dff / OVFQ_QK) * 4);
-        *ib = c.take<int16_t>(P * (dff / 16) * 2);
+        *iq = c.take<int8_t>(grouped_big ? i_recs * ovfq::kTiledQ : P * dff);
+        *is = c.take<float>(grouped_big ? i_recs * ovfq::kTiledS : P * (dff / OVFQ_QK) * 4);
+        *ib = c.take<int16_t>(grouped_big ? i_recs * ovfq::kTiledB : P * (dff / 16) * 2);
         *out = c.take<float>(P * dmodel * 4);
         if (host) {
             *hx = c.take<float>((size_t)rows * dmodel * 4);
@@ -1418,15 +1427,15 @@ static int moe_impl(ovfq_ctx* ctx, int E, const ovfq_weight* const* gate, const 
             if (route) *hl = c.take<float>((size_t)rows * E * 4);
         }
     };
-    int *off, *prow, *pof, *hidx = nullptr;
+    int *off, *prow, *pof, *pdst, *hidx = nullptr;
     float *pw, *g, *u, *is, *out, *hx = nullptr, *hw = nullptr, *hy = nullptr, *hl = nullptr;
     int8_t* iq;
     int16_t* ib;
     Carver sizing{nullptr};
-    carve(sizing, &off, &prow, &pof, &pw, &g, &u, &iq, &is, &ib, &out, &hx, &hidx, &hw, &hy, &hl);
+    carve(sizing, &off, &prow, &pof, &pdst, &pw, &g, &u, &iq, &is, &ib, &out, &hx, &hidx, &hw, &hy, &hl);
     if ((rc = ensure(ctx, ctx->moe, sizing.used))) return rc;
     Carver c{static_cast<char*>(ctx->moe.p)};
-    carve(c, &off, &prow, &pof, &pw, &g, &u, &iq, &is, &ib, &out, &hx, &hidx, &hw, &hy, &hl);
+    carve(c, &off, &prow, &pof, &pdst, &pw, &g, &u, &iq, &is, &ib, &out, &hx, &hidx, &hw, &hy, &hl);
     const float* xd = x;
     const float* ld = logits;
     int* idxd = const_cast<int*>(idx);  // written only when routing here (then the caller's output)
@@ -1446,24 +1455,26 @@ static int moe_impl(ovfq_ctx* ctx, int E, const ovfq_weight* const* gate, const 
         wd = hw;
         yd = hy;
     }
-    // the grouping plan and the Q8_K quantisation of x share one launch (neither depends on the other)
+    // the grouping plan and the Q8_K quantisation of x share one launch (neither depends on the other); the panel kernel
+    // takes the bsums as fp16
     const size_t n_x = (size_t)rows * dmodel;
     if ((rc = ensure(ctx, ctx->act_q, n_x)) || (rc = ensure(ctx, ctx->act_s, n_x / OVFQ_QK * sizeof(float))) ||
         (rc = ensure(ctx, ctx->act_b, n_x / 16 * sizeof(int16_t))))
         return rc;
-    const ovfq::ActQ act{(const int8_t*)ctx->act_q.p, (const float*)ctx->act_s.p, (const int16_t*)ctx->act_b.p};
+    int8_t* xq = (int8_t*)ctx->act_q.p;
+    float* xs = (float*)ctx->act_s.p;
+    int16_t* xb = (int16_t*)ctx->act_b.p;
+    const ovfq::ActQ act = grouped_big ? ovfq::ActQ{xq, xs, nullptr, (const uint16_t*)xb} : ovfq::ActQ{xq, xs, xb};
     int* tile_count = off + E + 1;
-    int* tiles = off + E + 2;
+    int* tiles = grouped_big ? off + E + 2 : nullptr;
+    if (!grouped_big) pdst = nullptr;
     if (route)
-        HIP_TRY(ovfq::launch_moe_route_plan(ld, rows, k, E, normalize, idxd, wd, off, prow, pof,
-                                            ovfq::kGroupedTileRows, grouped_big ? tiles : nullptr, tile_count, xd,
-                                            (int64_t)(n_x / OVFQ_QK), (int8_t*)ctx->act_q.p, (float*)ctx->act_s.p,
-                                            (int16_t*)ctx->act_b.p, ctx->stream));
+        HIP_TRY(ovfq::launch_moe_route_plan(ld, rows, k, E, normalize, idxd, wd, off, prow, pof, ovfq::kGroupedTileRows,
+                                            tiles, tile_count, pdst, xd, (int64_t)(n_x / OVFQ_QK), xq, xs, xb,
+                                            grouped_big, ctx->stream));
     else
-        HIP_TRY(ovfq::launch_moe_plan(idxd, rows, k, E, off, prow, pof, ovfq::kGroupedTileRows,
-                                      grouped_big ? tiles : nullptr, tile_count, xd, (int64_t)(n_x / OVFQ_QK),
-                                      (int8_t*)ctx->act_q.p, (float*)ctx->act_s.p, (int16_t*)ctx->act_b.p,
-                                      ctx->stream));
+        HIP_TRY(ovfq::launch_moe_plan(idxd, rows, k, E, off, prow, pof, ovfq::kGroupedTileRows, tiles, tile_count, pdst,
+                                      xd, (int64_t)(n_x / OVFQ_QK), xq, xs, xb, grouped_big, ctx->stream));
     const uint8_t* gw[OVFQ_MAX_EXPERTS];
     const uint8_t* uw[OVFQ_MAX_EXPERTS];
     const uint8_t* dw[OVFQ_MAX_EXPERTS];
@@ -1498,7 +1509,7 @@ static int moe_impl(ovfq_ctx* ctx, int E, const ovfq_weight* const* gate, const 
     D.rows = (int)P;
     D.expert_off = off;
     D.pair_row = nullptr;  // the intermediate is already pair-major
-    D.act = ovfq::ActQ{iq, is, ib};
+    D.act = grouped_big ? ovfq::ActQ{iq, is, nullptr, (const uint16_t*)ib, true} : ovfq::ActQ{iq, is, ib};
     D.pairs = (int)P;
     // With top-1 / top-2 and the down projection on the small-M path (the expert-stream or small-M kernel), the
     // combine is folded into it: each token output gets at most two float-atomic adds onto zero, whose sum does not
@@ -1521,7 +1532,8 @@ static int moe_impl(ovfq_ctx* ctx, int E, const ovfq_weight* const* gate, const 
         D.comb_tok = prow;
         D.comb_w = pw;
     }
-    HIP_TRY(ovfq::launch_gate_up_q8k(g, u, off, E, (int)P, dff, false, iq, is, ib, ctx->stream, fold));
+    HIP_TRY(ovfq::launch_gate_up_q8k(g, u, off, E, (int)P, dff, false, iq, is, ib, ctx->stream, fold,
+                                     grouped_big ? dt : 0, (uint16_t*)ib, pdst));
     if (grouped_big)
         HIP_TRY(ovfq::launch_mfma_grouped(dt, D, tiles, tile_count, max_tiles, ctx->stream));
     else
@@ -1562,14 +1574,14 @@ static int ffn_impl(ovfq_ctx* ctx, const ovfq_weight* gate, const ovfq_weight* u
     const size_t R = (size_t)rows;
     const ovfq_weight* dw[1] = {down};
     // the intermediate in the order that the down projection's kernel reads
-    const bool down_split = use_split(ctx, dff, rows, dw, 1);
+    const bool down_tiled = use_mid(ctx, dff, rows, dw, 1) != ovfq::MidKernel::kNone;
     const size_t recs = (size_t)ovfq::tiled_subs(rows) * (size_t)(dff / OVFQ_QK);
     auto carve = [&](Carver& c, float** g, float** u, int8_t** iq, float** is, int16_t** ib, float** hx, float** hy) {
         *g = c.take<float>(R * dff * 4);
         *u = c.take<float>(R * dff * 4);
-        *iq = c.take<int8_t>(down_split ? recs * ovfq::kTiledQ : R * dff);
-        *is = c.take<float>(down_split ? recs * ovfq::kTiledS : R * (dff / OVFQ_QK) * 4);
-        *ib = c.take<int16_t>(down_split ? recs * ovfq::kTiledB : R * (dff / 16) * 2);
+        *iq = c.take<int8_t>(down_tiled ? recs * ovfq::kTiledQ : R * dff);
+        *is = c.take<float>(down_tiled ? recs * ovfq::kTiledS : R * (dff / OVFQ_QK) * 4);
+        *ib = c.take<int16_t>(down_tiled ? recs * ovfq::kTiledB : R * (dff / 16) * 2);
         if (host) {
             *hx = c.take<float>(R * dmodel * 4);
             *hy = c.take<float>(R * dmodel * 4);
@@ -1594,20 +1606,20 @@ static int ffn_impl(ovfq_ctx* ctx, const ovfq_weight* gate, const ovfq_weight* u
     // gate/up (one launch; for one or a few short rows the Q8_K quantisation runs inside it)
     const ovfq_weight* gu[2] = {gate, up};
     float* gu_out[2] = {g, u};
-    if (quantize_in_launch(ctx, gate->type, dmodel, rows, 2, gate->out == up->out ? gate->out : 0)) {
+    const bool gu_tiled = use_mid(ctx, dmodel, rows, gu, 2) != ovfq::MidKernel::kNone;
+    if (!gu_tiled && quantize_in_launch(ctx, gate->type, dmodel, rows, 2, gate->out == up->out ? gate->out : 0)) {
         if ((rc = launch_projection(ctx, gu, 2, nullptr, gu_out, rows, ovfq::ActQ{nullptr, nullptr, nullptr}, xd)))
             return rc;
     } else {
         ovfq::ActQ act;
-        if ((rc = quantize_into_scratch(ctx, gate->type, xd, rows, dmodel, &act, use_split(ctx, dmodel, rows, gu, 2))))
-            return rc;
+        if ((rc = quantize_into_scratch(ctx, gate->type, xd, rows, dmodel, &act, gu_tiled))) return rc;
         if ((rc = launch_projection(ctx, gu, 2, nullptr, gu_out, rows, act))) return rc;
     }
     // act(gate) * up, quantised to Q8_K for the down projection
     HIP_TRY(ovfq::launch_gate_up_q8k(g, u, nullptr, 0, rows, dff, activation == OVFQ_FFN_GEGLU, iq, is, ib,
-                                     ctx->stream, ovfq::MoeFold{}, down_split ? down->type : 0, (uint16_t*)ib));
+                                     ctx->stream, ovfq::MoeFold{}, down_tiled ? down->type : 0, (uint16_t*)ib));
     float* dy[1] = {yd};
-    const ovfq::ActQ mid = down_split ? ovfq::ActQ{iq, is, nullptr, (const uint16_t*)ib, true} : ovfq::ActQ{iq, is, ib};
+    const ovfq::ActQ mid = down_tiled ? ovfq::ActQ{iq, is, nullptr, (const uint16_t*)ib, true} : ovfq::ActQ{iq, is, ib};
     if ((rc = launch_projection(ctx, dw, 1, nullptr, dy, rows, mid))) return rc;
     if (host && ((rc = io.down(y, yd, R * dmodel * 4)) || (rc = io.finish()))) return rc;
     return ok();

@@ -171,10 +171,12 @@ __global__ __launch_bounds__(64 * W, 2) void kquant_mfma_split_kernel(const PArg
                     wr, (__attribute__((address_space(3))) void*)(slot + 1024 * i), 16,
                     (int)(FS::start(dma_row[i] + (uint32_t)sb * F::kBytes) + dma_col[i]), 0, 0, 0);
     };
-    const uint32_t recs = (uint32_t)a.subs * (uint32_t)spr;
-    const __amdgpu_buffer_rsrc_t qr = make_rsrc(a.q, recs * 4096u);
-    const __amdgpu_buffer_rsrc_t br = make_rsrc(a.b, kMin ? recs * 512u : 0u);
-    const __amdgpu_buffer_rsrc_t sr = make_rsrc(a.s, recs * 64u);
+    // the activation from this workgroup's first tile on; tiles past the last read zeros
+    const uint64_t recs = (uint64_t)a.subs * (uint64_t)spr, rec0 = (uint64_t)(n0 / 16) * (uint64_t)spr;
+    const __amdgpu_buffer_rsrc_t qr = make_rsrc(a.q + rec0 * kTiledQ, rsrc_bytes(recs * kTiledQ, rec0 * kTiledQ));
+    const __amdgpu_buffer_rsrc_t br =
+        make_rsrc(a.b + (kMin ? rec0 * (kTiledB / 2) : 0), kMin ? rsrc_bytes(recs * kTiledB, rec0 * kTiledB) : 0u);
+    const __amdgpu_buffer_rsrc_t sr = make_rsrc(a.s + rec0 * (kTiledS / 4), rsrc_bytes(recs * kTiledS, rec0 * kTiledS));
 
     struct Act {
         u32x4 q[T][4];
@@ -182,16 +184,15 @@ __global__ __launch_bounds__(64 * W, 2) void kquant_mfma_split_kernel(const PArg
         uint32_t s;
     };
 
-    const uint32_t rec0 = (uint32_t)n0 / 16u * (uint32_t)spr;
     auto load_act = [&](int sb, Act& v) {
 #pragma unroll
         for (int s = 0; s < T; s++) {
-            const uint32_t rec = rec0 + (uint32_t)(s * spr + sb);
+            const uint32_t rec = (uint32_t)(s * spr + sb);
 #pragma unroll
             for (int t = 0; t < 4; t++) v.q[s][t] = ld4(qr, rec * 4096u + 1024u * t + 16u * (uint32_t)lane);
             if constexpr (kMin) v.b[s] = ld2(br, rec * 512u + 8u * (uint32_t)lane);
         }
-        v.s = ld1(sr, (rec0 + (uint32_t)(g * spr + sb)) * 64u + 4u * (uint32_t)r16);
+        v.s = ld1(sr, (uint32_t)(g * spr + sb) * 64u + 4u * (uint32_t)r16);
     };
 
     // Memory operations of the wave that may be in flight when a round's weights are read: all those issued after the
@@ -331,30 +332,378 @@ static hipError_t launch_split_w(int type, const PArgs& pa, int T, hipStream_t s
     return type == 12 ? launch_split_t<SplitQ4K, W>(pa, T, st) : launch_split_t<SplitQ6K, W>(pa, T, st);
 }
 
-// Work is (16-row weight tiles) x (16-row activation tiles); where it is little, the kernels that walk the whole contraction
-// in one workgroup leave the chip idle, and where it is much they share each operand among more outputs. Measured on MI355X
-// (graph replay with the quantise launch, us, the kernel chosen otherwise / this one):
-//   Q4_K 4096x4096       16 rows  9.6 /  8.7   64 rows 22.8 / 13.0   128 rows 23.6 / 17.2 (2048)   192 rows 24.1 / 24.4 (3072)
-//   Q4_K 2048x2048       16 rows  7.3 /  6.8   64 rows 14.6 /  9.0   256 rows 15.7 / 13.4 (2048)   320 rows 16.0 / 17.0 (2560)
-//   Q4_K 1024x14336      64 rows 59.8 / 24.1  512 rows 69.4 / 48.4 (2048)
-//   Q4_K q/k/v of 4096   16 rows 23.9 / 11.1   64 rows 23.8 / 18.4   128 rows 24.1 / 24.6 (3072)
-//   Q6_K 4096x14336      24 rows 40.1 / 23.1   64 rows 75.6 / 30.2   256 rows 93.9 / 80.5 (4096)   384 rows 106 / 117 (6144)
-//   Q6_K 4096x4096       64 rows 27.7 / 13.7  256 rows 32.6 / 31.8 (4096)   320 rows 37.1 / 39.1 (5120)
-// Up to 16 rows of a tall matrix the expert-stream kernel reads the weights faster (gate/up 2 x 14336x4096, 16 rows, 22.9 /
-// 24.3; 32768x2048 15.8 / 19.4), and for a few rows of 2048 or 3072 inputs the small-M kernel starts faster (2560x2560, 8
-// rows, 7.4 / 8.2). Past the small-M kernel's input size, and below the tiled kernel's rows, the alternative is
-// the general kernel (8192x28672 at 2 rows 33 / 36, 3 rows 40 / 36, 16 rows 137 / 38).
-bool split_preferred(int type, int in, int rows, long tiles) {
+// ------------------------------------------------------------------------------------------ panel kernel
+// Tall matrices and expert groups, 3 to 64 rows a tile: there are workgroups enough without splitting the contraction, but
+// the 64-row-tiled kernel of mfma.hip waited for every load of the next super-block before the barrier of each one, so a
+// super-block took a memory latency (1.8 us a step, whatever the rows). Here a workgroup's four waves own 16 weight rows
+// each against the same 16 T activation rows and walk the super-blocks in order, the sums in registers. A step's activation
+// tile is DMA'd into LDS one step ahead, each wave's weights two steps ahead into a ring of its own (mfma_split's slots),
+// and the one wait of a step leaves the weights of the next in flight. Rows are taken 16 at a time: 45 rows cost three tiles,
+// not 64 or 128 rows.
+// At 16 rows of gate/up (2 x 14336x4096, 66 MB) it is near the weights' stream (16 us beside the quantise launch); every 16
+// rows more add 4 us, half of their VALU work (operand build and fp32 tail, two waves a SIMD). us with the quantise
+// launch, before / after: 45 rows 46.5 / 28.2, 64 rows 47.3 / 32.3; the same in Q6_K, 64 rows 49.2 / 42.3; 8 experts of 40
+// pairs on average, gate/up 193 / 185, Q6_K down 245 / 125.
+struct PanelGroup {
+    const uint8_t* w0[kMaxExperts];
+    const uint8_t* w1[kMaxExperts];
+    const int* expert_off;
+    const int* pair_row;  // Src::kGather: activation row of each pair
+    const int* tiles;  // expert e | (tile i << 8): pairs expert_off[e] + [64 i, 64 i + 64)
+    const int* tile_count;
+    float* y0;
+    float* y1;
+    int n_rows;    // outputs per matrix
+    int o_tiles1;  // 64-row weight tiles of one matrix
+};
+
+struct PanelArgs {
+    PArgs p;  // job tiles, o_tiles: 64 weight rows
+    PanelGroup grp;
+};
+
+// Where the activation comes from: operand-ordered planes, those of expert groups, or the row-major planes of the tokens (with
+// fp16 bsums), gathered through the pairs' rows into the same order in LDS.
+enum class Src { kDense, kGroups, kGather };
+
+template <class FS, int T, Src SRC>
+__global__ __launch_bounds__(256, 2) void kquant_mfma_panel_kernel(const PanelArgs args) {
+    using F = typename FS::F;
+    constexpr bool kMin = F::kNumMfma == 3;
+    constexpr bool GRP = SRC != Src::kDense;
+    constexpr int W = 4;
+    constexpr int kSlot = 16 * 16 * FS::kPieces;
+    constexpr int kInstr = (FS::kPieces + 3) / 4;
+    __shared__ __align__(16) uint8_t ring[3][W][kSlot];
+    __shared__ __align__(16) uint8_t act0[T * 4096], act1[T * 4096];
+    __shared__ __align__(16) uint8_t bs0[kMin ? W * 512 : 16], bs1[kMin ? W * 512 : 16];
+    __shared__ __align__(16) float sc0[W * 16], sc1[W * 16];
+
+    const PArgs& a = args.p;
+    const int wave = wave_id();
+    const int lane = threadIdx.x & 63;
+    const int g = lane >> 4, r16 = lane & 15;
+    const int local = blockIdx.x >> 3;
+    const int o_tile = (blockIdx.x & 7) + 8 * (local / a.n_tiles);
+    const int n_tile = local % a.n_tiles;
+    if (o_tile >= a.o_tiles) return;  // uniform over the workgroup
+    const uint8_t* wptr;
+    const float* bias = nullptr;
+    float* y;
+    int n_out, o0, n0, m_end, sub0;  // output rows n0 .. m_end, activation tiles sub0 ..
+    if constexpr (GRP) {
+        if (n_tile >= args.grp.tile_count[0]) return;
+        const int te = args.grp.tiles[n_tile];
+        const int e = te & 0xff;
+        const int mat = o_tile >= args.grp.o_tiles1 ? 1 : 0;
+        wptr = mat ? args.grp.w1[e] : args.grp.w0[e];
+        y = mat ? args.grp.y1 : args.grp.y0;
+        n_out = args.grp.n_rows;
+        o0 = (o_tile - mat * args.grp.o_tiles1) * 64 + wave * 16;
+        const int pbeg = args.grp.expert_off[e];
+        n0 = pbeg + (te >> 8) * 64;
+        m_end = min(n0 + 64, args.grp.expert_off[e + 1]);
+        sub0 = pbeg / 16 + e + (te >> 8) * 4;
+    } else {
+        int j = 0;
+#pragma unroll
+        for (int t = 1; t < kMaxJobs; t++)
+            if (t < a.njobs && o_tile >= a.job[t].tile0) j = t;
+        wptr = a.job[j].w;
+        bias = a.job[j].bias;
+        y = a.job[j].y;
+        n_out = a.job[j].n_out;
+        o0 = (o_tile - a.job[j].tile0) * 64 + wave * 16;
+        n0 = n_tile * 16 * T;
+        m_end = min(n0 + 16 * T, a.m_rows);
+        sub0 = n_tile * T;
+    }
+    const int live = (m_end - n0 + 15) >> 4;  // 16-row tiles that hold rows
+    const int spr = a.spr;
+    const uint32_t row_bytes = (uint32_t)spr * F::kBytes;
+    const uint64_t wbase = (uint64_t)o0 * row_bytes;
+    const uint64_t wbase16 = wbase & ~15ull;
+    const __amdgpu_buffer_rsrc_t wr =
+        make_rsrc(wptr + wbase16, rsrc_bytes(((uint64_t)n_out * row_bytes + 15) & ~15ull, wbase16));
+    const uint32_t woff = (uint32_t)(wbase - wbase16) + (uint32_t)r16 * row_bytes;
+    uint32_t dma_row[kInstr], dma_col[kInstr];
+#pragma unroll
+    for (int i = 0; i < kInstr; i++) {
+        const uint32_t p = 64u * i + (uint32_t)lane;
+        dma_row[i] = (uint32_t)(wbase - wbase16) + p / FS::kPieces * row_bytes;
+        dma_col[i] = 16u * (p % FS::kPieces);
+    }
+    auto fetch = [&](int k, int sb) {
+#pragma unroll
+        for (int i = 0; i < kInstr; i++)
+            if (64 * i + 64 <= 16 * FS::kPieces || lane < 16 * FS::kPieces - 64 * i)
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                    wr, (__attribute__((address_space(3))) void*)(&ring[k][wave][0] + 1024 * i), 16,
+                    (int)(FS::start(dma_row[i] + (uint32_t)sb * F::kBytes) + dma_col[i]), 0, 0, 0);
+    };
+    // Activation: wave w moves a quarter of every tile, and tile w's bsums and scales. Offsets of the lane's pieces in
+    // super-block 0 and from one super-block to the next; tiles and rows past the launch's read zeros.
+    const bool gather = SRC == Src::kGather;
+    const uint64_t rec0 = gather ? 0 : (uint64_t)sub0 * (uint64_t)spr;
+    const uint64_t recs = gather ? 0 : (uint64_t)a.subs * (uint64_t)spr;
+    const uint64_t blocks = (uint64_t)a.m_rows * (uint64_t)spr;
+    const __amdgpu_buffer_rsrc_t qr = make_rsrc(
+        a.q + rec0 * kTiledQ, gather ? rsrc_bytes(blocks * kQK, 0) : rsrc_bytes(recs * kTiledQ, rec0 * kTiledQ));
+    const __amdgpu_buffer_rsrc_t br =
+        make_rsrc(a.b + (kMin ? rec0 * (kTiledB / 2) : 0),
+                  !kMin ? 0u : gather ? rsrc_bytes(blocks * 32, 0) : rsrc_bytes(recs * kTiledB, rec0 * kTiledB));
+    const __amdgpu_buffer_rsrc_t sr =
+        make_rsrc(a.s + rec0 * (kTiledS / 4),
+                  gather ? rsrc_bytes(blocks * 4, 0) : rsrc_bytes(recs * kTiledS, rec0 * kTiledS));
+    constexpr uint32_t kStepQ = SRC == Src::kGather ? kQK : kTiledQ, kStepB = SRC == Src::kGather ? 32 : kTiledB,
+                       kStepS = SRC == Src::kGather ? 4 : kTiledS;
+    uint32_t q_src[T], b_src[2], s_src;
+    if constexpr (SRC == Src::kGather) {
+        // Row by row, so that an instruction reads four rows' 256 contiguous bytes: in LDS, rows of 16 pieces XOR-swizzled by
+        // the row, so that the 16 lanes of one A read hit distinct banks. Bsums: 32 bytes a row, two lanes each.
+        constexpr uint32_t kAbsent = 0x80000000u;  // past every resource
+        auto act_row = [&](uint32_t i) -> uint32_t {  // activation row of the tile's row i
+            return n0 + (int)i < m_end ? (uint32_t)args.grp.pair_row[n0 + (int)i] : ~0u;
+        };
+#pragma unroll
+        for (int s = 0; s < T; s++) {
+            const uint32_t i = 4u * wave + (uint32_t)g, r = act_row(16u * s + i);
+            q_src[s] = r == ~0u ? kAbsent : r * (uint32_t)spr * kQK + 16u * F::src_piece((uint32_t)r16 ^ i);
+        }
+        const uint32_t rb = act_row(16u * wave + (((uint32_t)lane >> 1) & 15u)), rs = act_row(16u * wave + (uint32_t)r16);
+        b_src[0] = rb == ~0u ? kAbsent : rb * (uint32_t)spr * 32u + 16u * ((uint32_t)lane & 1u);
+        s_src = rs == ~0u ? kAbsent : rs * (uint32_t)spr * 4u;
+    } else {
+#pragma unroll
+        for (int s = 0; s < T; s++)
+            q_src[s] = (uint32_t)(s * spr) * (uint32_t)kTiledQ + 1024u * wave + 16u * (uint32_t)lane;
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+            b_src[i] = (uint32_t)(wave * spr) * (uint32_t)kTiledB + 256u * i + 4u * (uint32_t)lane;
+        s_src = (uint32_t)(wave * spr) * (uint32_t)kTiledS + 4u * (uint32_t)r16;
+    }
+    auto stage = [&](int sb, uint8_t* act, uint8_t* bs, float* sc) {
+#pragma unroll
+        for (int s = 0; s < T; s++)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                qr, (__attribute__((address_space(3))) void*)(act + s * 4096 + wave * 1024), 16,
+                (int)(q_src[s] + (uint32_t)sb * kStepQ), 0, 0, 0);
+        if constexpr (kMin && SRC == Src::kGather) {
+            if (lane < 32)
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(br, (__attribute__((address_space(3))) void*)(bs + wave * 512), 16,
+                                                         (int)(b_src[0] + (uint32_t)sb * kStepB), 0, 0, 0);
+        } else if constexpr (kMin) {
+#pragma unroll
+            for (int i = 0; i < 2; i++)
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                    br, (__attribute__((address_space(3))) void*)(bs + wave * 512 + i * 256), 4,
+                    (int)(b_src[i] + (uint32_t)sb * kStepB), 0, 0, 0);
+        }
+        if (lane < 16)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(sr, (__attribute__((address_space(3))) void*)(sc + wave * 16), 4,
+                                                     (int)(s_src + (uint32_t)sb * kStepS), 0, 0, 0);
+    };
+    const uint32_t slot_adr = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)&ring[0][wave][0] +
+                              (uint32_t)(16 * FS::kPieces * r16);
+
+    uint32_t a_off[4];  // the lane's A operand of MFMA t, and its bsums, in a tile's slot
+#pragma unroll
+    for (int t = 0; t < 4; t++)
+        a_off[t] = SRC == Src::kGather ? 256u * r16 + 16u * ((4u * t + (uint32_t)g) ^ (uint32_t)r16)
+                                       : 1024u * t + 16u * (uint32_t)lane;
+    const uint32_t b_off = SRC == Src::kGather ? 32u * r16 + 8u * g : 8u * (uint32_t)lane;
+    float out[T][4];
+#pragma unroll
+    for (int s = 0; s < T; s++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) out[s][i] = 0.0f;
+
+    auto step = [&](int sb, int k, const uint8_t* act, const uint8_t* bs, const float* sc, uint8_t* act_n, uint8_t* bs_n,
+                    float* sc_n) {
+        // This step's activation and weights have landed (only the next step's weights may be in flight), in every wave,
+        // and every wave is done with the slots that are filled next.
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_s_waitcnt(0x0070 | kInstr);  // vmcnt(kInstr) lgkmcnt(0)
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        stage(sb + 1, act_n, bs_n, sc_n);
+        asm volatile("" ::: "memory");
+        fetch(k == 0 ? 2 : k - 1, sb + 2);
+        const typename F::W w = FS::template read<63>(slot_adr + (uint32_t)(k * W * kSlot), woff + (uint32_t)sb * F::kBytes, g);
+        i32x4 op[4][F::kNumMfma];
+        F::template operands<0>(w, g, op[0]);
+        F::template operands<1>(w, g, op[1]);
+        F::template operands<2>(w, g, op[2]);
+        F::template operands<3>(w, g, op[3]);
+        const float d = F::d_of(w), dmin = F::dmin_of(w);
+        const u32x2 mb = F::min_operand(w, g);
+#pragma unroll
+        for (int s = 0; s < T; s++) {
+            if (GRP && s >= live) break;
+            i32x4 lo = {0, 0, 0, 0}, hi = {0, 0, 0, 0};
+#pragma unroll
+            for (int t = 0; t < 4; t++) {
+                const u32x4 av = *reinterpret_cast<const u32x4*>(act + s * 4096 + a_off[t]);
+                const i32x4 aop = i32x4{(int)av.x, (int)av.y, (int)av.z, (int)av.w};
+                lo = mfma16(aop, op[t][0], lo);
+                hi = mfma16(aop, op[t][1], hi);
+            }
+            const f32x4 q8s = *reinterpret_cast<const f32x4*>(sc + s * 16 + 4 * g);
+            if constexpr (kMin) {
+                const f16x4 bq = *reinterpret_cast<const f16x4*>(bs + s * 512 + b_off);
+                const f32x4 mn = __builtin_amdgcn_mfma_f32_16x16x16f16(bq, __builtin_bit_cast(f16x4, mb),
+                                                                      f32x4{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
+#pragma unroll
+                for (int i = 0; i < 4; i++) out[s][i] += q8s[i] * (d * (float)(lo[i] + (hi[i] << 3)) - dmin * mn[i]);
+            } else {
+#pragma unroll
+                for (int i = 0; i < 4; i++) out[s][i] += d * q8s[i] * (float)(lo[i] + (hi[i] << 8));
+            }
+        }
+    };
+    fetch(0, 0);
+    asm volatile("" ::: "memory");
+    stage(0, act0, bs0, sc0);
+    asm volatile("" ::: "memory");
+    fetch(1, 1);
+    int k = 0;
+    auto next_slot = [](int i) { return i == 2 ? 0 : i + 1; };
+    int sb = 0;
+    for (; sb + 1 < spr; sb += 2) {
+        step(sb, k, act0, bs0, sc0, act1, bs1, sc1);
+        k = next_slot(k);
+        step(sb + 1, k, act1, bs1, sc1, act0, bs0, sc0);
+        k = next_slot(k);
+    }
+    if (sb < spr) step(sb, k, act0, bs0, sc0, act1, bs1, sc1);
+
+    // y[n][o] = biasO + sum   (RT/Q4KDotKernel.cs:951, RT/Q6KDotKernel.cs:507)
+    const int o = o0 + r16;
+    const float bias_o = bias && o < n_out ? bias[o] : 0.0f;
+#pragma unroll
+    for (int s = 0; s < T; s++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int n = n0 + s * 16 + 4 * g + i;
+            if (n < m_end && o < n_out) y[(size_t)n * n_out + o] = bias ? bias_o + out[s][i] : out[s][i];
+        }
+    __builtin_amdgcn_s_waitcnt(0);  // no DMA lands in LDS that another workgroup may have by then
+}
+
+template <class FS>
+static hipError_t launch_panel_t(const PanelArgs& pa, int T, hipStream_t st) {
+    const dim3 grid((pa.p.o_tiles + 7) / 8 * 8 * pa.p.n_tiles), wg(256);
+    if (T == 1)
+        hipLaunchKernelGGL((kquant_mfma_panel_kernel<FS, 1, Src::kDense>), grid, wg, 0, st, pa);
+    else if (T == 2)
+        hipLaunchKernelGGL((kquant_mfma_panel_kernel<FS, 2, Src::kDense>), grid, wg, 0, st, pa);
+    else if (T == 3)
+        hipLaunchKernelGGL((kquant_mfma_panel_kernel<FS, 3, Src::kDense>), grid, wg, 0, st, pa);
+    else
+        hipLaunchKernelGGL((kquant_mfma_panel_kernel<FS, 4, Src::kDense>), grid, wg, 0, st, pa);
+    return hipGetLastError();
+}
+
+hipError_t launch_project_panel(int type, const ProjJob* jobs, int njobs, int in, int rows, ActQ act,
+                                hipStream_t st) {
+    PanelArgs pa{};
+    int tiles = 0;
+    for (int i = 0; i < njobs; i++) {
+        pa.p.job[i] = PJob{jobs[i].w, jobs[i].bias, jobs[i].y, jobs[i].n_rows, tiles};
+        tiles += (jobs[i].n_rows + 63) / 64;
+    }
+    pa.p.njobs = njobs;
+    pa.p.o_tiles = tiles;
+    pa.p.m_rows = rows;
+    pa.p.subs = (rows + 15) / 16;
+    pa.p.spr = in / kQK;
+    pa.p.q = act.q;
+    pa.p.s = act.s;
+    pa.p.b = act.bh;
+    if (type == 12 && !pa.p.b) return hipErrorInvalidValue;  // the Q4_K kernel reads the bsums
+    pa.p.n_tiles = (pa.p.subs + 3) / 4;
+    const int T = (pa.p.subs + pa.p.n_tiles - 1) / pa.p.n_tiles;
+    return type == 12 ? launch_panel_t<SplitQ4K>(pa, T, st) : launch_panel_t<SplitQ6K>(pa, T, st);
+}
+
+hipError_t launch_mfma_grouped(int type, const GroupLaunch& L, const int* tiles, const int* tile_count,
+                               int max_tiles, hipStream_t st) {
+    PanelArgs pa{};
+    const int o1 = (L.n_rows + 63) / 64;
+    pa.p.o_tiles = o1 * (L.w1 ? 2 : 1);
+    pa.p.n_tiles = max_tiles;
+    pa.p.subs = grouped_subs(L.pairs, L.experts);
+    pa.p.m_rows = L.rows;
+    pa.p.spr = L.in / kQK;
+    pa.p.q = L.act.q;
+    pa.p.s = L.act.s;
+    pa.p.b = L.act.bh;
+    if (L.act.tiled == (L.pair_row != nullptr) || (type == 12 && !pa.p.b)) return hipErrorInvalidValue;
+    if (L.comb) return hipErrorInvalidValue;  // the combine has its own launch
+    for (int e = 0; e < L.experts; e++) {
+        pa.grp.w0[e] = L.w0[e];
+        pa.grp.w1[e] = L.w1 ? L.w1[e] : nullptr;
+    }
+    pa.grp.expert_off = L.expert_off;
+    pa.grp.pair_row = L.pair_row;
+    pa.grp.tiles = tiles;
+    pa.grp.tile_count = tile_count;
+    pa.grp.y0 = L.y0;
+    pa.grp.y1 = L.y1;
+    pa.grp.n_rows = L.n_rows;
+    pa.grp.o_tiles1 = o1;
+    const dim3 grid((pa.p.o_tiles + 7) / 8 * 8 * max_tiles);
+    if (type == 12 && L.pair_row)
+        hipLaunchKernelGGL((kquant_mfma_panel_kernel<SplitQ4K, 4, Src::kGather>), grid, dim3(256), 0, st, pa);
+    else if (type == 12)
+        hipLaunchKernelGGL((kquant_mfma_panel_kernel<SplitQ4K, 4, Src::kGroups>), grid, dim3(256), 0, st, pa);
+    else if (L.pair_row)
+        hipLaunchKernelGGL((kquant_mfma_panel_kernel<SplitQ6K, 4, Src::kGather>), grid, dim3(256), 0, st, pa);
+    else
+        hipLaunchKernelGGL((kquant_mfma_panel_kernel<SplitQ6K, 4, Src::kGroups>), grid, dim3(256), 0, st, pa);
+    return hipGetLastError();
+}
+
+// Which kernel takes a batch whose activation the library quantises itself. Measured on MI355X (graph replay with the
+// quantise launch, us: the kernel chosen otherwise / split / panel):
+//   Q4_K 4096x4096       16 rows  9.7 /  8.7 / 14.3   64 rows 22.8 / 13.1 / 22.3   128 rows 23.7 / 17.9 / 23.0   192 rows 24.1 / 24.3 / 23.7
+//   Q4_K 1024x14336      64 rows 59.8 / 24.1 /   -   512 rows 69.4 / 48.4 /   -
+//   Q4_K q/k/v of 4096   16 rows 24.2 / 11.3 / 14.5   64 rows 23.9 / 18.5 / 22.9    96 rows 24.0 / 21.3 / 20.2   192 rows 32.7 / 34.7 / 31.1
+//   Q4_K 8192x8192       16 rows 21.7 / 16.8 / 24.1   64 rows 41.6 / 29.0 / 38.3    96 rows 41.8 / 39.7 / 33.2   256 rows 60.3 / 84.5 / 56.0
+//   Q4_K 14336x4096       8 rows 17.6 / 17.1 / 15.6   32 rows 23.8 / 22.4 / 17.5    64 rows 25.1 / 31.5 / 23.9   192 rows 48.8 / 69.6 / 46.6
+//   gate/up of 14336     16 rows 22.8 / 24.0 / 21.0   32 rows 45.7 / 31.6 / 23.8    64 rows 47.3 / 48.2 / 32.3   128 rows 50.6 / 87.0 / 56.1
+//   Q6_K 4096x14336      24 rows 40.0 / 23.7 / 64.2   64 rows 75.1 / 30.6 / 80.1   192 rows 92.4 / 66.2 / 81.8   384 rows  106 /  115 /  119
+//   Q6_K 14336x4096       8 rows 23.8 / 21.6 / 22.0   64 rows 37.5 / 33.8 / 29.6   160 rows 64.5 / 71.9 / 58.6   512 rows  127 /  172 /  121
+// So: the panel kernel on tall matrices (768 16-row tiles: it then has a workgroup for nearly every CU at any row count),
+// and on others from 65 rows, where the split kernel starts to read the weights twice, if it has a workgroup for
+// three of four CUs and (Q4_K) all of them run at once (q/k/v of 4096 at 331 rows, 576 workgroups: 41.2 / - / 45.6); the split kernel below that, while its work is small (weight tiles x activation tiles); beyond, and
+// where the wide (Q4_K) and pair-wide (Q6_K) kernels build each operand once for 128 rows, those of mfma.hip. Past the small-M
+// kernel's input size, and below the tiled kernel's rows, the alternative is the general kernel (8192x28672 at 2 rows 33 /
+// 36, 3 rows 40 / 36, 16 rows 137 / 38). Very tall matrices at 5 to 8 rows stay on the expert-stream kernel (128256x2048
+// 38.5, panel 39.8), and at 3 and 4 rows, where the multi-row decode kernel takes 65 and 76, only a pair does.
+MidKernel mid_kernel(int type, int in, int rows, long tiles, int count) {
     static const bool off = [] {
         const char* v = getenv("OVFQ_SPLIT");
         return v && *v == '0';
     }();
-    if (off || (type != 12 && type != 14) || rows < 2 || in % kQK) return false;
-    if (tiled_subs(rows) * 16 * in >= (int64_t)1 << 31) return false;  // 32-bit offsets into the padded planes
-    if (!mfma_small_supported(type, in) && rows < kMfmaMinRows) return rows > 2;
-    if (rows <= 8 && in > 1024 && in < 4096) return false;
-    if (rows <= 16) return tiles < 1024;
-    return tiles * ((rows + 15) / 16) <= (type == 14 ? 4096 : in <= 2048 ? 2048 : 2880);
+    if (off || (type != 12 && type != 14) || rows < 2 || in % kQK) return MidKernel::kNone;
+    if ((int64_t)in * 64 >= (int64_t)1 << 32) return MidKernel::kNone;  // 32-bit offsets into a workgroup's rows
+    const long subs = (rows + 15) / 16, work = tiles * subs;
+    const long panel_wgs = (tiles + 3) / 4 * ((subs + 3) / 4), wide_wgs = (tiles + 3) / 4 * ((rows + 127) / 128);
+    const bool pairwide = type == 14 && rows > 64 && wide_wgs >= 192 && wide_wgs <= 256;
+    if (!mfma_small_supported(type, in) && rows < kMfmaMinRows)
+        return rows == 2 ? MidKernel::kNone : tiles >= 768 ? MidKernel::kPanel : MidKernel::kSplit;
+    if (tiles >= 768) {
+        if (rows <= 4) return rows >= 3 && tiles >= 1536 && count == 1 ? MidKernel::kPanel : MidKernel::kNone;
+        if (rows <= 8 && tiles >= 1536) return MidKernel::kNone;
+        const bool panel = type == 12 ? rows <= 64 || work <= 10752 : rows <= 512 && !pairwide;
+        return panel ? MidKernel::kPanel : MidKernel::kNone;
+    }
+    if (rows <= 8 && in > 1024 && in < 4096) return MidKernel::kNone;  // 2560x2560 at 8 rows: small-M 7.4, split 8.2
+    if (rows > 64 && (type == 12 ? panel_wgs >= 192 && panel_wgs <= 512 && work <= 8192
+                                 : panel_wgs >= 256 && work > 3584 && rows <= 512 && !pairwide))
+        return MidKernel::kPanel;
+    return work <= (type == 14 ? 4096 : in <= 2048 ? 2048 : 2880) ? MidKernel::kSplit : MidKernel::kNone;
 }
 
 hipError_t launch_project_split(int type, const ProjJob* jobs, int njobs, int in, int rows, ActQ act,

@@ -119,7 +119,8 @@ __global__ __launch_bounds__(64) void moe_topk_kernel(const float* __restrict__ 
 // the general path of moe_plan_kernel computes.
 __device__ __forceinline__ void plan_one_wave(int ex, int rows, int k, int n_experts, int* __restrict__ expert_off,
                                               int* __restrict__ pair_row, int* __restrict__ pair_of, int nt,
-                                              int* __restrict__ tiles, int* __restrict__ tile_count) {
+                                              int* __restrict__ tiles, int* __restrict__ tile_count,
+                                              int* __restrict__ pair_dst) {
     const int lane = threadIdx.x & 63;
     const uint64_t below = (1ull << lane) - 1ull;
     const bool valid = lane < rows * k;
@@ -129,10 +130,13 @@ __device__ __forceinline__ void plan_one_wave(int ex, int rows, int k, int n_exp
         const int prev = __shfl(ex, lane - d < 0 ? 0 : lane - d, 64);
         if (slot >= d && prev == ex) claim = false;
     }
-    int pos = -1, off = 0, tb = 0;
+    int pos = -1, off = 0, tb = 0, dst = 0;
     for (int e = 0; e < n_experts; e++) {
         const uint64_t m = __ballot(claim && ex == e);
-        if (claim && ex == e) pos = off + __popcll(m & below);
+        if (claim && ex == e) {
+            pos = off + __popcll(m & below);
+            dst = 16 * (off / 16 + e) + pos - off;
+        }
         if (lane == 0) expert_off[e] = off;
         const int c = __popcll(m);
         if (tiles) {
@@ -148,6 +152,7 @@ __device__ __forceinline__ void plan_one_wave(int ex, int rows, int k, int n_exp
     }
     if (valid) pair_of[lane] = pos;
     if (pos >= 0) pair_row[pos] = lane / k;
+    if (pos >= 0 && pair_dst) pair_dst[pos] = dst;
 }
 
 // One workgroup. Expert e's pairs are the tokens n (ascending) with a slot j such that idx[n][j] == e (the first
@@ -166,12 +171,12 @@ __global__ __launch_bounds__(256) void moe_plan_kernel(const int* __restrict__ i
                                                        int* __restrict__ expert_off, int* __restrict__ pair_row,
                                                        int* __restrict__ pair_of, int staged, int nt,
                                                        int* __restrict__ tiles, int* __restrict__ tile_count,
-                                                       const float* __restrict__ x, int64_t n_blocks,
-                                                       int8_t* __restrict__ xq, float* __restrict__ xs,
-                                                       int16_t* __restrict__ xb) {
+                                                       int* __restrict__ pair_dst, const float* __restrict__ x,
+                                                       int64_t n_blocks, int8_t* __restrict__ xq,
+                                                       float* __restrict__ xs, int16_t* __restrict__ xb, int half16) {
     if (blockIdx.x > 0) {
         const int64_t blk = (int64_t)(blockIdx.x - 1) * 4 + wave_id();
-        if (blk < n_blocks) q8k_quantize_block(x, blk, xq, xs, xb);
+        if (blk < n_blocks) q8k_quantize_block(x, blk, xq, xs, xb, half16 != 0);
         return;
     }
     if (rows * k <= 64) {
@@ -179,10 +184,11 @@ __global__ __launch_bounds__(256) void moe_plan_kernel(const int* __restrict__ i
         if (wave_id() != 0) return;
         const int lane = threadIdx.x & 63;
         plan_one_wave(lane < rows * k ? idx_g[lane] : -1, rows, k, n_experts, expert_off, pair_row, pair_of, nt, tiles,
-                      tile_count);
+                      tile_count, pair_dst);
         return;
     }
     extern __shared__ int sidx[];
+    __shared__ int ebase[kMaxExperts];      // expert_off
     __shared__ int run[kMaxExperts];        // first position of the current chunk's claimers, per expert
     __shared__ int wcnt[4][kMaxExperts];    // claimers per wave of the current chunk, per expert
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
@@ -217,6 +223,7 @@ __global__ __launch_bounds__(256) void moe_plan_kernel(const int* __restrict__ i
         for (int e = 0; e < n_experts; e++) {
             const int c = run[e];
             run[e] = acc;
+            ebase[e] = acc;
             expert_off[e] = acc;
             acc += c;
             tbase[e] = tacc;
@@ -249,6 +256,7 @@ __global__ __launch_bounds__(256) void moe_plan_kernel(const int* __restrict__ i
                 for (int w = 0; w < wave; w++) p += wcnt[w][e];
                 pair_of[n * k + j] = p;
                 pair_row[p] = n;
+                if (pair_dst) pair_dst[p] = 16 * (ebase[e] / 16 + e) + p - ebase[e];
             }
         }
         __syncthreads();
@@ -268,12 +276,13 @@ __global__ __launch_bounds__(256) void moe_route_plan_kernel(const float* __rest
                                                              float* __restrict__ w_out, int* __restrict__ expert_off,
                                                              int* __restrict__ pair_row, int* __restrict__ pair_of,
                                                              int nt, int* __restrict__ tiles,
-                                                             int* __restrict__ tile_count, const float* __restrict__ x,
-                                                             int64_t n_blocks, int8_t* __restrict__ xq,
-                                                             float* __restrict__ xs, int16_t* __restrict__ xb) {
+                                                             int* __restrict__ tile_count, int* __restrict__ pair_dst,
+                                                             const float* __restrict__ x, int64_t n_blocks,
+                                                             int8_t* __restrict__ xq, float* __restrict__ xs,
+                                                             int16_t* __restrict__ xb, int half16) {
     if (blockIdx.x > 0) {
         const int64_t blk = (int64_t)(blockIdx.x - 1) * 4 + wave_id();
-        if (blk < n_blocks) q8k_quantize_block(x, blk, xq, xs, xb);
+        if (blk < n_blocks) q8k_quantize_block(x, blk, xq, xs, xb, half16 != 0);
         return;
     }
     if (wave_id() != 0) return;
@@ -319,7 +328,7 @@ __global__ __launch_bounds__(256) void moe_route_plan_kernel(const float* __rest
         if (i == slot) ex = v;
     }
     plan_one_wave(lane < rows * k ? ex : -1, rows, k, n_experts, expert_off, pair_row, pair_of, nt, tiles,
-                  tile_count);
+                  tile_count, pair_dst);
 }
 
 // ------------------------------------------------------------------------------------------ gate * up
@@ -335,7 +344,8 @@ __global__ __launch_bounds__(256) void gate_up_q8k_kernel(const float* __restric
                                                          const int* __restrict__ expert_off, int n_experts,
                                                          int max_pairs, int spr, int8_t* __restrict__ q,
                                                          float* __restrict__ s, int16_t* __restrict__ bs,
-                                                         uint16_t* __restrict__ bh, int tiled, const MoeFold fold) {
+                                                         uint16_t* __restrict__ bh, int tiled,
+                                                         const int* __restrict__ pair_dst, const MoeFold fold) {
     {
         const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
         for (int64_t j = i * 4; j < fold.y_len && j < i * 4 + 4; j++) fold.y[j] = 0.0f;
@@ -373,9 +383,9 @@ __global__ __launch_bounds__(256) void gate_up_q8k_kernel(const float* __restric
     const Q8KLane r = q8k_quantize_wave(v[0], v[1], v[2], v[3]);
     if (!live) return;
     if (tiled) {  // operand-ordered planes for a down weight of type `tiled` (quantize_q8k_tiled_kernel's layout)
-        const int64_t row = blk / spr;
-        const size_t rec = (size_t)(row >> 4) * spr + (size_t)(blk - row * spr);
-        const int r16 = (int)(row & 15), p = lane >> 2;
+        const int row = (int)(blk / spr), p = lane >> 2;
+        const int dst = pair_dst ? pair_dst[row] : row, r16 = dst & 15;
+        const size_t rec = (size_t)(dst >> 4) * spr + (size_t)(blk - (int64_t)row * spr);
         const int slot = tiled_slot(p, tiled == 14);
         *reinterpret_cast<uint32_t*>(q + rec * kTiledQ + slot * 256 + r16 * 16 + (lane & 3) * 4) = r.packed;
         if (tiled == 12 && (lane & 3) == 0)
@@ -450,19 +460,19 @@ bool moe_route_plan_fused(int rows, int k) { return rows * k <= 64 && k <= kMaxE
 
 hipError_t launch_moe_route_plan(const float* logits, int rows, int k, int n_experts, int normalize, int* idx,
                                  float* w, int* expert_off, int* pair_row, int* pair_of, int nt, int* tiles,
-                                 int* tile_count, const float* x, int64_t n_blocks, int8_t* xq, float* xs, int16_t* xb,
-                                 hipStream_t st) {
+                                 int* tile_count, int* pair_dst, const float* x, int64_t n_blocks, int8_t* xq,
+                                 float* xs, int16_t* xb, bool half16, hipStream_t st) {
     if (!moe_route_plan_fused(rows, k)) {
         hipError_t e = launch_moe_topk(logits, rows, n_experts, k, k, normalize, idx, w, st);
         if (e != hipSuccess) return e;
-        return launch_moe_plan(idx, rows, k, n_experts, expert_off, pair_row, pair_of, nt, tiles, tile_count, x,
-                               n_blocks, xq, xs, xb, st);
+        return launch_moe_plan(idx, rows, k, n_experts, expert_off, pair_row, pair_of, nt, tiles, tile_count, pair_dst,
+                               x, n_blocks, xq, xs, xb, half16, st);
     }
     const int64_t grid = 1 + (n_blocks + 3) / 4;
 #define OVFQ_ROUTE_PLAN(KM)                                                                                           \
     hipLaunchKernelGGL(moe_route_plan_kernel<KM>, dim3((unsigned)grid), dim3(256), 0, st, logits, rows, k, n_experts, \
-                       normalize, idx, w, expert_off, pair_row, pair_of, nt, tiles, tile_count, x, n_blocks, xq, xs,  \
-                       xb)
+                       normalize, idx, w, expert_off, pair_row, pair_of, nt, tiles, tile_count, pair_dst, x,         \
+                       n_blocks, xq, xs, xb, half16 ? 1 : 0)
     if (k <= 2)
         OVFQ_ROUTE_PLAN(2);
     else if (k <= 4)
@@ -478,30 +488,30 @@ hipError_t launch_moe_route_plan(const float* logits, int rows, int k, int n_exp
 }
 
 hipError_t launch_moe_plan(const int* idx, int rows, int k, int n_experts, int* expert_off, int* pair_row,
-                           int* pair_of, int nt, int* tiles, int* tile_count, const float* x, int64_t n_blocks,
-                           int8_t* xq, float* xs, int16_t* xb, hipStream_t st) {
+                           int* pair_of, int nt, int* tiles, int* tile_count, int* pair_dst, const float* x,
+                           int64_t n_blocks, int8_t* xq, float* xs, int16_t* xb, bool half16, hipStream_t st) {
     const size_t bytes = (size_t)rows * k * sizeof(int);
     const int staged = bytes <= 48 * 1024;
     const int64_t grid = 1 + (n_blocks + 3) / 4;
     hipLaunchKernelGGL(moe_plan_kernel, dim3((unsigned)grid), dim3(256), staged ? bytes : 0, st, idx, rows, k,
-                       n_experts, expert_off, pair_row, pair_of, staged, nt, tiles, tile_count, x, n_blocks, xq, xs,
-                       xb);
+                       n_experts, expert_off, pair_row, pair_of, staged, nt, tiles, tile_count, pair_dst, x,
+                       n_blocks, xq, xs, xb, half16 ? 1 : 0);
     return hipGetLastError();
 }
 
 hipError_t launch_gate_up_q8k(const float* gate, const float* up, const int* expert_off, int n_experts, int max_pairs,
                               int dff, bool gelu, int8_t* q, float* s, int16_t* b, hipStream_t st,
-                              const MoeFold& fold, int tiled, uint16_t* bh) {
+                              const MoeFold& fold, int tiled, uint16_t* bh, const int* pair_dst) {
     const int spr = dff / kQK;
     const int64_t waves = (int64_t)max_pairs * spr;
     const int64_t fold_threads = std::max<int64_t>((fold.y_len + 3) / 4, fold.slots);
     const dim3 grid((unsigned)std::max((waves + 3) / 4, (fold_threads + 255) / 256)), block(256);
     if (gelu)
         hipLaunchKernelGGL(gate_up_q8k_kernel<true>, grid, block, 0, st, gate, up, expert_off, n_experts, max_pairs, spr,
-                           q, s, b, bh, tiled, fold);
+                           q, s, b, bh, tiled, pair_dst, fold);
     else
         hipLaunchKernelGGL(gate_up_q8k_kernel<false>, grid, block, 0, st, gate, up, expert_off, n_experts, max_pairs,
-                           spr, q, s, b, bh, tiled, fold);
+                           spr, q, s, b, bh, tiled, pair_dst, fold);
     return hipGetLastError();
 }
 

@@ -167,15 +167,17 @@ __device__ __forceinline__ Q8KLane q8k_quantize_wave(float v0, float v1, float v
     return r;
 }
 
-// Q8_K block `blk` of x (256 floats) quantised by one wave: quants, bsums and scale written to q, bs, s.
+// Q8_K block `blk` of x (256 floats) quantised by one wave: quants, bsums (int16, or half16: as fp16, exact) and scale
+// written to q, bs, s.
 __device__ __forceinline__ void q8k_quantize_block(const float* __restrict__ x, int64_t blk, int8_t* __restrict__ q,
-                                                   float* __restrict__ s, int16_t* __restrict__ bs) {
+                                                   float* __restrict__ s, int16_t* __restrict__ bs, bool half16 = false) {
     const int lane = threadIdx.x & 63;
     const __amdgpu_buffer_rsrc_t xr = make_rsrc(x + blk * kQK, kQK * 4);
     const u32x4 raw = ld4(xr, lane * 16);
     const Q8KLane r = q8k_quantize_wave(as_float(raw.x), as_float(raw.y), as_float(raw.z), as_float(raw.w));
     reinterpret_cast<uint32_t*>(q + blk * kQK)[lane] = r.packed;
-    if ((lane & 3) == 0) bs[blk * 16 + (lane >> 2)] = (int16_t)r.group_sum;
+    if ((lane & 3) == 0)
+        bs[blk * 16 + (lane >> 2)] = half16 ? __builtin_bit_cast(int16_t, (_Float16)r.group_sum) : (int16_t)r.group_sum;
     if (lane == 0) s[blk] = r.scale;
 }
 

@@ -66,11 +66,15 @@ bool mfma_tiled_preferred(int type, int rows, int o_tiles, long out_rows);
 constexpr int kMfmaMinRows = 32;
 hipError_t launch_project_mfma(int type, const ProjJob* jobs, int njobs, int in, int rows, ActQ act,
                                hipStream_t st);
-// Batched K-quant projection with the contraction split over the waves of a workgroup (mfma_split.hip), any rows and K,
-// from operand-ordered planes (act.tiled); bit-identical to launch_project_kquant. split_preferred: the automatic choice of
-// that kernel for `rows` activation rows against weights of `tiles` 16-row tiles in all.
-bool split_preferred(int type, int in, int rows, long tiles);
+// Batched K-quant projections from operand-ordered planes (act.tiled), any rows and K, bit-identical to
+// launch_project_kquant (mfma_split.hip): the split kernel divides the contraction over the waves of a workgroup, the panel
+// kernel walks it with 64 weight rows a workgroup. mid_kernel: the automatic choice for `rows` activation rows against
+// `count` weights of `tiles` 16-row tiles in all (kNone: the kernels above and below).
+enum class MidKernel { kNone, kSplit, kPanel };
+MidKernel mid_kernel(int type, int in, int rows, long tiles, int count);
 hipError_t launch_project_split(int type, const ProjJob* jobs, int njobs, int in, int rows, ActQ act,
+                                hipStream_t st);
+hipError_t launch_project_panel(int type, const ProjJob* jobs, int njobs, int in, int rows, ActQ act,
                                 hipStream_t st);
 // Small-batch / grouped-expert K-quant projection. One or two matrices per expert (gate, up) of equal shape;
 // expert_off/pair_row (device arrays) select each expert's activation rows, or NULL for a single expert over
@@ -90,7 +94,7 @@ struct GroupLaunch {
     const int* pair_row;
     ActQ act;
     int pairs = 0;  // grouped launches: the pair count bound (rows x top_k), sizing the pair -> row map
-    // Grouped single-matrix launch_mfma_small launches only: instead of storing y0[pair][o], add
+    // Grouped single-matrix launches only: instead of storing y0[pair][o], add
     // comb_w[pair] * value to comb[comb_tok[pair]][o] with a float atomic (comb zeroed beforehand). Exact when at
     // most two pairs add to one output: (0 + a) + b == (0 + b) + a in fp32.
     float* comb = nullptr;
@@ -112,20 +116,23 @@ hipError_t launch_moe_topk(const float* logits, int rows, int n_experts, int k, 
                            float* w, hipStream_t st);
 // `tiles` (optional, else NULL): the experts' pair ranges in tiles of `nt` rows (expert | tile << 8), the count at
 // *tile_count; at most ceil(rows * k / nt) + n_experts entries. The same launch quantises the n_blocks Q8_K blocks
-// of x into xq / xs / xb (n_blocks may be 0).
+// of x into xq / xs / xb (half16: the bsums as fp16). `pair_dst` (optional, with tiles): the row of every pair in
+// operand-ordered planes, expert e's pairs from row 16 (expert_off[e] / 16 + e) on, so that every expert starts a 16-row
+// tile; grouped_subs(pairs, experts) tiles in all.
+inline int grouped_subs(int pairs, int experts) { return pairs / 16 + experts + 1; }
 hipError_t launch_moe_plan(const int* idx, int rows, int k, int n_experts, int* expert_off, int* pair_row,
-                           int* pair_of, int nt, int* tiles, int* tile_count, const float* x, int64_t n_blocks,
-                           int8_t* xq, float* xs, int16_t* xb, hipStream_t st);
+                           int* pair_of, int nt, int* tiles, int* tile_count, int* pair_dst, const float* x,
+                           int64_t n_blocks, int8_t* xq, float* xs, int16_t* xb, bool half16, hipStream_t st);
 // Router top-k (writing idx / w [rows][k]) and the plan above from router logits [rows][n_experts] (k <=
 // n_experts): one launch when moe_route_plan_fused(rows, k), else launch_moe_topk then launch_moe_plan.
 bool moe_route_plan_fused(int rows, int k);
 hipError_t launch_moe_route_plan(const float* logits, int rows, int k, int n_experts, int normalize, int* idx,
                                  float* w, int* expert_off, int* pair_row, int* pair_of, int nt, int* tiles,
-                                 int* tile_count, const float* x, int64_t n_blocks, int8_t* xq, float* xs, int16_t* xb,
-                                 hipStream_t st);
-// The batched int8-MFMA kernel over expert groups: tile list entry t covers rows [64 i, 64 i + 64) of expert e's
-// pairs; gate/up pairs (w1 set) share the launch. Activation rows are gathered through pair_row (NULL: pair p reads
-// row p); outputs are pair-major.
+                                 int* tile_count, int* pair_dst, const float* x, int64_t n_blocks, int8_t* xq,
+                                 float* xs, int16_t* xb, bool half16, hipStream_t st);
+// Expert groups of many pairs on the panel kernel (mfma_split.hip): tile list entry t covers rows [64 i, 64 i + 64) of
+// expert e's pairs; gate/up pairs (w1 set) share the launch, `comb` as in GroupLaunch. act: with pair_row the row-major planes
+// of the `rows` tokens, bsums as fp16 (act.bh); without, operand-ordered planes by pair_dst. Outputs are pair-major.
 hipError_t launch_mfma_grouped(int type, const GroupLaunch& launch, const int* tiles, const int* tile_count,
                                int max_tiles, hipStream_t st);
 constexpr int kGroupedTileRows = 64;
@@ -140,11 +147,12 @@ struct MoeFold {
     float* pw = nullptr;
 };
 // act(gate) * up (act: SiLU, or GELU with the tanh approximation), quantised to Q8_K for the down projection: row-major
-// planes, or, tiled = 12 / 14, the operand-ordered planes of launch_project_split for a down weight of that type (q, s,
-// bh; not with expert_off).
+// planes, or, tiled = 12 / 14, operand-ordered planes for a down weight of that type (q, s, bh), pair p at row pair_dst[p]
+// (NULL: row p).
 hipError_t launch_gate_up_q8k(const float* gate, const float* up, const int* expert_off, int n_experts, int max_pairs,
                               int dff, bool gelu, int8_t* q, float* s, int16_t* b, hipStream_t st,
-                              const MoeFold& fold = MoeFold{}, int tiled = 0, uint16_t* bh = nullptr);
+                              const MoeFold& fold = MoeFold{}, int tiled = 0, uint16_t* bh = nullptr,
+                              const int* pair_dst = nullptr);
 hipError_t launch_moe_combine(const float* out, const int* pair_of, const float* w, int rows, int k, int dmodel,
                               float* y, hipStream_t st);
 

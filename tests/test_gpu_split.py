@@ -1,7 +1,7 @@
-"""The split-contraction MFMA kernel (mfma_split.hip) against the oracle, bit for bit: every output is an exact integer
+"""The split and panel MFMA kernels (mfma_split.hip) against the oracle, bit for bit: every output is an exact integer
 dot per super-block and the reference's fp32 sum over the row (RT/Q4KDotKernel.cs:944-951, RT/Q6KDotKernel.cs:114-115).
 
-It takes batches whose activation is quantised by the call, by a rule on rows and shapes; the shapes here lie on both
+They take batches whose activation is quantised by the call, by a rule on rows and shapes; the shapes here lie on both
 sides of its tile edges: 3 .. 130 rows around multiples of 16 and 64, output counts off the 16-row tiles, one
 super-block to one more than the small-M kernel takes, four and eight waves, odd Q6_K super-block counts (rows that start
 2, 4, .. 14 bytes past a 16-byte boundary), a last block that ends inside a 16-byte piece.
@@ -102,3 +102,48 @@ def test_split_ffn_intermediate_matches_separate_calls(down):
     finally:
         ctx.set_batched_kernel("auto")
     assert torch.equal(y.view(torch.int32), ref.view(torch.int32))
+
+
+@pytest.mark.parametrize("fmt", ["q4k", "q6k"])
+@pytest.mark.parametrize("rows,k,shapes", [
+    (5, 512, [12300]),           # tall, one tile: the weights' last 64-row group partial
+    (17, 256, [12289]),          # one super-block, two tiles
+    (48, 768, [6200, 6200]),     # an odd number of super-blocks, a gate/up pair
+    (64, 512, [12288]),          # four full tiles
+    (70, 1280, [4096, 512, 520]),  # not tall: two activation tiles of three, the last rows absent
+])
+def test_panel_projection_bit_exact(orc, fmt, rows, k, shapes):
+    """The panel kernel (tall matrices; from 65 rows others): tile edges in both directions, one to five super-blocks."""
+    case("panel", fmt, rows, k, shapes)
+    rng = np.random.default_rng(rows * 31 + k)
+    made = [_weight(rng, fmt, n, k) for n in shapes]
+    x = normal(rng, (rows, k))
+    biases = [normal(rng, n) if i == 0 else None for i, n in enumerate(shapes)]
+    ys = ov.project_multi([w for _, w in made], t(x), rows=rows, biases=[None if b is None else t(b) for b in biases])
+    for i, (y, (blocks, _)) in enumerate(zip(ys, made)):
+        _check(y, _ref(orc, fmt, x, rows, blocks, k, shapes[i], biases[i]), f"job {i}")
+
+
+@pytest.mark.parametrize("down", ["q4k", "q6k"])
+@pytest.mark.parametrize("E,k,rows", [(3, 2, 33), (2, 2, 130), (8, 3, 90), (4, 1, 300)])
+def test_panel_expert_groups_match_small_batches(E, k, rows, down):
+    """Expert groups on the panel kernel (16 and more pairs an expert) against the same tokens in batches that the stream and
+    small-M kernels take: every projection is bit-identical, and so are the outputs. Slots with an expert out of range or
+    repeated add nothing; expert 0 gets tokens in runs, so that groups end on and off the 16- and 64-row tiles."""
+    case("panel experts", E, k, rows, down)
+    rng = np.random.default_rng(E * 100 + rows)
+    d, ff = 512, 768
+    gate, up = ([_weight(rng, "q4k", ff, d)[1] for _ in range(E)] for _ in range(2))
+    dw = [_weight(rng, down, d, ff)[1] for _ in range(E)]
+    x = normal(rng, (rows, d), 0.02)
+    idx = rng.integers(0, E, (rows, k)).astype(np.int32)
+    idx[:16, 0] = 0
+    idx[5, k - 1] = E + 3
+    idx[rows - 1, 0] = -1
+    wt = rng.random((rows, k)).astype(np.float32)
+    y = ov.moe_ffn(gate, up, dw, t(x), rows, k, t(idx), t(wt)).reshape(rows, d)
+    step = max(1, 8 * E // k - 1)
+    for r in range(0, rows, step):
+        m = min(step, rows - r)
+        ref = ov.moe_ffn(gate, up, dw, t(x[r:r + m]), m, k, t(idx[r:r + m]), t(wt[r:r + m])).reshape(m, d)
+        assert torch.equal(y[r:r + m].view(torch.int32), ref.view(torch.int32)), f"tokens {r} .. {r + m - 1}"
