@@ -147,3 +147,37 @@ def test_panel_expert_groups_match_small_batches(E, k, rows, down):
         m = min(step, rows - r)
         ref = ov.moe_ffn(gate, up, dw, t(x[r:r + m]), m, k, t(idx[r:r + m]), t(wt[r:r + m])).reshape(m, d)
         assert torch.equal(y[r:r + m].view(torch.int32), ref.view(torch.int32)), f"tokens {r} .. {r + m - 1}"
+
+
+@pytest.mark.parametrize("E,k,rows", [(8, 2, 33), (64, 8, 190), (3, 1, 257), (5, 3, 1000), (2, 2, 1024), (2, 1, 1025)])
+def test_plan_of_many_tokens(E, k, rows):
+    """The one-launch router and grouping plan (65 entries to 1024 tokens, 8 slots) against batches of up to 64 entries,
+    planned in one wave, and against the separate router; 1025 tokens take the general plan. Expert FFNs of one super-block
+    each way, bit-identical outputs."""
+    case("plan", E, k, rows)
+    rng = np.random.default_rng(E + rows)
+    d = ff = 256
+    gate, up, down = ([_weight(rng, "q4k", d, ff)[1] for _ in range(E)] for _ in range(3))
+    x, logits = normal(rng, (rows, d), 0.02), normal(rng, (rows, E))
+    y, idx, wt = ov.moe_ffn_routed(gate, up, down, t(x), rows, t(logits), k)
+    idx0 = torch.empty(rows * k, dtype=torch.int32, device=DEV)
+    wt0 = torch.empty(rows * k, device=DEV)
+    ov.MoeRouter.SelectTopK(t(logits), k, idx0, wt0, rows=rows)
+    assert torch.equal(idx, idx0) and torch.equal(wt.view(torch.int32), wt0.view(torch.int32))
+    # the caller's indices, one repeated and one out of range
+    idx = idx.reshape(rows, k).clone()
+    wt = wt.reshape(rows, k)
+    if k > 1:
+        idx[rows // 2, 1] = idx[rows // 2, 0]
+    idx[rows - 1, k - 1] = E
+    y2 = ov.moe_ffn(gate, up, down, t(x), rows, k, idx.reshape(-1), wt.reshape(-1)).reshape(rows, d)
+    step = 64 // k
+    for r in range(0, rows, step):
+        m = min(step, rows - r)
+        ref = ov.moe_ffn(gate, up, down, t(x[r:r + m]), m, k, idx[r:r + m].reshape(-1).contiguous(),
+                         wt[r:r + m].reshape(-1).contiguous()).reshape(m, d)
+        assert torch.equal(y2[r:r + m].view(torch.int32), ref.view(torch.int32)), f"tokens {r} .. {r + m - 1}"
+    same = torch.ones(rows, dtype=torch.bool, device=DEV)
+    same[rows // 2] = k == 1
+    same[rows - 1] = False
+    assert torch.equal(y.reshape(rows, d)[same].view(torch.int32), y2[same].view(torch.int32))
