@@ -703,7 +703,9 @@ MidKernel mid_kernel(int type, int in, int rows, long tiles, int count) {
     if (rows > 64 && (type == 12 ? panel_wgs >= 192 && panel_wgs <= 512 && work <= 8192
                                  : panel_wgs >= 256 && work > 3584 && rows <= 512 && !pairwide))
         return MidKernel::kPanel;
-    return work <= (type == 14 ? 4096 : in <= 2048 ? 2048 : 2880) ? MidKernel::kSplit : MidKernel::kNone;
+    // short rows (a launch of one or two rounds) past one 64-row tile: q/k/v of 2304 at 143 rows (1674) 16.0 / 16.5
+    const long most = type == 14 ? 4096 : rows <= 64 || in >= 4096 ? 2880 : 1536;
+    return work <= most ? MidKernel::kSplit : MidKernel::kNone;
 }
 
 hipError_t launch_project_split(int type, const ProjJob* jobs, int njobs, int in, int rows, ActQ act,
