@@ -98,143 +98,197 @@ __global__ __launch_bounds__(256) void quantize_q8_0_kernel(const float* __restr
     }
 }
 
-// ------------------------------------------------------------------------------------------ Q4_K encoder
-// GgmlQuant.EncodeQ4_KBlock (LD/GgmlQuant.cs:31-126): one thread per 256-element super-block.
-__global__ __launch_bounds__(256) void encode_q4k_kernel(const float* __restrict__ w, int64_t n_blocks,
-                                                          uint8_t* __restrict__ dst) {
-    const int64_t blk = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (blk >= n_blocks) return;
-    const float* src = w + blk * kQK;
-    float sub_scale[8], sub_min[8];
-    for (int j = 0; j < 8; j++) {
-        float lo = __builtin_inff(), hi = -__builtin_inff();
-        for (int e = 0; e < 32; e++) {
-            const float v = src[j * 32 + e];
-            if (v < lo) lo = v;
-            if (v > hi) hi = v;
-        }
-        if (lo > 0.0f) lo = 0.0f;
-        sub_scale[j] = (hi - lo) / 15.0f;
-        sub_min[j] = -lo;
-    }
-    float max_scale = 0.0f, max_min = 0.0f;
-    for (int j = 0; j < 8; j++) {
-        if (sub_scale[j] > max_scale) max_scale = sub_scale[j];
-        if (sub_min[j] > max_min) max_min = sub_min[j];
-    }
-    const float inv_scale = max_scale > 0.0f ? 63.0f / max_scale : 0.0f;
-    const float inv_min = max_min > 0.0f ? 63.0f / max_min : 0.0f;
-    uint32_t sc[8], m[8];
-    for (int j = 0; j < 8; j++) {
-        const int a = (int)rintf(inv_scale * sub_scale[j]);
-        const int c = (int)rintf(inv_min * sub_min[j]);
-        sc[j] = (uint32_t)(a < 63 ? a : 63);
-        m[j] = (uint32_t)(c < 63 ? c : 63);
-    }
-    const float d = max_scale / 63.0f;
-    const float dmin = max_min / 63.0f;
-    uint32_t* out = reinterpret_cast<uint32_t*>(dst + blk * kQ4KBytes);
-    out[0] = (uint32_t)float_to_half_rne(d) | ((uint32_t)float_to_half_rne(dmin) << 16);
-    // PackScalesMins (LD/GgmlQuant.cs:164-172), four bytes per 32-bit word.
-    uint32_t p0 = 0, p1 = 0, p2 = 0;
-    for (int j = 0; j < 4; j++) {
-        p0 |= ((sc[j] & 0x3f) | ((sc[j + 4] >> 4) << 6)) << (8 * j);
-        p1 |= ((m[j] & 0x3f) | ((m[j + 4] >> 4) << 6)) << (8 * j);
-        p2 |= ((sc[j + 4] & 0x0f) | ((m[j + 4] & 0x0f) << 4)) << (8 * j);
-    }
-    out[1] = p0;
-    out[2] = p1;
-    out[3] = p2;
-    // Nibbles from the float d / dmin (LD/GgmlQuant.cs:108-116): qs[32p+e] = q[64p+e] | q[64p+32+e] << 4.
-    for (int p = 0; p < 4; p++) {
-        const float es_lo = d * (float)sc[2 * p], em_lo = dmin * (float)m[2 * p];
-        const float es_hi = d * (float)sc[2 * p + 1], em_hi = dmin * (float)m[2 * p + 1];
-        for (int e4 = 0; e4 < 32; e4 += 4) {
-            uint32_t word = 0;
-            for (int k = 0; k < 4; k++) {
-                const int e = e4 + k;
-                int l0 = es_lo > 0.0f ? (int)rintf((src[64 * p + e] + em_lo) / es_lo) : 0;
-                int l1 = es_hi > 0.0f ? (int)rintf((src[64 * p + 32 + e] + em_hi) / es_hi) : 0;
-                l0 = l0 < 0 ? 0 : (l0 > 15 ? 15 : l0);
-                l1 = l1 < 0 ? 0 : (l1 > 15 ? 15 : l1);
-                word |= (uint32_t)(l0 | (l1 << 4)) << (8 * k);
-            }
-            out[4 + (32 * p + e4) / 4] = word;
-        }
+// ------------------------------------------------------------------------------------------ weight encoders
+// Both encoders spread a 256-element super-block over a 16-lane DPP row, sixteen consecutive elements a lane (four 16-byte
+// loads), so a wave covers four; per-block values are exchanged inside the row. They are bound by the source's stream: a
+// thread per super-block (1024 waves in all for 4096x4096, every load instruction touching 64 lines) was bound by those loads.
+// us before / after: Q4_K 4096x4096 118 / 18.0 (4.2 TB/s), 8192x8192 1287 / 73; Q6_K 242 / 20.4 and 1487 / 67.
+template <int kCtrl>
+__device__ __forceinline__ uint32_t dpp_u32(uint32_t v) {
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, kCtrl, 0xf, 0xf, false);
+}
+// The value of the lane whose number in the 16-lane row differs in bit 1, 2, 4 or 8.
+__device__ __forceinline__ uint32_t row_xor1(uint32_t v) { return dpp_u32<0xb1>(v); }
+__device__ __forceinline__ uint32_t row_xor2(uint32_t v) { return dpp_u32<0x4e>(v); }
+__device__ __forceinline__ uint32_t row_xor4(uint32_t v) { return dpp_u32<0x1b>(dpp_u32<0x141>(v)); }  // 7 - i, then i ^ 3
+__device__ __forceinline__ uint32_t row_xor8(uint32_t v) { return dpp_u32<0x128>(v); }
+__device__ __forceinline__ uint32_t f_bits(float f) { return __builtin_bit_cast(uint32_t, f); }
+
+typedef uint32_t u32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
+
+// Lane `l16` of row `lane >> 4` loads its sixteen elements of super-block blk0 + row (zeros past n_blocks).
+__device__ __forceinline__ void load_row16(const float* __restrict__ w, int64_t blk0, int64_t n_blocks, float (&v)[16]) {
+    const __amdgpu_buffer_rsrc_t xr =
+        make_rsrc(w + blk0 * kQK, rsrc_bytes((uint64_t)n_blocks * kQK * 4, (uint64_t)blk0 * kQK * 4));
+    const uint32_t off = (threadIdx.x & 63) * 64u;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const u32x4 t = ld4(xr, off + 16u * i);
+        v[4 * i] = as_float(t.x);
+        v[4 * i + 1] = as_float(t.y);
+        v[4 * i + 2] = as_float(t.z);
+        v[4 * i + 3] = as_float(t.w);
     }
 }
 
-// ------------------------------------------------------------------------------------------ Q6_K encoder
+// GgmlQuant.EncodeQ4_KBlock (LD/GgmlQuant.cs:31-126). Lane i holds half of sub-block i >> 1.
+__global__ __launch_bounds__(256) void encode_q4k_kernel(const float* __restrict__ w, int64_t n_blocks,
+                                                          uint8_t* __restrict__ dst) {
+    const int64_t blk0 = ((int64_t)blockIdx.x * 4 + wave_id()) * 4;
+    if (blk0 >= n_blocks) return;
+    const int lane = threadIdx.x & 63, l16 = lane & 15;
+    const int64_t blk = blk0 + (lane >> 4);
+    float v[16];
+    load_row16(w, blk0, n_blocks, v);
+    float lo = __builtin_inff(), hi = -__builtin_inff();
+#pragma unroll
+    for (int e = 0; e < 16; e++) {
+        if (v[e] < lo) lo = v[e];
+        if (v[e] > hi) hi = v[e];
+    }
+    const float lo1 = as_float(row_xor1(f_bits(lo))), hi1 = as_float(row_xor1(f_bits(hi)));
+    if (lo1 < lo) lo = lo1;
+    if (hi1 > hi) hi = hi1;
+    if (lo > 0.0f) lo = 0.0f;
+    const float sub_scale = (hi - lo) / 15.0f, sub_min = -lo;
+    float max_scale = 0.0f, max_min = 0.0f;  // over the row's eight sub-blocks
+    if (sub_scale > max_scale) max_scale = sub_scale;
+    if (sub_min > max_min) max_min = sub_min;
+    auto max_with = [&](uint32_t s, uint32_t m) {
+        if (as_float(s) > max_scale) max_scale = as_float(s);
+        if (as_float(m) > max_min) max_min = as_float(m);
+    };
+    max_with(row_xor2(f_bits(max_scale)), row_xor2(f_bits(max_min)));
+    max_with(row_xor4(f_bits(max_scale)), row_xor4(f_bits(max_min)));
+    max_with(row_xor8(f_bits(max_scale)), row_xor8(f_bits(max_min)));
+    const float inv_scale = max_scale > 0.0f ? 63.0f / max_scale : 0.0f;
+    const float inv_min = max_min > 0.0f ? 63.0f / max_min : 0.0f;
+    const int sa = (int)rintf(inv_scale * sub_scale), ma = (int)rintf(inv_min * sub_min);
+    const uint32_t sc = (uint32_t)(sa < 63 ? sa : 63), m = (uint32_t)(ma < 63 ? ma : 63);
+    const float d = max_scale / 63.0f;
+    const float dmin = max_min / 63.0f;
+    // Nibbles from the float d / dmin (LD/GgmlQuant.cs:108-116): qs[32p+e] = q[64p+e] | q[64p+32+e] << 4, a byte of four
+    // dwords each; the odd sub-blocks' go to the lanes of the even ones.
+    const float es = d * (float)sc, em = dmin * (float)m;
+    uint32_t q[4] = {0, 0, 0, 0};
+#pragma unroll
+    for (int e = 0; e < 16; e++) {
+        int l = es > 0.0f ? (int)rintf((v[e] + em) / es) : 0;
+        l = l < 0 ? 0 : (l > 15 ? 15 : l);
+        q[e >> 2] |= (uint32_t)l << (8 * (e & 3));
+    }
+#pragma unroll
+    for (int i = 0; i < 4; i++) q[i] |= row_xor2(q[i]) << 4;
+    // PackScalesMins (LD/GgmlQuant.cs:164-172), four bytes per 32-bit word: sub-block j < 4 (lane 2j) with j + 4.
+    const uint32_t sc4 = row_xor8(sc), m4 = row_xor8(m);
+    const bool packs = l16 < 8 && (l16 & 1) == 0;
+    const uint32_t at = 4u * (uint32_t)l16;  // 8 j
+    uint32_t p0 = packs ? ((sc & 0x3f) | ((sc4 >> 4) << 6)) << at : 0;
+    uint32_t p1 = packs ? ((m & 0x3f) | ((m4 >> 4) << 6)) << at : 0;
+    uint32_t p2 = packs ? ((sc4 & 0x0f) | ((m4 & 0x0f) << 4)) << at : 0;
+    p0 |= row_xor2(p0);
+    p1 |= row_xor2(p1);
+    p2 |= row_xor2(p2);
+    p0 |= row_xor4(p0);
+    p1 |= row_xor4(p1);
+    p2 |= row_xor4(p2);
+    if (blk >= n_blocks) return;
+    uint8_t* out = dst + blk * kQ4KBytes;  // any 4-byte-aligned address
+    if ((l16 & 2) == 0) *reinterpret_cast<u32x4_a4*>(out + 16 + 32 * (l16 >> 2) + 16 * (l16 & 1)) = u32x4{q[0], q[1], q[2], q[3]};
+    if (l16 == 0)
+        *reinterpret_cast<u32x4_a4*>(out) =
+            u32x4{(uint32_t)float_to_half_rne(d) | ((uint32_t)float_to_half_rne(dmin) << 16), p0, p1, p2};
+}
+
 // The build's own Q6_K encoder (the reference has none): the signed value of largest magnitude in each
 // 16-element sub-block maps to q = -32; one fp16 super-scale d = 1 / (-128 / largest sub-scale) carries 16
 // int8 sub-scales; quants are rint(x / (fp16(d) * sc)) clamped to [-32, 31], stored +32. The byte layout is
-// the inverse of GgmlDequant.DecodeQ6_KBlock (LD/GgmlDequant.cs:143-209).
+// the inverse of GgmlDequant.DecodeQ6_KBlock (LD/GgmlDequant.cs:143-209). Lane s holds sub-block s = 8 h + 2 p + l: the
+// elements 32 p + 16 l .. of half h. A wave's four 210-byte blocks are put together in LDS and stored as 210 dwords.
 __global__ __launch_bounds__(256) void encode_q6k_kernel(const float* __restrict__ w, int64_t n_blocks,
                                                           uint8_t* __restrict__ dst) {
-    const int64_t blk = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (blk >= n_blocks) return;
-    const float* src = w + blk * kQK;
-    uint8_t* out = dst + blk * kQ6KBytes;  // 210-byte stride: 2-byte aligned, so store 16-bit halves
-    float sub_scale[16];
-    float max_abs_scale = 0.0f, max_scale = 0.0f;
-    for (int s = 0; s < 16; s++) {
-        float amax = 0.0f, vmax = 0.0f;
-        for (int e = 0; e < 16; e++) {
-            const float v = src[s * 16 + e];
-            const float a = fabsf(v);
-            if (a > amax) {
-                amax = a;
-                vmax = v;
-            }
-        }
-        sub_scale[s] = amax > 0.0f ? vmax / -32.0f : 0.0f;
-        const float as = fabsf(sub_scale[s]);
-        if (as > max_abs_scale) {
-            max_abs_scale = as;
-            max_scale = sub_scale[s];
+    __shared__ __align__(16) uint16_t stage[4][4 * kQ6KBytes / 2];
+    const int wave = wave_id();
+    const int64_t blk0 = ((int64_t)blockIdx.x * 4 + wave) * 4;
+    if (blk0 >= n_blocks) return;
+    const int lane = threadIdx.x & 63, l16 = lane & 15;
+    float v[16];
+    load_row16(w, blk0, n_blocks, v);
+    float amax = 0.0f, vmax = 0.0f;
+#pragma unroll
+    for (int e = 0; e < 16; e++) {
+        const float a = fabsf(v[e]);
+        if (a > amax) {
+            amax = a;
+            vmax = v[e];
         }
     }
-    uint16_t* o16 = reinterpret_cast<uint16_t*>(out);
-    if (max_abs_scale == 0.0f) {
-        for (int i = 0; i < kQ6KBytes / 2; i++) o16[i] = 0;
-        return;
-    }
+    const float sub_scale = amax > 0.0f ? vmax / -32.0f : 0.0f;
+    // the first sub-scale of the largest magnitude
+    float max_scale = sub_scale;
+    uint32_t first = (uint32_t)l16;
+    auto larger = [&](uint32_t s, uint32_t i) {
+        const float o = fabsf(as_float(s)), mine = fabsf(max_scale);
+        if (o > mine || (o == mine && i < first)) {
+            max_scale = as_float(s);
+            first = i;
+        }
+    };
+    larger(row_xor1(f_bits(max_scale)), row_xor1(first));
+    larger(row_xor2(f_bits(max_scale)), row_xor2(first));
+    larger(row_xor4(f_bits(max_scale)), row_xor4(first));
+    larger(row_xor8(f_bits(max_scale)), row_xor8(first));
+    const bool zero = fabsf(max_scale) == 0.0f;  // the whole block: all bytes 0
     const float iscale = -128.0f / max_scale;
     const float d = 1.0f / iscale;
     const uint16_t dh = float_to_half_rne(d);
-    const float dd = half_bits_to_float(dh);
-    int sc[16];
-    for (int s = 0; s < 16; s++) {
-        const int v = (int)rintf(iscale * sub_scale[s]);
-        sc[s] = v < 127 ? v : 127;
-    }
-    for (int i = 0; i < 8; i++) {
-        o16[96 + i] = (uint16_t)((uint32_t)(sc[2 * i] & 0xff) | ((uint32_t)(sc[2 * i + 1] & 0xff) << 8));
-    }
-    o16[104] = dh;
-    auto quant = [&](int i) -> int {
-        const float ds = dd * (float)sc[i >> 4];
+    const int sv = (int)rintf(iscale * sub_scale);
+    const int sc = sv < 127 ? sv : 127;
+    const float ds = half_bits_to_float(dh) * (float)sc;
+    uint32_t nib[4] = {0, 0, 0, 0}, top[4] = {0, 0, 0, 0};
+    const int p = (l16 >> 1) & 3;
+#pragma unroll
+    for (int e = 0; e < 16; e++) {
         int l = 0;
         if (ds != 0.0f) {
-            l = (int)rintf(src[i] / ds);
+            l = (int)rintf(v[e] / ds);
             l = l < -32 ? -32 : (l > 31 ? 31 : l);
         }
-        return l + 32;
-    };
-    for (int h = 0; h < 2; h++) {
-        for (int l = 0; l < 32; l += 2) {
-            uint32_t qlA = 0, qlB = 0, qh = 0;
-            for (int k = 0; k < 2; k++) {
-                const int q1 = quant(128 * h + l + k), q2 = quant(128 * h + 32 + l + k);
-                const int q3 = quant(128 * h + 64 + l + k), q4 = quant(128 * h + 96 + l + k);
-                qlA |= (uint32_t)((q1 & 0x0f) | ((q3 & 0x0f) << 4)) << (8 * k);
-                qlB |= (uint32_t)((q2 & 0x0f) | ((q4 & 0x0f) << 4)) << (8 * k);
-                qh |= (uint32_t)((q1 >> 4) | ((q2 >> 4) << 2) | ((q3 >> 4) << 4) | ((q4 >> 4) << 6)) << (8 * k);
-            }
-            o16[(64 * h + l) / 2] = (uint16_t)qlA;
-            o16[(64 * h + 32 + l) / 2] = (uint16_t)qlB;
-            o16[(128 + 32 * h + l) / 2] = (uint16_t)qh;
+        const uint32_t qv = zero ? 0u : (uint32_t)(l + 32);
+        nib[e >> 2] |= (qv & 0x0f) << (8 * (e & 3));
+        top[e >> 2] |= (qv >> 4) << (8 * (e & 3));
+    }
+    // ql[64h + 32 (p & 1) + 16 l + i] = q of p & 1 | q of (p & 1) + 2 << 4; qh[32h + 16 l + i] = the four p's top bits
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        nib[i] |= row_xor4(nib[i]) << 4;
+        top[i] <<= 2 * p;
+        top[i] |= row_xor2(top[i]);
+        top[i] |= row_xor4(top[i]);
+    }
+    uint16_t* out = &stage[wave][(lane >> 4) * (kQ6KBytes / 2)];
+    const int h = l16 >> 3, l = l16 & 1;
+    if (p < 3) {  // p = 0, 1: ql; 2: qh
+        const int at = p < 2 ? 64 * h + 32 * p + 16 * l : 128 + 32 * h + 16 * l;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const uint32_t word = p < 2 ? nib[i] : top[i];
+            out[at / 2 + 2 * i] = (uint16_t)word;
+            out[at / 2 + 2 * i + 1] = (uint16_t)(word >> 16);
         }
+    }
+    reinterpret_cast<uint8_t*>(out)[192 + l16] = zero ? 0 : (uint8_t)sc;
+    if (l16 == 0) out[104] = zero ? 0 : dh;
+    wave_sync();
+    // four blocks are 210 dwords from a 4-byte-aligned address on; the last wave's may be fewer
+    const int64_t blocks = n_blocks - blk0 < 4 ? n_blocks - blk0 : 4;
+    uint8_t* base = dst + blk0 * kQ6KBytes;
+    if (blocks == 4) {
+        for (int i = lane; i < 4 * kQ6KBytes / 4; i += 64)
+            reinterpret_cast<uint32_t*>(base)[i] = reinterpret_cast<const uint32_t*>(stage[wave])[i];
+    } else {
+        for (int i = lane; i < (int)blocks * (kQ6KBytes / 2); i += 64)
+            reinterpret_cast<uint16_t*>(base)[i] = stage[wave][i];
     }
 }
 
@@ -410,13 +464,13 @@ hipError_t launch_q8_0_deinterleave(const void* gguf, int64_t n_blocks, int8_t* 
 
 hipError_t launch_encode_q4k(const float* w, int64_t n_blocks, uint8_t* dst, hipStream_t st) {
     if (n_blocks <= 0) return hipSuccess;
-    hipLaunchKernelGGL(encode_q4k_kernel, dim3((unsigned)((n_blocks + 255) / 256)), dim3(256), 0, st, w, n_blocks, dst);
+    hipLaunchKernelGGL(encode_q4k_kernel, dim3((unsigned)((n_blocks + 15) / 16)), dim3(256), 0, st, w, n_blocks, dst);
     return hipGetLastError();
 }
 
 hipError_t launch_encode_q6k(const float* w, int64_t n_blocks, uint8_t* dst, hipStream_t st) {
     if (n_blocks <= 0) return hipSuccess;
-    hipLaunchKernelGGL(encode_q6k_kernel, dim3((unsigned)((n_blocks + 255) / 256)), dim3(256), 0, st, w, n_blocks, dst);
+    hipLaunchKernelGGL(encode_q6k_kernel, dim3((unsigned)((n_blocks + 15) / 16)), dim3(256), 0, st, w, n_blocks, dst);
     return hipGetLastError();
 }
 
