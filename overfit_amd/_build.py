@@ -8,7 +8,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libovfq.so")
-SOURCES = ["quant.hip", "project.hip", "gemv.hip", "mfma.hip", "mfma_split.hip", "moe.hip", "heads.hip", "noalloc.hip", "api.cpp"]
+SOURCES = ["quant.hip", "project.hip", "gemv.hip", "mfma.hip", "mfma_split.hip", "q8_mid.hip", "moe.hip", "heads.hip", "noalloc.hip", "api.cpp"]
 
 HIPCC = os.environ.get("HIPCC", shutil.which("hipcc") or "/opt/rocm/bin/hipcc")
 
@@ -29,7 +29,7 @@ FLAGS = [
 # Per-file additions. The MFMA kernels accumulate in VGPRs instead of AGPRs: with AGPR accumulators the expert-stream
 # and small-M kernels copy every result out (v_accvgpr_read, 12 per super-block step) before the fp32 tail.
 _VGPR_FORM = ["-mllvm", "-amdgpu-mfma-vgpr-form=true"]
-FILE_FLAGS = {"mfma.hip": _VGPR_FORM, "mfma_split.hip": _VGPR_FORM}
+FILE_FLAGS = {"mfma.hip": _VGPR_FORM, "mfma_split.hip": _VGPR_FORM, "q8_mid.hip": _VGPR_FORM}
 
 
 def build(verbose: bool = False) -> str:

@@ -256,11 +256,25 @@ int weight_create(ovfq_ctx* ctx, int type, const void* blocks, size_t nbytes, co
     return ok();
 }
 
+// The same for the operand-ordered Q8_0 kernels: `planes` weight planes (heads) of `plane_in` inputs each.
+int quantize_q8_tiled_into_scratch(ovfq_ctx* c, const float* x_dev, int rows, int planes, int plane_in, ovfq::ActQ* act) {
+    const size_t recs = ovfq::q8_tiled_records(rows, planes, plane_in);
+    int rc;
+    if ((rc = ensure(c, c->act_q, recs * ovfq::kQ8TiledQ)) ||
+        (rc = ensure(c, c->act_s, recs * ovfq::kQ8TiledS * sizeof(float))))
+        return rc;
+    *act = ovfq::ActQ{(const int8_t*)c->act_q.p, (const float*)c->act_s.p, nullptr, nullptr, true};
+    HIP_TRY(ovfq::launch_quantize_q8_0_tiled(x_dev, rows, planes, plane_in, (int8_t*)c->act_q.p, (float*)c->act_s.p,
+                                             c->stream));
+    return OVFQ_OK;
+}
+
 // Quantises `rows` activation rows of length `in` for weight type `type` into the context scratch.
 int quantize_into_scratch(ovfq_ctx* c, int type, const float* x_dev, int rows, int in, ovfq::ActQ* act,
                           bool tiled = false) {
     const size_t n = (size_t)rows * in;
     int rc;
+    if (tiled && type == OVFQ_TYPE_Q8_0) return quantize_q8_tiled_into_scratch(c, x_dev, rows, 1, in, act);
     if (tiled) {
         const size_t recs = (size_t)ovfq::tiled_subs(rows) * (size_t)(in / OVFQ_QK);
         if ((rc = ensure(c, c->act_q, recs * ovfq::kTiledQ)) || (rc = ensure(c, c->act_s, recs * ovfq::kTiledS)) ||
@@ -377,6 +391,16 @@ ovfq::MidKernel use_mid(const ovfq_ctx* c, int in, int rows, const ovfq_weight* 
     return ovfq::mid_kernel(type, in, rows, tiles, count);
 }
 
+// The operand-ordered Q8_0 kernels (q8_mid.hip), chosen where the activation is quantised: from 2 to 512 rows that the decode
+// GEMV does not take (rows * K <= 32768, up to 8 rows; at 8 rows, us, GEMV / these: 4096x4096 10.4 / 11.5, 14336x4096 19.7 /
+// 20.7, 2048x2048 6.9 / 7.9; 4096x14336, which it does not take, at 4 rows 22.2 against the row kernel's 51.6). Up to 16 rows
+// of fewer than 512 inputs the MFMA kernel's one-wave workgroups are done before a split has paid (320x96 at 16 rows 4.5 /
+// 5.0, 512x512 5.9 / 5.4).
+bool use_q8_mid(const ovfq_ctx* c, int type, int in, int rows) {
+    return type == OVFQ_TYPE_Q8_0 && c->batched_kernel == OVFQ_BATCHED_AUTO && ovfq::mid_enabled() &&
+           ovfq::q8_0_mid_supported(1, in, rows) && (in >= 512 || rows > 16) && !(gemv_enabled() && ovfq::q8_0_gemv_rows_supported(in, rows));
+}
+
 // Whether the projection launch quantises its fp32 input itself instead of a separate Q8_K / Q8_0 launch: one row on
 // a decode kernel (K <= 8192), or up to 64 super-blocks of rows on the multi-row decode kernel.
 bool quantize_in_launch(const ovfq_ctx* c, int type, int in, int rows, int count, int pair_out = 0) {
@@ -405,7 +429,13 @@ int launch_projection(ovfq_ctx* c, const ovfq_weight* const* ws, int count, cons
         return fail(OVFQ_ERR_SIZE, "in-launch quantisation of %d rows needs the multi-row decode kernel", rows);
     // Every kernel below reads either the fp32 input (decode kernels that quantise it) or the quantised activation.
     if (!x && (!act.q || !act.s)) return fail(OVFQ_ERR_NULL, "projection launch without a quantised activation");
-    if (act.tiled) {
+    if (act.tiled && type == OVFQ_TYPE_Q8_0) {
+        for (int i = 0; i < count; i++) {
+            const int8_t* wq = reinterpret_cast<const int8_t*>(jobs[i].w);
+            HIP_TRY(ovfq::launch_q8_0_mid(&wq, &jobs[i].ws, 1, false, in, jobs[i].n_rows, rows, jobs[i].bias, act.q, act.s,
+                                          jobs[i].y, c->stream));
+        }
+    } else if (act.tiled) {
         if (use_mid(c, in, rows, ws, count) == ovfq::MidKernel::kPanel)
             HIP_TRY(ovfq::launch_project_panel(type, jobs, count, in, rows, act, c->stream));
         else
@@ -1016,7 +1046,8 @@ static int project_impl(ovfq_ctx* ctx, int count, const ovfq_weight* const* ws, 
             bd[i] = biases ? biases[i] : nullptr;
         }
     }
-    const bool tiled = use_mid(ctx, in, rows, ws, count) != ovfq::MidKernel::kNone;
+    const bool tiled = use_mid(ctx, in, rows, ws, count) != ovfq::MidKernel::kNone ||
+                       use_q8_mid(ctx, ws[0]->type, in, rows);
     if (!tiled && quantize_in_launch(ctx, ws[0]->type, in, rows, count,
                                      count == 2 && ws[0]->out == ws[1]->out ? ws[0]->out : 0)) {
         // Decode: the Q8_K quantisation happens inside the projection launch.
@@ -1234,7 +1265,7 @@ static int heads_impl(ovfq_ctx* ctx, int H, const ovfq_weight* const* wo, const 
     if (!host && ((rc = check_dev_align(x, "input")) || (rc = check_dev_align(y, "output")) ||
                   (rc = check_dev_align(bias, "bias"))))
         return rc;
-    // Batches from 32 rows: the int8-MFMA kernel streams each head's Wo once per 16-64 activation rows; fewer rows take
+    // Batches from 32 rows past those that q8_mid.hip takes (below): the int8-MFMA kernel streams each head's Wo once per 16-64 activation rows; fewer rows take
     // the decode kernel, one launch per 8 rows. MI355X, Llama-3-8B Wo (32 x 4096x128), graph replay, us, MFMA / per-8
     // launches: 9 rows 36.9 / 19.5, 16 rows 37.6 / 28.7, 32 rows 46.4 / 47.7, 64 rows 64.7 / 89.2, 512 rows 73.3 /
     // 628.8. OVFQ_HEADS_MFMA_MIN_ROWS sets the switch (measurements).
@@ -1249,6 +1280,12 @@ static int heads_impl(ovfq_ctx* ctx, int H, const ovfq_weight* const* wo, const 
     int R = 0;
     for (int r = rows < ovfq::kHeadsMaxRows ? rows : ovfq::kHeadsMaxRows; r >= 1 && !R && !mfma; r--)
         if (ovfq::q8_0_heads_supported(H, hd, r)) R = r;
+    // The operand-ordered kernels where they run (up to 512 rows) where the decode kernel needs a second launch, else
+    // from 6 rows of 2048 inputs and 8 rows of 512 (MI355X, us, decode launches / these: 32 x 4096x128 at 4 / 6 / 8 / 16 rows
+    // 10.6 / 12.4 / 18.1 / 27.0, 11.7 / 11.8 / 11.8 / 11.9; 14 x 896x64 at 6 / 8 / 9 rows 7.5 / 8.7 / 12.9, 7.8 / 7.8 / 7.8;
+    // 64 x 8192x128 at 4 / 5 rows, the second in two launches, 21.2 / 36.1, 25.9 / 25.9; 4 x 128x32 at 16 rows 10.7 / 5.7).
+    const bool mid = ctx->batched_kernel == OVFQ_BATCHED_AUTO && ovfq::mid_enabled() && ovfq::q8_0_mid_supported(H, hd, rows) &&
+                     (mfma || (R && (rows > R || rows >= (K >= 2048 ? 6 : K >= 512 ? 8 : 9))));
     if (!R && !mfma) return fail(OVFQ_ERR_SIZE, "n_heads x head_dim (%d) too large for one launch", K);
     std::lock_guard<std::mutex> lk(ctx->mu);
     HIP_TRY(hipSetDevice(ctx->device));
@@ -1273,6 +1310,12 @@ static int heads_impl(ovfq_ctx* ctx, int H, const ovfq_weight* const* wo, const 
         ws[h] = wo[h]->scales;
     }
     ovfq::ActQ act{nullptr, nullptr, nullptr};
+    if (mid) {
+        if ((rc = quantize_q8_tiled_into_scratch(ctx, xd, rows, H, hd, &act))) return rc;
+        HIP_TRY(ovfq::launch_q8_0_mid(wq, ws, H, true, hd, dm, rows, bd, act.q, act.s, yd, ctx->stream));
+        if (host && ((rc = io.down(y, yd, (size_t)rows * dm * 4)) || (rc = io.finish()))) return rc;
+        return ok();
+    }
     if (mfma) {
         if ((rc = quantize_into_scratch(ctx, OVFQ_TYPE_Q8_0, xd, rows, K, &act))) return rc;
         HIP_TRY(ovfq::launch_q8_0_heads_mfma(wq, ws, H, hd, dm, rows, bd, act, yd, ctx->stream));

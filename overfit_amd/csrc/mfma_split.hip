@@ -664,6 +664,14 @@ hipError_t launch_mfma_grouped(int type, const GroupLaunch& L, const int* tiles,
     return hipGetLastError();
 }
 
+bool mid_enabled() {
+    static const bool on = [] {
+        const char* v = getenv("OVFQ_SPLIT");
+        return !(v && *v == '0');
+    }();
+    return on;
+}
+
 // Which kernel takes a batch whose activation the library quantises itself. Measured on MI355X (graph replay with the
 // quantise launch, us: the kernel chosen otherwise / split / panel):
 //   Q4_K 4096x4096       16 rows  9.7 /  8.7 / 14.3   64 rows 22.8 / 13.1 / 22.3   128 rows 23.7 / 17.9 / 23.0   192 rows 24.1 / 24.3 / 23.7
@@ -682,11 +690,7 @@ hipError_t launch_mfma_grouped(int type, const GroupLaunch& L, const int* tiles,
 // 36, 3 rows 40 / 36, 16 rows 137 / 38). Very tall matrices at 5 to 8 rows stay on the expert-stream kernel (128256x2048
 // 38.5, panel 39.8), and at 3 and 4 rows, where the multi-row decode kernel takes 65 and 76, only a pair does.
 MidKernel mid_kernel(int type, int in, int rows, long tiles, int count) {
-    static const bool off = [] {
-        const char* v = getenv("OVFQ_SPLIT");
-        return v && *v == '0';
-    }();
-    if (off || (type != 12 && type != 14) || rows < 2 || in % kQK) return MidKernel::kNone;
+    if (!mid_enabled() || (type != 12 && type != 14) || rows < 2 || in % kQK) return MidKernel::kNone;
     if ((int64_t)in * 64 >= (int64_t)1 << 32) return MidKernel::kNone;  // 32-bit offsets into a workgroup's rows
     const long subs = (rows + 15) / 16, work = tiles * subs;
     const long panel_wgs = (tiles + 3) / 4 * ((subs + 3) / 4), wide_wgs = (tiles + 3) / 4 * ((rows + 127) / 128);

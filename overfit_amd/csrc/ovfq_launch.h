@@ -71,6 +71,7 @@ hipError_t launch_project_mfma(int type, const ProjJob* jobs, int njobs, int in,
 // kernel walks it with 64 weight rows a workgroup. mid_kernel: the automatic choice for `rows` activation rows against
 // `count` weights of `tiles` 16-row tiles in all (kNone: the kernels above and below).
 enum class MidKernel { kNone, kSplit, kPanel };
+bool mid_enabled();  // false with OVFQ_SPLIT=0 (measurements): neither these kernels nor those of q8_mid.hip
 MidKernel mid_kernel(int type, int in, int rows, long tiles, int count);
 hipError_t launch_project_split(int type, const ProjJob* jobs, int njobs, int in, int rows, ActQ act,
                                 hipStream_t st);
@@ -202,6 +203,18 @@ hipError_t launch_q8_0_heads(const int8_t* const* wq, const float* const* ws, in
 bool q8_0_heads_mfma_supported(int n_heads, int head_dim, int rows);
 hipError_t launch_q8_0_heads_mfma(const int8_t* const* wq, const float* const* ws, int n_heads, int head_dim,
                                   int d_model, int rows, const float* bias, ActQ act, float* y, hipStream_t st);
+// Both projections for 2 .. 512 rows from an operand-ordered Q8_0 activation (q8_mid.hip), bit-identical to the others: per 16
+// rows and group of up to four blocks of a plane (a whole weight, or one head's) kQ8TiledQ bytes of quants and kQ8TiledS
+// scales, q8_tiled_records(rows, planes, plane_in) of them.
+constexpr int kQ8TiledQ = 2048, kQ8TiledS = 64;
+inline size_t q8_tiled_records(int rows, int planes, int plane_in) {
+    return (size_t)((rows + 15) / 16) * (size_t)planes * (size_t)((plane_in / 32 + 3) / 4);
+}
+bool q8_0_mid_supported(int planes, int plane_in, int rows);
+hipError_t launch_quantize_q8_0_tiled(const float* x, int rows, int planes, int plane_in, int8_t* q, float* s,
+                                      hipStream_t st);
+hipError_t launch_q8_0_mid(const int8_t* const* wq, const float* const* ws, int planes, bool heads, int plane_in, int n_out,
+                           int rows, const float* bias, const int8_t* q, const float* s, float* y, hipStream_t st);
 
 // GGUF Q8_0 (34-byte blocks) -> int8 quant plane + f32 scale plane.
 hipError_t launch_q8_0_deinterleave(const void* gguf, int64_t n_blocks, int8_t* q, float* s, hipStream_t st);
