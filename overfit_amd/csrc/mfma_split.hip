@@ -21,6 +21,7 @@
 // With the quantise launch, before / after: 24 rows 40.1 / 23.1 us, 64 rows 75.6 / 30.2; Q4_K 4096x4096 at 64 rows 22.8 /
 // 13.0.
 #include <algorithm>
+#include <cmath>
 #include <cstdlib>
 
 #include "kquant_mfma.h"
@@ -376,8 +377,9 @@ __global__ __launch_bounds__(256, 2) void kquant_mfma_panel_kernel(const PanelAr
     constexpr int kInstr = (FS::kPieces + 3) / 4;
     __shared__ __align__(16) uint8_t ring[3][W][kSlot];
     __shared__ __align__(16) uint8_t act0[T * 4096], act1[T * 4096];
-    __shared__ __align__(16) uint8_t bs0[kMin ? W * 512 : 16], bs1[kMin ? W * 512 : 16];
-    __shared__ __align__(16) float sc0[W * 16], sc1[W * 16];
+    constexpr int kPerW = (T + W - 1) / W;  // tiles whose bsums and scales a wave brings in: wave, wave + W, ..
+    __shared__ __align__(16) uint8_t bs0[kMin ? kPerW * W * 512 : 16], bs1[kMin ? kPerW * W * 512 : 16];
+    __shared__ __align__(16) float sc0[kPerW * W * 16], sc1[kPerW * W * 16];
 
     const PArgs& a = args.p;
     const int wave = wave_id();
@@ -494,14 +496,16 @@ __global__ __launch_bounds__(256, 2) void kquant_mfma_panel_kernel(const PanelAr
                                                          (int)(b_src[0] + (uint32_t)sb * kStepB), 0, 0, 0);
         } else if constexpr (kMin) {
 #pragma unroll
-            for (int i = 0; i < 2; i++)
+            for (int i = 0; i < 2 * kPerW; i++)
                 __builtin_amdgcn_raw_ptr_buffer_load_lds(
-                    br, (__attribute__((address_space(3))) void*)(bs + wave * 512 + i * 256), 4,
-                    (int)(b_src[i] + (uint32_t)sb * kStepB), 0, 0, 0);
+                    br, (__attribute__((address_space(3))) void*)(bs + (wave + i / 2 * W) * 512 + i % 2 * 256), 4,
+                    (int)(b_src[i % 2] + (uint32_t)(i / 2 * W * spr + sb) * kStepB), 0, 0, 0);
         }
         if (lane < 16)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(sr, (__attribute__((address_space(3))) void*)(sc + wave * 16), 4,
-                                                     (int)(s_src + (uint32_t)sb * kStepS), 0, 0, 0);
+#pragma unroll
+            for (int i = 0; i < kPerW; i++)
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(sr, (__attribute__((address_space(3))) void*)(sc + (wave + i * W) * 16),
+                                                         4, (int)(s_src + (uint32_t)(i * W * spr + sb) * kStepS), 0, 0, 0);
     };
     const uint32_t slot_adr = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)&ring[0][wave][0] +
                               (uint32_t)(16 * FS::kPieces * r16);
@@ -599,9 +603,31 @@ static hipError_t launch_panel_t(const PanelArgs& pa, int T, hipStream_t st) {
         hipLaunchKernelGGL((kquant_mfma_panel_kernel<FS, 2, Src::kDense>), grid, wg, 0, st, pa);
     else if (T == 3)
         hipLaunchKernelGGL((kquant_mfma_panel_kernel<FS, 3, Src::kDense>), grid, wg, 0, st, pa);
-    else
+    else if (T == 4)
         hipLaunchKernelGGL((kquant_mfma_panel_kernel<FS, 4, Src::kDense>), grid, wg, 0, st, pa);
+    else if constexpr (FS::F::kNumMfma == 3)  // Q4_K: two workgroups' LDS still fit a CU
+        hipLaunchKernelGGL((kquant_mfma_panel_kernel<FS, 5, Src::kDense>), grid, wg, 0, st, pa);
     return hipGetLastError();
+}
+
+// 16-row activation tiles of a panel workgroup, and the launch's time by that choice in units of a Q4_K CU's time for one
+// tile over the inputs (3.0 us at 4096). By the busiest XCD: up to one workgroup a CU, whose waits nothing hides, takes
+// 3.9 / 4.8 / 6.1 / 7.6 at T = 2 .. 5; the two that run at once take T + 0.8 each, less where not every CU has the second; so do
+// further ones (q/k/v of 4096, us at T = 2 / 3 / 4 / 5: 96 rows 21.9 / 20.0 / 22.8 / 26.4, 160 rows 23.3 / 27.0 / 30.8 / 27.5,
+// 331 rows 44.8 / 41.1 / 46.6 / 39.4, 512 rows 54.7 / 59.4 / 50.6 / 56.4; gate/up of 14336 at 65 rows 50.1 / 48.1 / 55.1 / 39.6). Even shares of at
+// most four tiles for short inputs at over 400 rows, where the estimate fails (2304x2304 at 512 rows, T = 4 / 3 21.7 / 24.9),
+// and for Q6_K, whose operand build leaves a step of five units before its first tile.
+static double panel_cost(int type, int in, long o_tiles, long subs, int* T) {
+    const auto cost = [&](int t) {
+        const double w = (double)((o_tiles + 7) / 8 * ((subs + t - 1) / t)) / 32.0;
+        if (w <= 1.0) return 2.6 + 0.38 * t + 0.122 * t * t;
+        return (t + 0.8) * (w <= 2.0 ? 1.6 + 0.2 * w : std::ceil(w)) + (w > 2.0 ? 0.5 : 0.0);
+    };
+    *T = (int)((subs + (subs + 3) / 4 - 1) / ((subs + 3) / 4));
+    if (type == 12 && !(in < 4096 && subs > 25))
+        for (int t = (int)std::min(5l, subs); t >= 2; t--)
+            if (cost(t) < cost(*T)) *T = t;
+    return cost(*T);
 }
 
 hipError_t launch_project_panel(int type, const ProjJob* jobs, int njobs, int in, int rows, ActQ act,
@@ -621,8 +647,9 @@ hipError_t launch_project_panel(int type, const ProjJob* jobs, int njobs, int in
     pa.p.s = act.s;
     pa.p.b = act.bh;
     if (type == 12 && !pa.p.b) return hipErrorInvalidValue;  // the Q4_K kernel reads the bsums
-    pa.p.n_tiles = (pa.p.subs + 3) / 4;
-    const int T = (pa.p.subs + pa.p.n_tiles - 1) / pa.p.n_tiles;
+    int T;
+    panel_cost(type, in, tiles, pa.p.subs, &T);
+    pa.p.n_tiles = (pa.p.subs + T - 1) / T;
     return type == 12 ? launch_panel_t<SplitQ4K>(pa, T, st) : launch_panel_t<SplitQ6K>(pa, T, st);
 }
 
@@ -682,10 +709,17 @@ bool mid_enabled() {
 //   gate/up of 14336     16 rows 22.8 / 24.0 / 21.0   32 rows 45.7 / 31.6 / 23.8    64 rows 47.3 / 48.2 / 32.3   128 rows 50.6 / 87.0 / 56.1
 //   Q6_K 4096x14336      24 rows 40.0 / 23.7 / 64.2   64 rows 75.1 / 30.6 / 80.1   192 rows 92.4 / 66.2 / 81.8   384 rows  106 /  115 /  119
 //   Q6_K 14336x4096       8 rows 23.8 / 21.6 / 22.0   64 rows 37.5 / 33.8 / 29.6   160 rows 64.5 / 71.9 / 58.6   512 rows  127 /  172 /  121
-// So: the panel kernel on tall matrices (768 16-row tiles: it then has a workgroup for nearly every CU at any row count),
-// and on others from 65 rows, where the split kernel starts to read the weights twice, if it has a workgroup for
-// three of four CUs and (Q4_K) all of them run at once (q/k/v of 4096 at 331 rows, 576 workgroups: 41.2 / - / 45.6); the split kernel below that, while its work is small (weight tiles x activation tiles); beyond, and
-// where the wide (Q4_K) and pair-wide (Q6_K) kernels build each operand once for 128 rows, those of mfma.hip. Past the small-M
+// So: the panel kernel on tall matrices (768 16-row tiles: it then has a workgroup for nearly every CU at any row count) up to
+// 64 rows. On others the split kernel, while its work is small (weight tiles x activation tiles). Past 64 rows, where that
+// starts to read the weights twice, Q4_K takes the least of three estimates in panel_cost's units: the panel kernel's; 0.55
+// (0.48 from 8192 inputs) for 256 of the split kernel's 16 x 16 tiles (4096x4096 at 96 / 192 rows 14.9 / 24.3, 1024x14336 at
+// 400 rows 42.0); and those of mfma.hip, 4.5 + 6.3 for
+// 256 workgroups of the wide kernel (gate/up of 14336 at 128 / 256 / 512 rows 52.6 / 88.7 / 154) or 6.8 + 2.5 for 256 of the
+// 64-row kernel, which has more than two for each CU (q/k/v of 4096 at 331 / 512 rows 42.8 / 47.7, of 5120 at 331 rows 52.4;
+// with fewer it lost to the panel kernel at every size). us before / now: q/k/v of 4096 at 160 / 200 / 331 rows 30.8 / 31.5 /
+// 42.8, 23.3 / 28.0 / 39.4; 4096x4096 at 128 / 160 / 300 rows 18.2 / 23.1 / 31.9, 17.1 / 20.2 / 28.3; gate/up of 14336 at 65 /
+// 160 rows 48.5 / 79.1, 39.6 / 71.2. Q6_K takes the panel kernel where it has a workgroup for every CU and the split kernel's
+// work has grown, except where the pair-wide kernel builds each operand once for 128 rows. Past the small-M
 // kernel's input size, and below the tiled kernel's rows, the alternative is the general kernel (8192x28672 at 2 rows 33 /
 // 36, 3 rows 40 / 36, 16 rows 137 / 38). Very tall matrices at 5 to 8 rows stay on the expert-stream kernel (128256x2048
 // 38.5, panel 39.8), and at 3 and 4 rows, where the multi-row decode kernel takes 65 and 76, only a pair does.
@@ -697,18 +731,25 @@ MidKernel mid_kernel(int type, int in, int rows, long tiles, int count) {
     const bool pairwide = type == 14 && rows > 64 && wide_wgs >= 192 && wide_wgs <= 256;
     if (!mfma_small_supported(type, in) && rows < kMfmaMinRows)
         return rows == 2 ? MidKernel::kNone : tiles >= 768 ? MidKernel::kPanel : MidKernel::kSplit;
+    // short rows (a launch of one or two rounds) past one 64-row tile: q/k/v of 2304 at 143 rows (1674) 16.0 / 16.5
+    const long most = type == 14 ? 4096 : rows <= 64 || in >= 4096 ? 2880 : 1536;
+    if (type == 12 && rows > 64) {
+        const long o_tiles = (tiles + 3) / 4, grid64 = o_tiles * ((rows + 63) / 64), split_n = (subs + 3) / 4;
+        int T;
+        const double panel = rows <= 512 || work <= 8192 ? panel_cost(type, in, o_tiles, subs, &T) : 1e30;
+        const double split =
+            tiles < 768 && work <= most ? (in < 8192 ? 0.55 : 0.48) / 256 * (double)(tiles * split_n * ((subs + split_n - 1) / split_n)) : 1e30;
+        const double other = wide_wgs >= 448 ? 4.5 + 6.3 / 256 * (double)wide_wgs : grid64 > 512 ? 6.8 + 2.5 / 256 * (double)grid64 : 1e30;
+        if (panel < split && panel < 0.97 * other) return MidKernel::kPanel;
+        return split < other ? MidKernel::kSplit : MidKernel::kNone;
+    }
     if (tiles >= 768) {
         if (rows <= 4) return rows >= 3 && tiles >= 1536 && count == 1 ? MidKernel::kPanel : MidKernel::kNone;
         if (rows <= 8 && tiles >= 1536) return MidKernel::kNone;
-        const bool panel = type == 12 ? rows <= 64 || work <= 10752 : rows <= 512 && !pairwide;
-        return panel ? MidKernel::kPanel : MidKernel::kNone;
+        return type == 12 || (rows <= 512 && !pairwide) ? MidKernel::kPanel : MidKernel::kNone;
     }
     if (rows <= 8 && in > 1024 && in < 4096) return MidKernel::kNone;  // 2560x2560 at 8 rows: small-M 7.4, split 8.2
-    if (rows > 64 && (type == 12 ? panel_wgs >= 192 && panel_wgs <= 512 && work <= 8192
-                                 : panel_wgs >= 256 && work > 3584 && rows <= 512 && !pairwide))
-        return MidKernel::kPanel;
-    // short rows (a launch of one or two rounds) past one 64-row tile: q/k/v of 2304 at 143 rows (1674) 16.0 / 16.5
-    const long most = type == 14 ? 4096 : rows <= 64 || in >= 4096 ? 2880 : 1536;
+    if (rows > 64 && panel_wgs >= 256 && work > 3584 && rows <= 512 && !pairwide) return MidKernel::kPanel;
     return work <= most ? MidKernel::kSplit : MidKernel::kNone;
 }
 

@@ -124,6 +124,20 @@ def test_panel_projection_bit_exact(orc, fmt, rows, k, shapes):
         _check(y, _ref(orc, fmt, x, rows, blocks, k, shapes[i], biases[i]), f"job {i}")
 
 
+@pytest.mark.parametrize("rows,k,n", [
+    (75, 256, 27990),    # five activation tiles a workgroup, the last rows of the fifth and the last weight rows absent
+    (80, 512, 28100),    # five full tiles
+    (150, 512, 28672),   # two workgroups of five
+])
+def test_panel_of_five_tiles_bit_exact(orc, rows, k, n):
+    case("panel of five", rows, k, n)
+    rng = np.random.default_rng(rows + k + n)
+    blocks, w = _weight(rng, "q4k", n, k)
+    x, bias = normal(rng, (rows, k)), normal(rng, n)
+    y = ov.project(w, t(x).view(-1), rows=rows, bias=t(bias))
+    _check(y, _ref(orc, "q4k", x, rows, blocks, k, n, bias), "panel of five")
+
+
 @pytest.mark.parametrize("down", ["q4k", "q6k"])
 @pytest.mark.parametrize("E,k,rows", [(3, 2, 33), (2, 2, 130), (8, 3, 90), (4, 1, 300)])
 def test_panel_expert_groups_match_small_batches(E, k, rows, down):
