@@ -163,7 +163,8 @@ struct Q8Cursor {
 // flight. Bound by the block values' three vector operations: of 42.8 us at 4096x4096 and 512 rows some 6 go to the quantise
 // launch and 30 are left with the DMAs taken out. Eight waves a workgroup, each with half the rows, were no faster (512 rows
 // 43.4; 64 rows 20.6 instead of 19.5), nor were more groups in flight.
-template <int T, bool kHeads>
+// J: blocks of a group that are computed (planes of fewer than four blocks).
+template <int T, bool kHeads, int J = 4>
 __global__ __launch_bounds__(256, 2) void q8_0_panel_kernel(const Q8Args a) {
     __shared__ __align__(16) uint8_t ring[3][4][kQ8Slot];
     __shared__ __align__(16) uint8_t act0[T * 2048], act1[T * 2048], act2[T * 2048];
@@ -237,9 +238,9 @@ __global__ __launch_bounds__(256, 2) void q8_0_panel_kernel(const Q8Args a) {
             const u32x4 q1 = *reinterpret_cast<const u32x4*>(act + s * 2048 + 1024 + 16 * lane);
             const f32x16 sp = q8_scales(as_float(sc[s * 64 + lane] & in), b.scale);
             const i32x4 d[4] = {q8_mfma(q0.x, q0.y, b.b[0]), q8_mfma(q0.z, q0.w, b.b[1]), q8_mfma(q1.x, q1.y, b.b[2]),
-                                q8_mfma(q1.z, q1.w, b.b[3])};
+                                q8_mfma(q1.z, q1.w, b.b[3])};  // those past J are dropped by the compiler
 #pragma unroll
-            for (int j = 0; j < 4; j++)
+            for (int j = 0; j < J; j++)
 #pragma unroll
                 for (int i = 0; i < 4; i++) acc[s][i] += sp[4 * j + i] * (float)d[j][i];
         }
@@ -464,6 +465,17 @@ hipError_t launch_quantize_q8_0_tiled(const float* x, int rows, int planes, int 
     return hipGetLastError();
 }
 
+template <bool kHeads, int J>
+static hipError_t launch_panel_t(const Q8Args& a, int T, dim3 grid, hipStream_t st) {
+    if (T == 2)
+        hipLaunchKernelGGL((q8_0_panel_kernel<2, kHeads, J>), grid, dim3(256), 0, st, a);
+    else if (T == 3)
+        hipLaunchKernelGGL((q8_0_panel_kernel<3, kHeads, J>), grid, dim3(256), 0, st, a);
+    else
+        hipLaunchKernelGGL((q8_0_panel_kernel<4, kHeads, J>), grid, dim3(256), 0, st, a);
+    return hipGetLastError();
+}
+
 template <bool kHeads>
 static hipError_t launch_panel(Q8Args& a, hipStream_t st) {
     a.o_tiles = (a.n_out + 63) / 64;
@@ -473,7 +485,7 @@ static hipError_t launch_panel(Q8Args& a, hipStream_t st) {
     int T = 2;
     double best = 1e30;
     for (int t = 2; t <= 4; t++) {
-        const double n = (double)(((long)a.o_tiles * ((a.subs + t - 1) / t) + 255) / 256);
+        const double n = (double)(((long)((a.o_tiles + 7) / 8) * ((a.subs + t - 1) / t) + 31) / 32);  // of the busiest XCD
         const double cost = n * (t + 0.84) + (n == 1 ? 1.0 : 0.0);
         if (cost < best) {
             best = cost;
@@ -482,13 +494,10 @@ static hipError_t launch_panel(Q8Args& a, hipStream_t st) {
     }
     a.n_tiles = (a.subs + T - 1) / T;
     const dim3 grid((a.o_tiles + 7) / 8 * 8 * a.n_tiles);
-    if (T == 2)
-        hipLaunchKernelGGL((q8_0_panel_kernel<2, kHeads>), grid, dim3(256), 0, st, a);
-    else if (T == 3)
-        hipLaunchKernelGGL((q8_0_panel_kernel<3, kHeads>), grid, dim3(256), 0, st, a);
-    else
-        hipLaunchKernelGGL((q8_0_panel_kernel<4, kHeads>), grid, dim3(256), 0, st, a);
-    return hipGetLastError();
+    const int wnb = a.in / 32;
+    if constexpr (kHeads)
+        if (wnb < 4) return wnb < 3 ? launch_panel_t<true, 2>(a, T, grid, st) : launch_panel_t<true, 3>(a, T, grid, st);
+    return launch_panel_t<kHeads, 4>(a, T, grid, st);
 }
 
 template <bool kHeads>
@@ -502,7 +511,8 @@ static hipError_t launch_mid(Q8Args& a, hipStream_t st) {
     a.o_tiles = (a.n_out + 15) / 16;
     const int T = a.subs == 1 ? 1 : 2;
     a.n_tiles = (a.subs + T - 1) / T;
-    const long wgs = (long)a.o_tiles * a.n_tiles;
+    const long wgs = (long)((a.o_tiles + 7) / 8) * a.n_tiles * 8;  // as the busiest XCD has them (293x1088 at 370 rows, 228
+                                                                   // workgroups, 36 on three XCDs: 14.5, panel 9.8)
     if (wgs > 256 && (T == 2 || wgs > 512)) return launch_panel<kHeads>(a, st);
     const dim3 grid((a.o_tiles + 7) / 8 * 8 * a.n_tiles);
     if (wgs > 256 || ng <= 4) {

@@ -83,6 +83,8 @@ def test_project_bit_exact(orc, rows, k, n):
     (65, 3, 128, 4100),  # panel of 32 rows
     (150, 5, 96, 4031),  # panel of 48
     (120, 2, 160, 14330),  # panel of 64
+    (150, 3, 64, 4031),  # two of a group's four blocks computed
+    (65, 2, 32, 4100),   # one
 ])
 def test_heads_bit_exact(orc, rows, H, hd, dm):
     print("[case] q8 mid heads", rows, H, hd, dm, flush=True, file=sys.stderr)
