@@ -1281,11 +1281,12 @@ static int heads_impl(ovfq_ctx* ctx, int H, const ovfq_weight* const* wo, const 
     for (int r = rows < ovfq::kHeadsMaxRows ? rows : ovfq::kHeadsMaxRows; r >= 1 && !R && !mfma; r--)
         if (ovfq::q8_0_heads_supported(H, hd, r)) R = r;
     // The operand-ordered kernels where they run (up to 512 rows) where the decode kernel needs a second launch, else
-    // from 6 rows of 2048 inputs and 8 rows of 512 (MI355X, us, decode launches / these: 32 x 4096x128 at 4 / 6 / 8 / 16 rows
+    // from 6 rows of 4096 inputs and 8 rows of 512 (MI355X, us, decode launches / these: 32 x 4096x128 at 4 / 6 / 8 / 16 rows
     // 10.6 / 12.4 / 18.1 / 27.0, 11.7 / 11.8 / 11.8 / 11.9; 14 x 896x64 at 6 / 8 / 9 rows 7.5 / 8.7 / 12.9, 7.8 / 7.8 / 7.8;
+    // 16 x 2048x128 at 6 rows, eager calls, 8.6 / 10.0;
     // 64 x 8192x128 at 4 / 5 rows, the second in two launches, 21.2 / 36.1, 25.9 / 25.9; 4 x 128x32 at 16 rows 10.7 / 5.7).
     const bool mid = ctx->batched_kernel == OVFQ_BATCHED_AUTO && ovfq::mid_enabled() && ovfq::q8_0_mid_supported(H, hd, rows) &&
-                     (mfma || (R && (rows > R || rows >= (K >= 2048 ? 6 : K >= 512 ? 8 : 9))));
+                     (mfma || (R && (rows > R || rows >= (K >= 4096 ? 6 : K >= 512 ? 8 : 9))));
     if (!R && !mfma) return fail(OVFQ_ERR_SIZE, "n_heads x head_dim (%d) too large for one launch", K);
     std::lock_guard<std::mutex> lk(ctx->mu);
     HIP_TRY(hipSetDevice(ctx->device));
