@@ -97,8 +97,7 @@ OVFQ_API int ovfq_ctx_scratch_bytes(ovfq_ctx* ctx, size_t* live, size_t* retired
  * kernel does not take keep the automatic choice (routed experts: only SMALL / TILED apply). For Q8_0 weights,
  * TILED forces the tiled int8-MFMA kernel from 2 rows, ROWS the multi-row decode kernel (up to 8 rows, rows *
  * input_size <= 32768) and SMALL the row kernel (automatic: the decode kernel where it takes the shape, else the MFMA
- * kernel from 8 rows, for inputs up to 8192 from 6 rows, or from 4 with 8192 outputs or more). Every choice gives
- * bit-identical outputs. Counterpart of the reference's test-only A/B toggle
+ * kernels). Every choice gives bit-identical outputs. Counterpart of the reference's test-only A/B toggle
  * BatchedQuantProjection.UseWeightStationaryQ4K (RT/BatchedQuantProjection.cs:21-24): for parity tests and
  * benches that cover every kernel on one shape. */
 #define OVFQ_BATCHED_AUTO 0
@@ -269,9 +268,9 @@ OVFQ_API int ovfq_project_multi_prequantized_dev(ovfq_ctx* ctx, int count, const
  *   y[n] = bias (or zero), then for h = 0, 1, ..., n_heads - 1:  y[n] += Q8DotKernel.Project(x[n][h], wo[h]) (no bias)
  * — the per-head projections of RT/CachedSingleHeadAttention.cs:323-337 and the ascending head reduction of
  * RT/CachedMultiHeadAttention.cs:185-194, :292-297 (prefill rows: :600-614, :689-711), bit-identical. Up to 8 rows run
- * in one decode launch, up to 31 in launches of 8; batches of 32 rows or more (prefill) quantise the rows once and run
- * on int8 MFMA, each head's Wo streamed once per 64 rows (ovfq_ctx_set_batched_kernel: OVFQ_BATCHED_TILED forces that
- * kernel, SMALL / ROWS the decode launches). Replaces the n_heads separate projections plus the host sum. */
+ * in one decode launch; batches (from 6 to 9 rows on, by the input size) quantise the rows once and run on int8 MFMA
+ * (ovfq_ctx_set_batched_kernel: OVFQ_BATCHED_TILED forces the 64-row-tiled kernel, SMALL / ROWS the decode launches).
+ * Replaces the n_heads separate projections plus the host sum. */
 OVFQ_API int ovfq_project_heads_q8_0(ovfq_ctx* ctx, int n_heads, const ovfq_weight* const* wo, const float* x,
                                      int rows, const float* bias, float* y);
 OVFQ_API int ovfq_project_heads_q8_0_dev(ovfq_ctx* ctx, int n_heads, const ovfq_weight* const* wo, const float* x,

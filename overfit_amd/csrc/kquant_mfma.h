@@ -56,13 +56,6 @@ struct Q4KMfma {
         w.q[1] = ld4(r, off + 16 + 64 + 16 * g);
         return w;
     }
-    // The loads alone, and the block from them: a kernel that holds a block across a loop iteration keeps the loaded
-    // words (for Q6_K, before their byte shifts), so that nothing waits for them before they are used.
-    using Raw = W;
-    __device__ __forceinline__ static Raw load_raw(__amdgpu_buffer_rsrc_t r, uint32_t off, int g) {
-        return load(r, off, g);
-    }
-    __device__ __forceinline__ static W unpack(const Raw& w, uint32_t, int) { return w; }
     // The min MFMA's B operand for lane group g: m_{2g}, m_{2g}, m_{2g+1}, m_{2g+1} in fp16, from the eight 6-bit
     // mins (LD/GgmlDequant.cs:64-79 unpacking; lane group g takes sub-blocks 2g and 2g + 1).
     __device__ __forceinline__ static u32x2 min_operand(const W& w, int g) {
