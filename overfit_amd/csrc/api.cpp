@@ -368,7 +368,7 @@ bool use_gemv_rows(const ovfq_ctx* c, int type, int in, int rows, int count, int
 }
 
 // The split or the panel kernel (mfma_split.hip) for batches that the multi-row decode kernel does not take, by the shape
-// rule of mid_kernel. They read operand-ordered activation planes, so the choice is made where the activation is
+// rule of mid_rule.h. They read operand-ordered activation planes, so the choice is made where the activation is
 // quantised (the callers that quantise here; a caller's own quantised activation keeps the other kernels).
 ovfq::MidKernel use_mid(const ovfq_ctx* c, int in, int rows, const ovfq_weight* const* ws, int count) {
     const int type = ws[0]->type;
@@ -378,15 +378,7 @@ ovfq::MidKernel use_mid(const ovfq_ctx* c, int in, int rows, const ovfq_weight* 
     const int pair_out = count == 2 && ws[0]->out == ws[1]->out ? ws[0]->out : 0;
     long tiles = 0;
     for (int i = 0; i < count; i++) tiles += (ws[i]->out + 15) / 16;
-    // The multi-row decode kernel works through a row in items of 16 super-blocks; where the last item is mostly empty
-    // (5120 inputs: 20 of 32) these kernels take over at 3 rows, and for three or more weights at 2 (MI355X, us, multi-row /
-    // split kernel: 5120x5120 2 rows 9.5 / 10.6, 3 rows 11.2 / 10.7, q/k/v of 5120 inputs 2 rows 13.9 / 12.6, 6 rows 22.4 /
-    // 12.8; q/k/v of 4096 inputs, no empty part, 5 rows 10.2 / 10.8). It also loses on one very tall matrix (128256x2048 at 3
-    // rows 64.9, panel kernel 39.1).
-    const int spr = in / OVFQ_QK;
-    const bool short_item = spr > 16 && 2 * ((spr + 15) / 16 * 16) >= 3 * spr;
-    if (use_gemv_rows(c, type, in, rows, count, pair_out) && !(short_item && (rows >= 3 || count >= 3)) &&
-        !(rows >= 3 && count == 1 && tiles >= 1536))
+    if (use_gemv_rows(c, type, in, rows, count, pair_out) && !ovfq::mid_over_decode(type, in, rows, tiles, count))
         return ovfq::MidKernel::kNone;
     return ovfq::mid_kernel(type, in, rows, tiles, count);
 }

@@ -20,8 +20,6 @@
 // each other. Every further 16 rows add 3 us: the activation from L2 (0.9 MB a workgroup and 64 rows) and the exchange.
 // With the quantise launch, before / after: 24 rows 40.1 / 23.1 us, 64 rows 75.6 / 30.2; Q4_K 4096x4096 at 64 rows 22.8 /
 // 13.0.
-#include <algorithm>
-#include <cmath>
 #include <cstdlib>
 
 #include "kquant_mfma.h"
@@ -610,26 +608,6 @@ static hipError_t launch_panel_t(const PanelArgs& pa, int T, hipStream_t st) {
     return hipGetLastError();
 }
 
-// 16-row activation tiles of a panel workgroup, and the launch's time by that choice in units of a Q4_K CU's time for one
-// tile over the inputs (3.0 us at 4096). By the busiest XCD: up to one workgroup a CU, whose waits nothing hides, takes
-// 3.9 / 4.8 / 6.1 / 7.6 at T = 2 .. 5; the two that run at once take T + 0.8 each, less where not every CU has the second; so do
-// further ones (q/k/v of 4096, us at T = 2 / 3 / 4 / 5: 96 rows 21.9 / 20.0 / 22.8 / 26.4, 160 rows 23.3 / 27.0 / 30.8 / 27.5,
-// 331 rows 44.8 / 41.1 / 46.6 / 39.4, 512 rows 54.7 / 59.4 / 50.6 / 56.4; gate/up of 14336 at 65 rows 50.1 / 48.1 / 55.1 / 39.6). Even shares of at
-// most four tiles for short inputs at over 400 rows, where the estimate fails (2304x2304 at 512 rows, T = 4 / 3 21.7 / 24.9),
-// and for Q6_K, whose operand build leaves a step of five units before its first tile.
-static double panel_cost(int type, int in, long o_tiles, long subs, int* T) {
-    const auto cost = [&](int t) {
-        const double w = (double)((o_tiles + 7) / 8 * ((subs + t - 1) / t)) / 32.0;
-        if (w <= 1.0) return 2.6 + 0.38 * t + 0.122 * t * t;
-        return (t + 0.8) * (w <= 2.0 ? 1.6 + 0.2 * w : std::ceil(w)) + (w > 2.0 ? 0.5 : 0.0);
-    };
-    *T = (int)((subs + (subs + 3) / 4 - 1) / ((subs + 3) / 4));
-    if (type == 12 && !(in < 4096 && subs > 25))
-        for (int t = (int)std::min(5l, subs); t >= 2; t--)
-            if (cost(t) < cost(*T)) *T = t;
-    return cost(*T);
-}
-
 hipError_t launch_project_panel(int type, const ProjJob* jobs, int njobs, int in, int rows, ActQ act,
                                 hipStream_t st) {
     PanelArgs pa{};
@@ -699,58 +677,9 @@ bool mid_enabled() {
     return on;
 }
 
-// Which kernel takes a batch whose activation the library quantises itself. Measured on MI355X (graph replay with the
-// quantise launch, us: the kernel chosen otherwise / split / panel):
-//   Q4_K 4096x4096       16 rows  9.7 /  8.7 / 14.3   64 rows 22.8 / 13.1 / 22.3   128 rows 23.7 / 17.9 / 23.0   192 rows 24.1 / 24.3 / 23.7
-//   Q4_K 1024x14336      64 rows 59.8 / 24.1 /   -   512 rows 69.4 / 48.4 /   -
-//   Q4_K q/k/v of 4096   16 rows 24.2 / 11.3 / 14.5   64 rows 23.9 / 18.5 / 22.9    96 rows 24.0 / 21.3 / 20.2   192 rows 32.7 / 34.7 / 31.1
-//   Q4_K 8192x8192       16 rows 21.7 / 16.8 / 24.1   64 rows 41.6 / 29.0 / 38.3    96 rows 41.8 / 39.7 / 33.2   256 rows 60.3 / 84.5 / 56.0
-//   Q4_K 14336x4096       8 rows 17.6 / 17.1 / 15.6   32 rows 23.8 / 22.4 / 17.5    64 rows 25.1 / 31.5 / 23.9   192 rows 48.8 / 69.6 / 46.6
-//   gate/up of 14336     16 rows 22.8 / 24.0 / 21.0   32 rows 45.7 / 31.6 / 23.8    64 rows 47.3 / 48.2 / 32.3   128 rows 50.6 / 87.0 / 56.1
-//   Q6_K 4096x14336      24 rows 40.0 / 23.7 / 64.2   64 rows 75.1 / 30.6 / 80.1   192 rows 92.4 / 66.2 / 81.8   384 rows  106 /  115 /  119
-//   Q6_K 14336x4096       8 rows 23.8 / 21.6 / 22.0   64 rows 37.5 / 33.8 / 29.6   160 rows 64.5 / 71.9 / 58.6   512 rows  127 /  172 /  121
-// So: the panel kernel on tall matrices (768 16-row tiles: it then has a workgroup for nearly every CU at any row count) up to
-// 64 rows. On others the split kernel, while its work is small (weight tiles x activation tiles). Past 64 rows, where that
-// starts to read the weights twice, Q4_K takes the least of three estimates in panel_cost's units: the panel kernel's; 0.55
-// (0.48 from 8192 inputs) for 256 of the split kernel's 16 x 16 tiles (4096x4096 at 96 / 192 rows 14.9 / 24.3, 1024x14336 at
-// 400 rows 42.0); and those of mfma.hip, 4.5 + 6.3 for
-// 256 workgroups of the wide kernel (gate/up of 14336 at 128 / 256 / 512 rows 52.6 / 88.7 / 154) or 6.8 + 2.5 for 256 of the
-// 64-row kernel, which has more than two for each CU (q/k/v of 4096 at 331 / 512 rows 42.8 / 47.7, of 5120 at 331 rows 52.4;
-// with fewer it lost to the panel kernel at every size). us before / now: q/k/v of 4096 at 160 / 200 / 331 rows 30.8 / 31.5 /
-// 42.8, 23.3 / 28.0 / 39.4; 4096x4096 at 128 / 160 / 300 rows 18.2 / 23.1 / 31.9, 17.1 / 20.2 / 28.3; gate/up of 14336 at 65 /
-// 160 rows 48.5 / 79.1, 39.6 / 71.2. Q6_K takes the panel kernel where it has a workgroup for every CU and the split kernel's
-// work has grown, except where the pair-wide kernel builds each operand once for 128 rows. Past the small-M
-// kernel's input size, and below the tiled kernel's rows, the alternative is the general kernel (8192x28672 at 2 rows 33 /
-// 36, 3 rows 40 / 36, 16 rows 137 / 38). Very tall matrices at 5 to 8 rows stay on the expert-stream kernel (128256x2048
-// 38.5, panel 39.8), and at 3 and 4 rows, where the multi-row decode kernel takes 65 and 76, only a pair does.
 MidKernel mid_kernel(int type, int in, int rows, long tiles, int count) {
-    if (!mid_enabled() || (type != 12 && type != 14) || rows < 2 || in % kQK) return MidKernel::kNone;
-    if ((int64_t)in * 64 >= (int64_t)1 << 32) return MidKernel::kNone;  // 32-bit offsets into a workgroup's rows
-    const long subs = (rows + 15) / 16, work = tiles * subs;
-    const long panel_wgs = (tiles + 3) / 4 * ((subs + 3) / 4), wide_wgs = (tiles + 3) / 4 * ((rows + 127) / 128);
-    const bool pairwide = type == 14 && rows > 64 && wide_wgs >= 192 && wide_wgs <= 256;
-    if (!mfma_small_supported(type, in) && rows < kMfmaMinRows)
-        return rows == 2 ? MidKernel::kNone : tiles >= 768 ? MidKernel::kPanel : MidKernel::kSplit;
-    // short rows (a launch of one or two rounds) past one 64-row tile: q/k/v of 2304 at 143 rows (1674) 16.0 / 16.5
-    const long most = type == 14 ? 4096 : rows <= 64 || in >= 4096 ? 2880 : 1536;
-    if (type == 12 && rows > 64) {
-        const long o_tiles = (tiles + 3) / 4, grid64 = o_tiles * ((rows + 63) / 64), split_n = (subs + 3) / 4;
-        int T;
-        const double panel = rows <= 512 || work <= 8192 ? panel_cost(type, in, o_tiles, subs, &T) : 1e30;
-        const double split =
-            tiles < 768 && work <= most ? (in < 8192 ? 0.55 : 0.48) / 256 * (double)(tiles * split_n * ((subs + split_n - 1) / split_n)) : 1e30;
-        const double other = wide_wgs >= 448 ? 4.5 + 6.3 / 256 * (double)wide_wgs : grid64 > 512 ? 6.8 + 2.5 / 256 * (double)grid64 : 1e30;
-        if (panel < split && panel < 0.97 * other) return MidKernel::kPanel;
-        return split < other ? MidKernel::kSplit : MidKernel::kNone;
-    }
-    if (tiles >= 768) {
-        if (rows <= 4) return rows >= 3 && tiles >= 1536 && count == 1 ? MidKernel::kPanel : MidKernel::kNone;
-        if (rows <= 8 && tiles >= 1536) return MidKernel::kNone;
-        return type == 12 || (rows <= 512 && !pairwide) ? MidKernel::kPanel : MidKernel::kNone;
-    }
-    if (rows <= 8 && in > 1024 && in < 4096) return MidKernel::kNone;  // 2560x2560 at 8 rows: small-M 7.4, split 8.2
-    if (rows > 64 && panel_wgs >= 256 && work > 3584 && rows <= 512 && !pairwide) return MidKernel::kPanel;
-    return work <= most ? MidKernel::kSplit : MidKernel::kNone;
+    if (!mid_enabled() || (type != 12 && type != 14) || in % kQK) return MidKernel::kNone;
+    return mid_choice(type, in, rows, tiles, count);
 }
 
 hipError_t launch_project_split(int type, const ProjJob* jobs, int njobs, int in, int rows, ActQ act,

@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "mid_rule.h"
+
 namespace ovfq {
 
 constexpr int kMaxJobs = 4;
@@ -68,9 +70,8 @@ hipError_t launch_project_mfma(int type, const ProjJob* jobs, int njobs, int in,
                                hipStream_t st);
 // Batched K-quant projections from operand-ordered planes (act.tiled), any rows and K, bit-identical to
 // launch_project_kquant (mfma_split.hip): the split kernel divides the contraction over the waves of a workgroup, the panel
-// kernel walks it with 64 weight rows a workgroup. mid_kernel: the automatic choice for `rows` activation rows against
-// `count` weights of `tiles` 16-row tiles in all (kNone: the kernels above and below).
-enum class MidKernel { kNone, kSplit, kPanel };
+// kernel walks it with 64 weight rows a workgroup. mid_kernel: the automatic choice (mid_choice) for `rows` activation rows
+// against `count` weights of `tiles` 16-row tiles in all.
 bool mid_enabled();  // false with OVFQ_SPLIT=0 (measurements): neither these kernels nor those of q8_mid.hip
 MidKernel mid_kernel(int type, int in, int rows, long tiles, int count);
 hipError_t launch_project_split(int type, const ProjJob* jobs, int njobs, int in, int rows, ActQ act,

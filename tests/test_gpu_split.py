@@ -2,9 +2,10 @@
 dot per super-block and the reference's fp32 sum over the row (RT/Q4KDotKernel.cs:944-951, RT/Q6KDotKernel.cs:114-115).
 
 They take batches whose activation is quantised by the call, by a rule on rows and shapes; the shapes here lie on both
-sides of its tile edges: 3 .. 130 rows around multiples of 16 and 64, output counts off the 16-row tiles, one
+sides of its tile edges: 3 .. 150 rows around multiples of 16 and 64, output counts off the 16-row tiles, one
 super-block to one more than the small-M kernel takes, four and eight waves, odd Q6_K super-block counts (rows that start
-2, 4, .. 14 bytes past a 16-byte boundary), a last block that ends inside a 16-byte piece.
+2, 4, .. 14 bytes past a 16-byte boundary), a last block that ends inside a 16-byte piece. test_kernel_choice.py checks
+that the rule sends each list to the kernel that it names.
 """
 import sys
 
@@ -48,18 +49,22 @@ def _ref(orc, fmt, x, rows, blocks, k, n, bias):
     return (orc.q4k_project_batched if fmt == "q4k" else orc.q6k_project_batched)(x, rows, blocks, k, n, bias)
 
 
-@pytest.mark.parametrize("fmt", ["q4k", "q6k"])
-@pytest.mark.parametrize("rows,k,n", [
-    (9, 256, 33),      # one super-block: three of four waves idle
+SPLIT = [
+    (17, 256, 33),     # one super-block: three of four waves idle
     (3, 16640, 17),    # past the small-M kernel's inputs, from 3 rows; an incomplete last round of eight waves
     (5, 4352, 250),    # 17 super-blocks
-    (16, 2048, 48),    # exactly one tile, one round of eight waves
+    (16, 4096, 48),    # exactly one tile, two rounds of eight waves
     (17, 1792, 65),    # two tiles, four waves
     (33, 2304, 97),    # three tiles, two rounds
     (64, 2560, 16),    # four tiles
     (65, 3328, 31),    # two workgroups of three tiles, the last rows of the second absent
     (130, 768, 1000),  # nine tiles over three workgroups, four waves with one idle
-])
+]
+SPLIT_FUSED = [(2, 4352, [7000, 48, 130]), (40, 1024, [256, 64, 70, 16])]
+
+
+@pytest.mark.parametrize("fmt", ["q4k", "q6k"])
+@pytest.mark.parametrize("rows,k,n", SPLIT + [(9, 256, 33), (16, 2048, 48)])  # the last two stay on the small-M kernel
 def test_split_projection_bit_exact(orc, fmt, rows, k, n):
     case("split", fmt, rows, k, n)
     rng = np.random.default_rng(rows * 7919 + k + n)
@@ -69,10 +74,10 @@ def test_split_projection_bit_exact(orc, fmt, rows, k, n):
     _check(ov.project(w, t(x), rows=rows), _ref(orc, fmt, x, rows, blocks, k, n, None), "no bias")
 
 
-@pytest.mark.parametrize("rows,k,shapes", [(2, 4352, [128, 48, 50]), (40, 1024, [256, 64, 70, 16])])
+@pytest.mark.parametrize("rows,k,shapes", SPLIT_FUSED + [(2, 4352, [128, 48, 50])])
 def test_split_fused_projections_bit_exact(orc, rows, k, shapes):
     """Several weights in one launch, none a multiple of the tile (2 rows of 17 super-blocks: the launch that the multi-row
-    decode kernel's mostly empty last item would slow down)."""
+    decode kernel's mostly empty last item would slow down; with few outputs it stays there)."""
     case("split fused", rows, k, shapes)
     rng = np.random.default_rng(rows + k)
     made = [_weight(rng, "q4k", n, k) for n in shapes]
@@ -104,14 +109,19 @@ def test_split_ffn_intermediate_matches_separate_calls(down):
     assert torch.equal(y.view(torch.int32), ref.view(torch.int32))
 
 
-@pytest.mark.parametrize("fmt", ["q4k", "q6k"])
-@pytest.mark.parametrize("rows,k,shapes", [
+PANEL = [
     (5, 512, [12300]),           # tall, one tile: the weights' last 64-row group partial
     (17, 256, [12289]),          # one super-block, two tiles
     (48, 768, [6200, 6200]),     # an odd number of super-blocks, a gate/up pair
     (64, 512, [12288]),          # four full tiles
     (70, 1280, [4096, 512, 520]),  # not tall: two activation tiles of three, the last rows absent
-])
+    (150, 768, [14330]),           # three activation tiles of four, the last of two and ragged; the last weight rows absent
+    (250, 1280, [4000, 520]),      # four of four, an odd number of 210-byte blocks a row
+]
+
+
+@pytest.mark.parametrize("fmt", ["q4k", "q6k"])
+@pytest.mark.parametrize("rows,k,shapes", PANEL)
 def test_panel_projection_bit_exact(orc, fmt, rows, k, shapes):
     """The panel kernel (tall matrices; from 65 rows others): tile edges in both directions, one to five super-blocks."""
     case("panel", fmt, rows, k, shapes)
@@ -124,11 +134,14 @@ def test_panel_projection_bit_exact(orc, fmt, rows, k, shapes):
         _check(y, _ref(orc, fmt, x, rows, blocks, k, shapes[i], biases[i]), f"job {i}")
 
 
-@pytest.mark.parametrize("rows,k,n", [
+PANEL_OF_FIVE = [
     (75, 256, 27990),    # five activation tiles a workgroup, the last rows of the fifth and the last weight rows absent
     (80, 512, 28100),    # five full tiles
     (150, 512, 28672),   # two workgroups of five
-])
+]
+
+
+@pytest.mark.parametrize("rows,k,n", PANEL_OF_FIVE)
 def test_panel_of_five_tiles_bit_exact(orc, rows, k, n):
     case("panel of five", rows, k, n)
     rng = np.random.default_rng(rows + k + n)
