@@ -154,9 +154,10 @@ OVFQ_API int ovfq_weight_create_experts_gguf_dev(ovfq_ctx* ctx, int type, const 
                                                  int input_size, int output_size, int n_experts, ovfq_weight** out);
 OVFQ_API int ovfq_weight_destroy(ovfq_weight* w);
 /* Opt-in MFMA-ready copy of a Q6_K weight, written on the device: for every 16 output rows and super-block, the
- * int8 weight operands the batched (M >= 32) int8-MFMA kernel otherwise rebuilds from the GGUF bytes for every
- * activation tile, plus the block scale. Batched projections whose weights all have it skip that build; outputs
- * are bit-identical with or without it. Costs 8704 bytes per 16 rows and super-block (~2.5x the Q6_K bytes), freed
+ * int8 weight operands the tiled int8-MFMA kernel otherwise rebuilds from the GGUF bytes for every
+ * activation tile, plus the block scale. Batches of more than 128 rows whose weights all have it skip that build;
+ * smaller ones, and those of few outputs, mostly run on kernels that build each operand once for up to 64 rows and
+ * are faster than the copy. Outputs are bit-identical with or without it. Costs 8704 bytes per 16 rows and super-block (~2.5x the Q6_K bytes), freed
  * with the weight; the GGUF blocks stay resident for decode. Idempotent. For a Q4_K weight the call succeeds and
  * changes nothing (its operands are cheaper to build than to stream); other types: OVFQ_ERR_TYPE. The reference's
  * counterpart is its opt-in repacked CPU layout (RT/Q4KRepack.cs, RT/Q6KRepack.cs): a load-time layout change

@@ -377,10 +377,14 @@ ovfq::MidKernel use_mid(const ovfq_ctx* c, int in, int rows, const ovfq_weight* 
         return ovfq::MidKernel::kNone;
     const int pair_out = count == 2 && ws[0]->out == ws[1]->out ? ws[0]->out : 0;
     long tiles = 0;
-    for (int i = 0; i < count; i++) tiles += (ws[i]->out + 15) / 16;
+    bool prepared = true;
+    for (int i = 0; i < count; i++) {
+        tiles += (ws[i]->out + 15) / 16;
+        prepared = prepared && ws[i]->mfma;
+    }
     if (use_gemv_rows(c, type, in, rows, count, pair_out) && !ovfq::mid_over_decode(type, in, rows, tiles, count))
         return ovfq::MidKernel::kNone;
-    return ovfq::mid_kernel(type, in, rows, tiles, count);
+    return ovfq::mid_kernel(type, in, rows, tiles, count, prepared);
 }
 
 // The operand-ordered Q8_0 kernels (q8_mid.hip), chosen where the activation is quantised: from 2 to 512 rows that the decode

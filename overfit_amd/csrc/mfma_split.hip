@@ -677,9 +677,9 @@ bool mid_enabled() {
     return on;
 }
 
-MidKernel mid_kernel(int type, int in, int rows, long tiles, int count) {
+MidKernel mid_kernel(int type, int in, int rows, long tiles, int count, bool prepared) {
     if (!mid_enabled() || (type != 12 && type != 14) || in % kQK) return MidKernel::kNone;
-    return mid_choice(type, in, rows, tiles, count);
+    return mid_choice(type, in, rows, tiles, count, prepared);
 }
 
 hipError_t launch_project_split(int type, const ProjJob* jobs, int njobs, int in, int rows, ActQ act,

@@ -80,8 +80,14 @@ inline bool mid_over_decode(int type, int in, int rows, long tiles, int count) {
 // the alternative is the general kernel (8192x28672 at 2 rows 33 / 36, 3 rows 40 / 36, 16 rows 137 / 38). Very tall matrices at 5
 // to 8 rows stay on the expert-stream kernel (128256x2048 38.5, panel 39.8), and at 3 and 4 rows, where the multi-row decode
 // kernel takes 65 and 76, only a pair does.
+// Weights that all carry their MFMA-ready copy (`prepared`, Q6_K): the tiled kernel that reads it has no operands to build. Up
+// to 128 rows the split and panel kernels are the faster all the same (us, prepared / split / panel: 4096x14336 at 64 and 128
+// rows 77.4 / 32.2 / -, 87.8 / 49.3 / -, 14336x4096 at 64 rows 39.0 / - / 30.8, 28672x8192 at 128 rows 147 / - / 134); past that the
+// panel kernel loses (14336x4096 at 160 / 512 rows 54.2 / - / 59.5, 101 / - / 128, 8192x8192 at 512 rows 116 / - / 145) and the split
+// kernel wins as long as it has one pass (1024x14336 at 512 rows 88.0 / 53.8 / -, 4096x4096 at 160 / 200 rows 31.3 / 27.6 / -,
+// 31.6 / 32.6 / -, 2048x2048 at 256 / 400 rows 18.7 / 15.0 / -, 19.1 / 22.9 / -).
 // `in` % 256 == 0; `tiles`: 16-row weight tiles of the `count` weights.
-inline MidKernel mid_choice(int type, int in, int rows, long tiles, int count) {
+inline MidKernel mid_choice(int type, int in, int rows, long tiles, int count, bool prepared = false) {
     constexpr int kSmallMaxIn = 16384, kTiledMinRows = 32;
     if (rows < 2 || (int64_t)in * 64 >= (int64_t)1 << 32) return MidKernel::kNone;  // 32-bit offsets into a workgroup's rows
     const bool q6 = type == 14, tall = tiles >= 768;
@@ -106,6 +112,8 @@ inline MidKernel mid_choice(int type, int in, int rows, long tiles, int count) {
     const long units = spr == 4 ? 2560 : 1536;
     const bool split_fits = !tall && (is_short ? tiles * split_n * (split_t + 2) <= (q6 && spr > 1 ? 2 * units : units)
                                                : work <= (q6 ? 4096 : 2880));
+    if (prepared && rows > 128)
+        return split_fits && work <= (spr < 8 ? 1536 : is_short ? 2048 : 2560) ? MidKernel::kSplit : MidKernel::kNone;
     if (!q6 && rows > 64) {
         if (is_short && split_fits) return MidKernel::kSplit;
         int T;

@@ -71,9 +71,9 @@ hipError_t launch_project_mfma(int type, const ProjJob* jobs, int njobs, int in,
 // Batched K-quant projections from operand-ordered planes (act.tiled), any rows and K, bit-identical to
 // launch_project_kquant (mfma_split.hip): the split kernel divides the contraction over the waves of a workgroup, the panel
 // kernel walks it with 64 weight rows a workgroup. mid_kernel: the automatic choice (mid_choice) for `rows` activation rows
-// against `count` weights of `tiles` 16-row tiles in all.
+// against `count` weights of `tiles` 16-row tiles in all (prepared: every one with its MFMA-ready copy).
 bool mid_enabled();  // false with OVFQ_SPLIT=0 (measurements): neither these kernels nor those of q8_mid.hip
-MidKernel mid_kernel(int type, int in, int rows, long tiles, int count);
+MidKernel mid_kernel(int type, int in, int rows, long tiles, int count, bool prepared);
 hipError_t launch_project_split(int type, const ProjJob* jobs, int njobs, int in, int rows, ActQ act,
                                 hipStream_t st);
 hipError_t launch_project_panel(int type, const ProjJob* jobs, int njobs, int in, int rows, ActQ act,

@@ -62,8 +62,8 @@ class _ResidentWeight:
         return n.value
 
     def prepare_mfma(self):
-        """Adds the opt-in MFMA-ready copy of a Q6_K weight (ovfq_weight_prepare_mfma): batched projections
-        (M >= 32) then skip the per-block operand build, bit-identically, for ~2.5x the weight's bytes. A no-op for
+        """Adds the opt-in MFMA-ready copy of a Q6_K weight (ovfq_weight_prepare_mfma): batches of more
+        than 128 rows then skip the per-block operand build, bit-identically, for ~2.5x the weight's bytes. A no-op for
         Q4_K weights. Returns self."""
         raise_for_status(self._ctx.lib.ovfq_weight_prepare_mfma(self._ctx.handle, self.handle), self._ctx.lib)
         return self

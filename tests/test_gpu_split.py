@@ -89,6 +89,30 @@ def test_split_fused_projections_bit_exact(orc, rows, k, shapes):
         _check(y, _ref(orc, "q4k", x, rows, blocks, k, shapes[i], bias if i == 1 else None), f"job {i}")
 
 
+def test_prepared_weight_keeps_the_kernel_that_reads_its_copy(orc):
+    """200 rows of 512 inputs on the automatic choice: without its MFMA-ready copy the weight takes the split kernel, with it
+    the tiled one. Which ran shows in the scratch of a fresh context (operand-ordered planes are laid out in whole 16-row
+    tiles, row-major ones hold the bsums twice); the bits are the same."""
+    case("prepared")
+    rng = np.random.default_rng(12)
+    rows, k, n = 200, 512, 2048
+    blocks = set_subnormal_scales(random_q6k_blocks(rng, n * (k // 256)), q6=True).reshape(-1)
+    x = normal(rng, (rows, k))
+    ref = _ref(orc, "q6k", x, rows, blocks, k, n, None)
+    live = {}
+    for kind, prepare, kernel in (("plain", False, "auto"), ("prepared", True, "auto"), ("tiled", False, "tiled")):
+        ctx = ov.Context(0)
+        ctx.set_batched_kernel(kernel)
+        w = ov.Q6KWeight(blocks, k, n, ctx=ctx)
+        if prepare:
+            w.prepare_mfma()
+        _check(ov.project(w, t(x).view(-1), rows=rows), ref, kind)
+        live[kind] = ctx.scratch_bytes()[0]
+        del w
+        ctx.close()
+    assert live["prepared"] == live["tiled"] != live["plain"], live
+
+
 @pytest.mark.parametrize("down", ["q4k", "q6k"])
 def test_split_ffn_intermediate_matches_separate_calls(down):
     """The FFN's intermediate, quantised in the down kernel's operand order, against the same FFN with another kernel

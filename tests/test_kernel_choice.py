@@ -20,6 +20,9 @@ SOURCE = """
 extern "C" int choice(int type, int in, int rows, long tiles, int count) {
     return (int)ovfq::mid_choice(type, in, rows, tiles, count);
 }
+extern "C" int choice_prepared(int type, int in, int rows, long tiles, int count) {
+    return (int)ovfq::mid_choice(type, in, rows, tiles, count, true);
+}
 extern "C" int over_decode(int type, int in, int rows, long tiles, int count) {
     return ovfq::mid_over_decode(type, in, rows, tiles, count);
 }
@@ -42,7 +45,7 @@ def rule(tmp_path_factory):
                    check=True)
     lib = ctypes.CDLL(str(d / "rule.so"))
     args = [ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_long, ctypes.c_int]
-    lib.choice.argtypes = lib.over_decode.argtypes = args
+    lib.choice.argtypes = lib.choice_prepared.argtypes = lib.over_decode.argtypes = args
     lib.panel_tiles.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.c_long, ctypes.c_long]
     return lib
 
@@ -90,6 +93,19 @@ FASTER = [
 @pytest.mark.parametrize("fmt,k,rows,ns,kernel", FASTER)
 def test_short_and_small_batches_take_the_faster_kernel(rule, fmt, k, rows, ns, kernel):
     assert choose(rule, fmt, k, rows, ns) == kernel
+
+
+@pytest.mark.parametrize("k,n,rows,kernel", [
+    (4096, 14336, 64, "panel"), (4096, 14336, 160, "none"), (4096, 14336, 512, "none"), (8192, 28672, 128, "panel"),
+    (8192, 28672, 160, "none"), (8192, 8192, 320, "none"), (2048, 2048, 400, "none"), (2048, 2048, 256, "split"),
+    (14336, 4096, 64, "split"), (14336, 4096, 160, "split"), (14336, 4096, 256, "none"), (14336, 1024, 512, "split"),
+    (4096, 4096, 160, "split"), (4096, 4096, 200, "none"),
+])
+def test_prepared_weights_use_their_copy(rule, k, n, rows, kernel):
+    """Q6_K weights with the MFMA-ready copy: past 128 rows never the panel kernel, which builds the operands again."""
+    assert ("none", "split", "panel")[rule.choice_prepared(14, k, rows, (n + 15) // 16, 1)] == kernel
+    for r in range(129, 1100, 37):
+        assert rule.choice_prepared(14, k, r, (n + 15) // 16, 1) != 2
 
 
 @pytest.mark.parametrize("fmt", list(FORMATS))
