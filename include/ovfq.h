@@ -27,8 +27,8 @@
  *  - Scratch and HIP graphs: the context grows its device scratch on demand (activation quantisation, FFN and
  *    MoE intermediates, host staging) and never frees a superseded buffer before ovfq_ctx_destroy (or
  *    ovfq_ctx_release_retired), so a graph captured from _dev calls stays valid after later, larger calls on the
- *    same context. Work captured into a graph and work issued eagerly on the same context share that scratch:
- *    they must not run concurrently.
+ *    same context. A call that is itself being captured may grow it too. Work captured into a graph and work issued
+ *    eagerly on the same context share that scratch: they must not run concurrently.
  */
 #ifndef OVFQ_H
 #define OVFQ_H

@@ -99,7 +99,13 @@ int ensure(ovfq_ctx* c, DevBuf& b, size_t bytes) {
     if (cap < 2 * b.cap) cap = 2 * b.cap;
     cap = (cap + 255) & ~size_t(255);
     void* p = nullptr;
-    HIP_TRY(hipMalloc(&p, cap));
+    // The call may be captured (and the first of its size): an allocation is no stream work, but the runtime refuses it, and
+    // ends the capture, unless the thread's capture mode is relaxed.
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    HIP_TRY(hipThreadExchangeStreamCaptureMode(&mode));
+    const hipError_t e = hipMalloc(&p, cap);
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    HIP_TRY(e);
     if (b.p) {
         c->retired.push_back(b.p);
         c->retired_bytes += b.cap;

@@ -196,6 +196,64 @@ def test_graph_replay_after_scratch_growth(orc):
     ctx.close()
 
 
+@pytest.mark.parametrize("what", ["qkv", "heads"])
+def test_capture_of_a_call_that_grows_the_scratch(orc, what):
+    """Calls captured without an eager call of their size before: two rows of q/k/v of 5120 inputs on a fresh context (the
+    split kernel's activation planes; the multi-row decode kernel, which would take fewer outputs, needs none), and 512 rows
+    of heads of 32 inputs after 520 (their operand-ordered planes are four times the row-major ones of the larger batch).
+    Every replay, with eager work between, gives the oracle's bits."""
+    case("capture with growth", what)
+    ctx = ov.Context(0)
+    rng = np.random.default_rng(22)
+    if what == "qkv":
+        k, rows, shapes = 5120, 2, [5120, 1024, 1024]
+        blocks = [random_q4k_blocks(rng, n * k // 256).reshape(n, -1) for n in shapes]
+        ws = [ov.Q4KWeight(b, k, n, ctx=ctx) for b, n in zip(blocks, shapes)]
+        x = normal(rng, (rows, k))
+        refs = [orc.q4k_project_batched(x, rows, b, k, n, None) for b, n in zip(blocks, shapes)]
+    else:
+        H, hd, rows, shapes = 8, 32, 512, [64]
+        planes = [orc.q8_quantize_rows(normal(rng, (64, hd), 0.05)) for _ in range(H)]
+        ws = [ov.Q8Weight(q, s, hd, 64, ctx=ctx) for q, s in planes]
+        x = normal(rng, (rows, H * hd))
+        q, s = [p[0].reshape(64, hd) for p in planes], [p[1].reshape(64, 1) for p in planes]
+        refs = [orc.q8_project_heads(x, rows, q, s, hd, 64, None)]
+    xd = t(x)
+    ys = [torch.empty(rows * n, device=DEV) for n in shapes]
+    xl, yl = t(normal(rng, (520, 256))), torch.empty(520 * 64, device=DEV)
+
+    def step():
+        if what == "qkv":
+            ctx.project_multi_dev(ws, xd, ys, rows=rows)
+        else:
+            ov.project_heads_q8_0(ws, xd, rows=rows, out=ys[0])
+
+    side = torch.cuda.Stream()
+    ctx.set_stream(side.cuda_stream)
+    if what == "heads":
+        ov.project_heads_q8_0(ws, xl, rows=520, out=yl)
+    torch.cuda.synchronize()
+    before = ctx.scratch_bytes()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=side):
+        step()
+    ctx.set_stream(torch.cuda.current_stream().cuda_stream)
+    assert ctx.scratch_bytes() > before, "the captured call was to grow the scratch"
+    for rep in range(3):
+        for y in ys:
+            y.fill_(float("nan"))
+        g.replay()
+        torch.cuda.synchronize()
+        for y, ref in zip(ys, refs):
+            assert np.array_equal(y.cpu().numpy().view(np.uint32), ref.reshape(-1).view(np.uint32)), f"replay {rep}"
+        step()  # eager work between the replays
+        torch.cuda.synchronize()
+    del g, ws
+    import gc
+    gc.collect()
+    ctx.close()
+
+
 def test_moe_ffn_dev_into_host_mapped_output(orc):
     """ovfq_moe_ffn_dev with top-2 routing folds the combine into float atomics on y only when y is device
     memory; a y in pinned (host-mapped) memory takes the combine launch. Both give the same bits."""
