@@ -1448,8 +1448,16 @@ static int moe_impl(ovfq_ctx* ctx, int E, const ovfq_weight* const* gate, const 
     const bool small_ok = ovfq::mfma_small_supported(gt, dmodel) && ovfq::mfma_small_supported(dt, dff);
     const bool grouped_big = !small_ok || ctx->batched_kernel == OVFQ_BATCHED_TILED ||
                              (ctx->batched_kernel == OVFQ_BATCHED_AUTO && P >= (size_t)grouped_min * E);
+    // With more than a 64-row tile of pairs each, on average, the panel kernel's 16-row steps save little and the 64-row-tiled
+    // kernel's are shorter (MI355X, us, tiled / panel, 2048x4096 Q4_K experts: gate/up of 64 /
+    // 80 / 200 / 1024 pairs each on average 45.6 / 47.8, 56.2 / 62.8, 99 / 116, 446 / 516; Q6_K 58.6 / 62.8, 74.4 / 79.8, 138 / 149,
+    // 557 / 618; 768x3584 Q4_K, 160 pairs 61.0 / 77.0). The down projection, from operand-ordered planes there, stays longer on the
+    // panel kernel (Q4_K 80 / 128 / 256 pairs 40.0 / 30.2, 42.9 / 49.0, 67.5 / 73.2; Q6_K 128 / 256 / 512 61.2 / 59.2, 109 / 94.7, 160 / 160).
+    const bool forced_tiled = ctx->batched_kernel == OVFQ_BATCHED_TILED;
+    const bool gu_panel = grouped_big && !forced_tiled && P <= (size_t)64 * E;
+    const bool dn_panel = grouped_big && !forced_tiled && (dt == OVFQ_TYPE_Q6_K || P < (size_t)128 * E);
     const int max_tiles = (int)((P + ovfq::kGroupedTileRows - 1) / ovfq::kGroupedTileRows) + E;
-    // grouped_big: the intermediate in operand-ordered planes, every expert's pairs from a 16-row tile of their own on
+    // dn_panel: the intermediate in operand-ordered planes, every expert's pairs from a 16-row tile of their own on
     const size_t i_recs = (size_t)ovfq::grouped_subs((int)P, E) * (size_t)(dff / OVFQ_QK);
     auto carve = [&](Carver& c, int** off, int** prow, int** pof, int** pdst, float** pw, float** g, float** u, int8_t** iq,
                      float** is, int16_t** ib, float** out, float** hx, int** hidx, float** hw, float** hy,
@@ -1457,13 +1465,13 @@ static int moe_impl(ovfq_ctx* ctx, int E, const ovfq_weight* const* gate, const 
         *off = c.take<int>((size_t)(E + 2 + max_tiles) * 4);  // expert_off[E + 1], tile count, tile list
         *prow = c.take<int>(P * 4);
         *pof = c.take<int>(P * 4);
-        *pdst = c.take<int>(grouped_big ? P * 4 : 0);
+        *pdst = c.take<int>(dn_panel ? P * 4 : 0);
         *pw = c.take<float>(P * 4);
         *g = c.take<float>(P * dff * 4);
         *u = c.take<float>(P * dff * 4);
-        *iq = c.take<int8_t>(grouped_big ? i_recs * ovfq::kTiledQ : P * dff);
-        *is = c.take<float>(grouped_big ? i_recs * ovfq::kTiledS : P * (dff / OVFQ_QK) * 4);
-        *ib = c.take<int16_t>(grouped_big ? i_recs * ovfq::kTiledB : P * (dff / 16) * 2);
+        *iq = c.take<int8_t>(dn_panel ? i_recs * ovfq::kTiledQ : P * dff);
+        *is = c.take<float>(dn_panel ? i_recs * ovfq::kTiledS : P * (dff / OVFQ_QK) * 4);
+        *ib = c.take<int16_t>(dn_panel ? i_recs * ovfq::kTiledB : P * (dff / 16) * 2);
         *out = c.take<float>(P * dmodel * 4);
         if (host) {
             *hx = c.take<float>((size_t)rows * dmodel * 4);
@@ -1510,17 +1518,17 @@ static int moe_impl(ovfq_ctx* ctx, int E, const ovfq_weight* const* gate, const 
     int8_t* xq = (int8_t*)ctx->act_q.p;
     float* xs = (float*)ctx->act_s.p;
     int16_t* xb = (int16_t*)ctx->act_b.p;
-    const ovfq::ActQ act = grouped_big ? ovfq::ActQ{xq, xs, nullptr, (const uint16_t*)xb} : ovfq::ActQ{xq, xs, xb};
+    const ovfq::ActQ act = gu_panel ? ovfq::ActQ{xq, xs, nullptr, (const uint16_t*)xb} : ovfq::ActQ{xq, xs, xb};
     int* tile_count = off + E + 1;
     int* tiles = grouped_big ? off + E + 2 : nullptr;
-    if (!grouped_big) pdst = nullptr;
+    if (!dn_panel) pdst = nullptr;
     if (route)
         HIP_TRY(ovfq::launch_moe_route_plan(ld, rows, k, E, normalize, idxd, wd, off, prow, pof, ovfq::kGroupedTileRows,
                                             tiles, tile_count, pdst, xd, (int64_t)(n_x / OVFQ_QK), xq, xs, xb,
-                                            grouped_big, ctx->stream));
+                                            gu_panel, ctx->stream));
     else
         HIP_TRY(ovfq::launch_moe_plan(idxd, rows, k, E, off, prow, pof, ovfq::kGroupedTileRows, tiles, tile_count, pdst,
-                                      xd, (int64_t)(n_x / OVFQ_QK), xq, xs, xb, grouped_big, ctx->stream));
+                                      xd, (int64_t)(n_x / OVFQ_QK), xq, xs, xb, gu_panel, ctx->stream));
     const uint8_t* gw[OVFQ_MAX_EXPERTS];
     const uint8_t* uw[OVFQ_MAX_EXPERTS];
     const uint8_t* dw[OVFQ_MAX_EXPERTS];
@@ -1542,7 +1550,9 @@ static int moe_impl(ovfq_ctx* ctx, int E, const ovfq_weight* const* gate, const 
     L.pair_row = prow;
     L.act = act;
     L.pairs = (int)P;
-    if (grouped_big)
+    if (grouped_big && !gu_panel)
+        HIP_TRY(ovfq::launch_mfma_grouped_tiled(gt, L, tiles, tile_count, max_tiles, ctx->stream));
+    else if (gu_panel)
         HIP_TRY(ovfq::launch_mfma_grouped(gt, L, tiles, tile_count, max_tiles, ctx->stream));
     else
         HIP_TRY(ovfq::launch_mfma_small(gt, L, ctx->stream));
@@ -1555,7 +1565,7 @@ static int moe_impl(ovfq_ctx* ctx, int E, const ovfq_weight* const* gate, const 
     D.rows = (int)P;
     D.expert_off = off;
     D.pair_row = nullptr;  // the intermediate is already pair-major
-    D.act = grouped_big ? ovfq::ActQ{iq, is, nullptr, (const uint16_t*)ib, true} : ovfq::ActQ{iq, is, ib};
+    D.act = dn_panel ? ovfq::ActQ{iq, is, nullptr, (const uint16_t*)ib, true} : ovfq::ActQ{iq, is, ib};
     D.pairs = (int)P;
     // With top-1 / top-2 and the down projection on the small-M path (the expert-stream or small-M kernel), the
     // combine is folded into it: each token output gets at most two float-atomic adds onto zero, whose sum does not
@@ -1579,8 +1589,10 @@ static int moe_impl(ovfq_ctx* ctx, int E, const ovfq_weight* const* gate, const 
         D.comb_w = pw;
     }
     HIP_TRY(ovfq::launch_gate_up_q8k(g, u, off, E, (int)P, dff, false, iq, is, ib, ctx->stream, fold,
-                                     grouped_big ? dt : 0, (uint16_t*)ib, pdst));
-    if (grouped_big)
+                                     dn_panel ? dt : 0, (uint16_t*)ib, pdst));
+    if (grouped_big && !dn_panel)
+        HIP_TRY(ovfq::launch_mfma_grouped_tiled(dt, D, tiles, tile_count, max_tiles, ctx->stream));
+    else if (dn_panel)
         HIP_TRY(ovfq::launch_mfma_grouped(dt, D, tiles, tile_count, max_tiles, ctx->stream));
     else
         HIP_TRY(ovfq::launch_mfma_small(dt, D, ctx->stream));

@@ -5,7 +5,7 @@
 //   2. group the (token, top-k slot) pairs by expert, tokens ascending, and quantise
 //      the tokens' activation to Q8_K in the same launch                            -> moe_plan_kernel
 //   3. per expert: gate/up = batched projections of its tokens, all experts in one launch (mfma.hip: the
-//      expert-stream kernel for few pairs, else the small-M or panel MFMA kernel)
+//      expert-stream kernel for few pairs, else the small-M, panel or tiled MFMA kernel)
 //   4. SiLU(gate) * up, quantised to Q8_K for the down projection                    -> gate_up_q8k_kernel
 //   5. per expert: down projection of its pairs, one launch                      (mfma.hip, as step 3)
 //   6. y[token] = sum over top-k slots, in slot order, of weight * expert output     -> moe_combine_kernel

@@ -96,7 +96,7 @@ struct GroupLaunch {
     const int* pair_row;
     ActQ act;
     int pairs = 0;  // grouped launches: the pair count bound (rows x top_k), sizing the pair -> row map
-    // Grouped single-matrix launches only: instead of storing y0[pair][o], add
+    // Grouped single-matrix launch_mfma_small launches only: instead of storing y0[pair][o], add
     // comb_w[pair] * value to comb[comb_tok[pair]][o] with a float atomic (comb zeroed beforehand). Exact when at
     // most two pairs add to one output: (0 + a) + b == (0 + b) + a in fp32.
     float* comb = nullptr;
@@ -132,11 +132,15 @@ hipError_t launch_moe_route_plan(const float* logits, int rows, int k, int n_exp
                                  float* w, int* expert_off, int* pair_row, int* pair_of, int nt, int* tiles,
                                  int* tile_count, int* pair_dst, const float* x, int64_t n_blocks, int8_t* xq,
                                  float* xs, int16_t* xb, bool half16, hipStream_t st);
-// Expert groups of many pairs on the panel kernel (mfma_split.hip): tile list entry t covers rows [64 i, 64 i + 64) of
-// expert e's pairs; gate/up pairs (w1 set) share the launch, `comb` as in GroupLaunch. act: with pair_row the row-major planes
-// of the `rows` tokens, bsums as fp16 (act.bh); without, operand-ordered planes by pair_dst. Outputs are pair-major.
+// Expert groups of some pairs on the panel kernel (mfma_split.hip): tile list entry t covers rows [64 i, 64 i + 64) of
+// expert e's pairs; gate/up pairs (w1 set) share the launch. act: with pair_row the row-major planes of the `rows` tokens,
+// bsums as fp16 (act.bh); without, operand-ordered planes by pair_dst. Outputs are pair-major.
 hipError_t launch_mfma_grouped(int type, const GroupLaunch& launch, const int* tiles, const int* tile_count,
                                int max_tiles, hipStream_t st);
+// Expert groups of many pairs on the 64-row-tiled kernel (mfma.hip), the same tile list. act: row-major planes with int16
+// bsums, gathered through pair_row (NULL: pair p reads row p).
+hipError_t launch_mfma_grouped_tiled(int type, const GroupLaunch& launch, const int* tiles, const int* tile_count,
+                                     int max_tiles, hipStream_t st);
 constexpr int kGroupedTileRows = 64;
 // Work for a MoE step whose down projection adds into its output (GroupLaunch::comb), done in the launch before it:
 // y[0 .. y_len) = 0, and pw[pair_of[i]] = w[i] for the slots i < slots that hold a pair (pair_of[i] >= 0).

@@ -175,28 +175,33 @@ def test_panel_of_five_tiles_bit_exact(orc, rows, k, n):
     _check(y, _ref(orc, "q4k", x, rows, blocks, k, n, bias), "panel of five")
 
 
-@pytest.mark.parametrize("down", ["q4k", "q6k"])
-@pytest.mark.parametrize("E,k,rows", [(3, 2, 33), (2, 2, 130), (8, 3, 90), (4, 1, 300)])
-def test_panel_expert_groups_match_small_batches(E, k, rows, down):
-    """Expert groups on the panel kernel (16 and more pairs an expert) against the same tokens in batches that the stream and
-    small-M kernels take: every projection is bit-identical, and so are the outputs. Slots with an expert out of range or
-    repeated add nothing; expert 0 gets tokens in runs, so that groups end on and off the 16- and 64-row tiles."""
-    case("panel experts", E, k, rows, down)
+@pytest.mark.parametrize("gate,down", [("q4k", "q4k"), ("q4k", "q6k"), ("q6k", "q6k")])
+@pytest.mark.parametrize("E,k,rows,first", [
+    (3, 2, 33, 16), (8, 3, 90, 16),  # 16 to 64 pairs an expert: panel kernel both ways
+    (6, 2, 150, 90),                 # the same, expert 0 with a second, ragged 64-row tile
+    (4, 1, 300, 16),                 # 75: gate/up on the tiled kernel, down on the panel kernel
+    (2, 2, 130, 16),                 # 129: Q4_K down on the tiled kernel too
+])
+def test_expert_groups_match_small_batches(E, k, rows, first, gate, down):
+    """Expert groups on the panel and 64-row-tiled kernels (16 and more pairs an expert) against the same tokens in batches
+    that the stream and small-M kernels take: every projection is bit-identical, and so are the outputs. Slots with an
+    expert out of range or repeated add nothing; expert 0 gets a run of tokens, so that groups end on and off the tiles."""
+    case("experts", E, k, rows, gate, down)
     rng = np.random.default_rng(E * 100 + rows)
     d, ff = 512, 768
-    gate, up = ([_weight(rng, "q4k", ff, d)[1] for _ in range(E)] for _ in range(2))
+    gw, up = ([_weight(rng, gate, ff, d)[1] for _ in range(E)] for _ in range(2))
     dw = [_weight(rng, down, d, ff)[1] for _ in range(E)]
     x = normal(rng, (rows, d), 0.02)
     idx = rng.integers(0, E, (rows, k)).astype(np.int32)
-    idx[:16, 0] = 0
+    idx[:first, 0] = 0
     idx[5, k - 1] = E + 3
     idx[rows - 1, 0] = -1
     wt = rng.random((rows, k)).astype(np.float32)
-    y = ov.moe_ffn(gate, up, dw, t(x), rows, k, t(idx), t(wt)).reshape(rows, d)
+    y = ov.moe_ffn(gw, up, dw, t(x), rows, k, t(idx), t(wt)).reshape(rows, d)
     step = max(1, 8 * E // k - 1)
     for r in range(0, rows, step):
         m = min(step, rows - r)
-        ref = ov.moe_ffn(gate, up, dw, t(x[r:r + m]), m, k, t(idx[r:r + m]), t(wt[r:r + m])).reshape(m, d)
+        ref = ov.moe_ffn(gw, up, dw, t(x[r:r + m]), m, k, t(idx[r:r + m]), t(wt[r:r + m])).reshape(m, d)
         assert torch.equal(y[r:r + m].view(torch.int32), ref.view(torch.int32)), f"tokens {r} .. {r + m - 1}"
 
 
