@@ -393,14 +393,15 @@ ovfq::MidKernel use_mid(const ovfq_ctx* c, int in, int rows, const ovfq_weight* 
     return ovfq::mid_kernel(type, in, rows, tiles, count, prepared);
 }
 
-// The operand-ordered Q8_0 kernels (q8_mid.hip), chosen where the activation is quantised: from 2 to 512 rows that the decode
-// GEMV does not take (rows * K <= 32768, up to 8 rows; at 8 rows, us, GEMV / these: 4096x4096 10.4 / 11.5, 14336x4096 19.7 /
-// 20.7, 2048x2048 6.9 / 7.9; 4096x14336, which it does not take, at 4 rows 22.2 against the row kernel's 51.6). Up to 16 rows
-// of fewer than 512 inputs the MFMA kernel's one-wave workgroups are done before a split has paid (320x96 at 16 rows 4.5 /
-// 5.0, 512x512 5.9 / 5.4).
-bool use_q8_mid(const ovfq_ctx* c, int type, int in, int rows) {
-    return type == OVFQ_TYPE_Q8_0 && c->batched_kernel == OVFQ_BATCHED_AUTO && ovfq::mid_enabled() &&
-           ovfq::q8_0_mid_supported(1, in, rows) && (in >= 512 || rows > 16) && !(gemv_enabled() && ovfq::q8_0_gemv_rows_supported(in, rows));
+// The operand-ordered Q8_0 kernels (q8_mid.hip), chosen where the activation is quantised, for 2 to 512 rows by the rule of
+// mid_rule.h.
+bool use_q8_mid(const ovfq_ctx* c, int in, int rows, const ovfq_weight* const* ws, int count) {
+    if (ws[0]->type != OVFQ_TYPE_Q8_0 || c->batched_kernel != OVFQ_BATCHED_AUTO || !ovfq::mid_enabled() ||
+        !ovfq::q8_0_mid_supported(1, in, rows) || (gemv_enabled() && ovfq::q8_0_gemv_rows_supported(in, rows)))
+        return false;
+    int out = 0;
+    for (int i = 0; i < count; i++) out = ws[i]->out > out ? ws[i]->out : out;
+    return ovfq::q8_mid_choice(in, out, rows);
 }
 
 // Whether the projection launch quantises its fp32 input itself instead of a separate Q8_K / Q8_0 launch: one row on
@@ -1049,7 +1050,7 @@ static int project_impl(ovfq_ctx* ctx, int count, const ovfq_weight* const* ws, 
         }
     }
     const bool tiled = use_mid(ctx, in, rows, ws, count) != ovfq::MidKernel::kNone ||
-                       use_q8_mid(ctx, ws[0]->type, in, rows);
+                       use_q8_mid(ctx, in, rows, ws, count);
     if (!tiled && quantize_in_launch(ctx, ws[0]->type, in, rows, count,
                                      count == 2 && ws[0]->out == ws[1]->out ? ws[0]->out : 0)) {
         // Decode: the Q8_K quantisation happens inside the projection launch.

@@ -134,4 +134,18 @@ inline MidKernel mid_choice(int type, int in, int rows, long tiles, int count, b
     return tall && rows <= 512 ? MidKernel::kPanel : MidKernel::kNone;
 }
 
+// Whether the operand-ordered Q8_0 kernels (q8_mid.hip) take a batch that they support and the decode GEMV does not (rows * in <=
+// 32768, up to 8 rows; at 8 rows, us, GEMV / these: 4096x4096 10.4 / 11.5, 14336x4096 19.7 / 20.7, 2048x2048 6.9 / 7.9; 4096x14336,
+// which it does not take, at 4 rows 22.2 against the row kernel's 51.6). `out`: the outputs of the largest weight. Up to 16 rows
+// of fewer than 512 inputs (32 rows of one block) the MFMA kernel's one-wave workgroups are done before a split has paid (320x96
+// at 16 rows 4.5 / 5.0, 512x512 5.9 / 5.4, 502x32 at 17 rows 5.4 / 6.0). Rows of few blocks leave the panel kernel little to walk for its fixed share: with many outputs the 64 x 64
+// tile kernel is faster (us, that / these: 14146x32 at 146 rows 8.4 / 9.4, 4736x64 at 473 rows 8.5 / 9.4, 32729x320 at 214 rows 24.1 /
+// 27.2; 24718x672 at 179 rows 26.9 / 29.2, 18313x1216 at 375 rows 52.2 / 54.8; from 2048 inputs on
+// these won at every size).
+inline bool q8_mid_choice(int in, long out, int rows) {
+    if (in < 512 && rows <= (in < 64 ? 32 : 16)) return false;
+    const long outs = out * rows;
+    return in < 512 ? outs <= 1l << 20 : in < 2048 ? outs <= 3l << 20 : true;
+}
+
 }  // namespace ovfq

@@ -1,7 +1,7 @@
-"""The rule that sends K-quant batches to the split and panel kernels (overfit_amd/csrc/mid_rule.h), compiled for the host.
+"""The rules that send batches to the split and panel kernels (overfit_amd/csrc/mid_rule.h), compiled for the host.
 
-Its choice cannot be seen in the outputs, which are the same bits from every kernel. Checked here: the shapes by which
-test_gpu_split.py means to run a kernel do run it; batches that measured faster on the kernels used otherwise stay there; the
+Their choice cannot be seen in the outputs, which are the same bits from every kernel. Checked here: the shapes by which
+test_gpu_split.py and test_gpu_q8_mid.py mean to run a kernel do run it; batches that measured faster on the kernels used otherwise stay there; the
 bounds on which the kernels' addressing rests.
 """
 import ctypes
@@ -11,6 +11,7 @@ import subprocess
 
 import pytest
 
+import test_gpu_q8_mid as q8_mid
 import test_gpu_split as split
 
 CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "overfit_amd", "csrc")
@@ -26,6 +27,7 @@ extern "C" int choice_prepared(int type, int in, int rows, long tiles, int count
 extern "C" int over_decode(int type, int in, int rows, long tiles, int count) {
     return ovfq::mid_over_decode(type, in, rows, tiles, count);
 }
+extern "C" int q8_mid(int in, long out, int rows) { return ovfq::q8_mid_choice(in, out, rows); }
 extern "C" int panel_tiles(int type, int in, long o_tiles, long subs) {
     int T;
     ovfq::panel_cost(type, in, o_tiles, subs, &T);
@@ -46,6 +48,7 @@ def rule(tmp_path_factory):
     lib = ctypes.CDLL(str(d / "rule.so"))
     args = [ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_long, ctypes.c_int]
     lib.choice.argtypes = lib.choice_prepared.argtypes = lib.over_decode.argtypes = args
+    lib.q8_mid.argtypes = [ctypes.c_int, ctypes.c_long, ctypes.c_int]
     lib.panel_tiles.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.c_long, ctypes.c_long]
     return lib
 
@@ -106,6 +109,17 @@ def test_prepared_weights_use_their_copy(rule, k, n, rows, kernel):
     assert ("none", "split", "panel")[rule.choice_prepared(14, k, rows, (n + 15) // 16, 1)] == kernel
     for r in range(129, 1100, 37):
         assert rule.choice_prepared(14, k, r, (n + 15) // 16, 1) != 2
+
+
+def test_q8_0(rule):
+    for rows, k, n in q8_mid.PROJECT:
+        assert not (rows <= 8 and rows * k <= 32768)  # the decode kernel
+        assert rule.q8_mid(k, n, rows), (rows, k, n)
+    # measured faster on the 64 x 64 tile kernel by 5 to 20 %, or on these by 4 to 30 %
+    for k, n, rows in [(32, 14146, 146), (64, 4736, 473), (96, 21403, 499), (320, 32729, 214), (672, 24718, 179), (1216, 18313, 375)]:
+        assert not rule.q8_mid(k, n, rows), (k, n, rows)
+    for k, n, rows in [(128, 4096, 256), (320, 2000, 300), (1024, 4096, 512), (4096, 14336, 512), (14336, 4096, 300), (4096, 4096, 12)]:
+        assert rule.q8_mid(k, n, rows), (k, n, rows)
 
 
 @pytest.mark.parametrize("fmt", list(FORMATS))
