@@ -6,8 +6,8 @@
 // (RT/CachedMultiHeadAttention.cs:600-614, :689-710): each head's sum added to the running output in ascending order.
 //
 // A block is one v_mfma_i32_16x16x32_i8 per 16 x 16 tile. The scale products of four blocks come from one
-// v_mfma_f32_16x16x1_4b_f32 (sixteen products a lane, each a single multiplication added to zero: compared with v_mul_f32 on
-// 2 x 10^8 random pairs, subnormal factors and products, infinities and NaN among them, no value differed), which leaves the
+// v_mfma_f32_16x16x1_4b_f32 (sixteen products a lane, each a single multiplication added to zero, subnormal and non-finite
+// factors and products included: test_gpu_q8_mid.py compares a million pairs of any exponent), which leaves the
 // vector units a conversion, a multiplication and an addition per block value instead of those, the product and the loads of
 // its factors. A sum never is -0, so that blocks past a plane's end can be added as zeros.
 //

@@ -86,26 +86,39 @@ def test_heads_bit_exact(orc, H, hd, dm, rows):
         _check(y.cpu().numpy(), ref, f"bias={b is not None}")
 
 
-@pytest.mark.parametrize("H,hd,dm,rows", [
+HEADS_BATCHED = [
     (32, 128, 4096, 512),  # Llama-3-8B prefill: 512 rows, 64-row MFMA tiles
-    (32, 128, 4096, 32),   # the first automatic MFMA row count: 32-row tiles
+    (32, 128, 4096, 32),   # 32-row tiles
     (32, 128, 1000, 33),   # 64-row tiles with a partial last tile, partial output tile
     (8, 64, 200, 40),      # two blocks per head: every group partial
     (6, 96, 72, 37),       # three blocks per head
     (4, 256, 136, 70),     # eight blocks per head: two groups per head
     (3, 160, 24, 100),     # five blocks per head: a full group and a partial one
     (1, 32, 16, 64),       # one head of one block
-])
-def test_heads_batched_mfma_bit_exact(orc, H, hd, dm, rows):
-    case("heads mfma", H, hd, dm, rows)
+]
+# past the 512 rows of q8_mid.hip's kernels the automatic choice is the 64-row-tiled kernel too
+HEADS_LONG = [(5, 64, 200, 513), (3, 96, 72, 520), (2, 160, 136, 600), (32, 128, 1000, 530)]
+
+
+@pytest.mark.parametrize("kernel,H,hd,dm,rows", [(k, *s) for k in ("auto", "tiled") for s in HEADS_BATCHED] +
+                         [("auto", *s) for s in HEADS_LONG])
+def test_heads_batched_mfma_bit_exact(orc, kernel, H, hd, dm, rows):
+    """Batches on the automatic choice (up to 512 rows the kernels of q8_mid.hip) and on the 64-row-tiled MFMA kernel,
+    forced."""
+    case("heads mfma", kernel, H, hd, dm, rows)
+    ctx = ov.default_context()
     rng = np.random.default_rng(H * 11 + hd + dm + rows)
     qs, ss, ws = _heads(orc, rng, H, hd, dm)
     x = normal(rng, (rows, H * hd))
     x[rows - 1, -32:] = 0.0  # an all-zero block
     bias = normal(rng, dm)
     for b in (None, bias):
-        y = ov.project_heads_q8_0(ws, t(x), rows=rows, bias=None if b is None else t(b))
-        torch.cuda.synchronize()
+        ctx.set_batched_kernel(kernel)
+        try:
+            y = ov.project_heads_q8_0(ws, t(x), rows=rows, bias=None if b is None else t(b))
+            torch.cuda.synchronize()
+        finally:
+            ctx.set_batched_kernel("auto")
         ref = orc.q8_project_heads(x, rows, qs, ss, hd, dm, b)
         _check(y.cpu().numpy(), ref, f"bias={b is not None}")
 

@@ -224,10 +224,12 @@ def test_kquant_prefill_bit_exact(orc, ctx, batched, kernel, fmt, rows, k, n):
 
 
 @pytest.mark.parametrize("fmt", ["q4k", "q6k"])
-def test_kquant_prefill_128_row_tiles(orc, ctx, fmt):
-    """From 1024 rows the tiled kernel stages 128 activation rows per workgroup: 1100 rows (a partial last tile),
-    130 outputs (a partial 64-row weight tile), with a bias, before and after the MFMA-ready copy (Q6_K)."""
+def test_kquant_prefill_128_row_tiles(orc, ctx, batched, fmt):
+    """From 1024 rows the tiled kernel (forced: so few outputs go to the split kernel) stages 128 activation rows per
+    workgroup: 1100 rows (a partial last tile), 130 outputs (a partial 64-row weight tile), with a bias, before and after
+    the MFMA-ready copy (Q6_K)."""
     case("prefill 128-row tiles", fmt)
+    batched("tiled")
     rows, k, n = 1100, 512, 130
     rng = np.random.default_rng(1100)
     blocks = _kq_blocks(rng, fmt, n, k)
@@ -244,12 +246,13 @@ def test_kquant_prefill_128_row_tiles(orc, ctx, fmt):
 
 
 @pytest.mark.parametrize("rows,k,shapes", [(200, 512, [14300]), (129, 256, [14336]), (300, 256, [9000, 9000])])
-def test_kquant_prefill_wide_tiles(orc, ctx, rows, k, shapes):
-    """Q4_K launches whose 128-row grid reaches 448 workgroups take the wide tiled kernel (128 activation rows per
-    workgroup in two 64-row LDS halves): ragged last activation tiles (200, 129 and 300 rows), a partial last 64-row
+def test_kquant_prefill_wide_tiles(orc, ctx, batched, rows, k, shapes):
+    """Q4_K launches of the tiled kernel (forced: the automatic choice is the panel kernel for some of these) whose
+    128-row grid reaches 448 workgroups take its wide form (128 activation rows per workgroup in two 64-row LDS halves): ragged last activation tiles (200, 129 and 300 rows), a partial last 64-row
     weight tile, a fused pair, a bias; from the fp32 input (the quantiser's fp16 bsums) and from a prequantised
     activation whose bsums are not the group sums (the caller's int16 bsums read as the reference's Dot does)."""
     case("prefill wide tiles", rows, k, shapes)
+    batched("tiled")
     rng = np.random.default_rng(rows * 13 + k + sum(shapes))
     blocks = [_kq_blocks(rng, "q4k", n, k) for n in shapes]
     ws = [ov.Q4KWeight(b, k, n) for b, n in zip(blocks, shapes)]
@@ -277,12 +280,14 @@ def test_kquant_prefill_wide_tiles(orc, ctx, rows, k, shapes):
 
 @pytest.mark.parametrize("fmt,rows,k,shapes", [("q6k", 200, 768, [260]), ("q6k", 130, 3328, [250]),
                                                ("q4k", 256, 768, [4096, 1024, 1000]), ("q4k", 500, 1280, [4000])])
-def test_kquant_prefill_pair_kernel(orc, ctx, fmt, rows, k, shapes):
-    """Launches whose 64-row grid leaves each CU one or two tiles take the pair kernel (two waves per 16 weight rows
-    on alternate super-blocks, the odd wave's block values added by the even one in ascending order): an odd number of
-    super-blocks (3, 5: the last has no partner), partial weight and activation tiles, a multi-job launch, a bias; from
-    the fp32 input and, for Q4_K, a prequantised activation whose bsums are not the group sums."""
+def test_kquant_prefill_pair_kernel(orc, ctx, batched, fmt, rows, k, shapes):
+    """Launches of the tiled kernel (forced: fp32 inputs of these sizes go to the split and panel kernels, a caller's
+    quantised activation comes here) whose 64-row grid leaves each CU one or two tiles take the pair kernel (two waves per
+    16 weight rows on alternate super-blocks, the odd wave's block values added by the even one in ascending order): an odd
+    number of super-blocks (3, 5, 13: the last has no partner), partial weight and activation tiles, a multi-job launch, a
+    bias; from the fp32 input and from a prequantised activation, for Q4_K one whose bsums are not the group sums."""
     case("prefill pair kernel", fmt, rows, k, shapes)
+    batched("tiled")
     rng = np.random.default_rng(rows * 17 + k + sum(shapes))
     blocks = [_kq_blocks(rng, fmt, n, k) for n in shapes]
     Wt = ov.Q4KWeight if fmt == "q4k" else ov.Q6KWeight
@@ -297,15 +302,20 @@ def test_kquant_prefill_pair_kernel(orc, ctx, fmt, rows, k, shapes):
     torch.cuda.synchronize()
     for i, (y, ref) in enumerate(zip(ys, refs)):
         assert_bit_exact(y.cpu().numpy().reshape(rows, -1), ref, f"pair kernel {fmt} rows={rows} job {i}")
-    if fmt != "q4k":
-        return
     q, s, b = orc.quantize_q8k(x)
+    y = torch.empty(rows * shapes[0], device=DEV)
+    batched("auto")
+    if fmt != "q4k":
+        ctx.project_prequantized_dev(ws[0], t(q), t(s), t(b), y, rows=rows)
+        torch.cuda.synchronize()
+        ref = proj(x, rows, blocks[0], k, shapes[0], None)
+        assert_bit_exact(y.cpu().numpy().reshape(rows, -1), ref, f"pair kernel {fmt} prequantized rows={rows}")
+        return
     b = (b.astype(np.int32) + rng.integers(-9, 10, b.shape)).clip(-2048, 2048).astype(np.int16)
     ref = np.zeros((rows, shapes[0]), np.float32)
     rc = orc.lib().orc_q4k_project_batched_prequantized(rows, orc.P(np.ascontiguousarray(blocks[0], np.uint8)), k,
                                                          shapes[0], None, orc.P(ref), orc.P(q), orc.P(s), orc.P(b))
     assert rc == 0
-    y = torch.empty(rows * shapes[0], device=DEV)
     ctx.project_prequantized_dev(ws[0], t(q), t(s), t(b), y, rows=rows)
     torch.cuda.synchronize()
     assert_bit_exact(y.cpu().numpy().reshape(rows, -1), ref, f"pair kernel prequantized shifted bsums rows={rows}")
@@ -676,8 +686,9 @@ def test_stream_kernel_dense_q6k_bit_exact(orc, batched, rows, k, n):
 @pytest.mark.parametrize("rows", [2, 3, 4, 5])
 def test_gate_up_pair_rows_boundary_bit_exact(orc, ctx, rows):
     """A gate/up-shaped Q4_K pair tall enough for the expert-stream kernel (6144 rows each: 768 16-row tiles) under
-    the automatic choice: 2 rows on the multi-row decode kernel, from 3 rows on the stream kernel; each output
-    bit-exact against the oracle, both through the fp32 entry point and the prequantised one."""
+    the automatic choice: 2 rows on the multi-row decode kernel, 3 and 4 on the stream kernel, 5 on the panel kernel (the
+    stream kernel from a quantised activation); each output bit-exact against the oracle, both through the fp32 entry point
+    and the prequantised one."""
     case("gate/up pair boundary", rows)
     n, k = 6144, 256
     rng = np.random.default_rng(600 + rows)
@@ -689,7 +700,13 @@ def test_gate_up_pair_rows_boundary_bit_exact(orc, ctx, rows):
     ctx.project_multi_dev([wg, wu], t(x), [g, u], rows=rows)
     torch.cuda.synchronize()
     assert_bit_exact(g.cpu().numpy().reshape(rows, n), orc.q4k_project_batched(x, rows, bg, k, n, None), "pair gate")
-    assert_bit_exact(u.cpu().numpy().reshape(rows, n), orc.q4k_project_batched(x, rows, bu, k, n, None), "pair up")
+    ref_u = orc.q4k_project_batched(x, rows, bu, k, n, None)
+    assert_bit_exact(u.cpu().numpy().reshape(rows, n), ref_u, "pair up")
+    q, s, b = orc.quantize_q8k(x)
+    u.fill_(float("nan"))
+    ctx.project_multi_prequantized_dev([wg, wu], t(q), t(s), t(b), [g, u], rows=rows)
+    torch.cuda.synchronize()
+    assert_bit_exact(u.cpu().numpy().reshape(rows, n), ref_u, "pair up prequantised")
 
 
 def test_moe_ffn_skewed_routing(orc):
@@ -1035,10 +1052,12 @@ def test_moe_ffn_many_tokens(orc):
     _moe_check(y.cpu().numpy(), ref, "300 tokens top-3")
 
 
-def test_moe_ffn_grouped_tile_boundaries(orc):
-    """Many pairs per expert take the batched MFMA kernel over 64-row expert tiles: an expert with exactly 64 pairs
-    (one full tile), one with 66 (a full tile and a 2-row tile), one with none."""
-    case("moe grouped tiles", 130)
+@pytest.mark.parametrize("kernel", ["auto", "tiled"])
+def test_moe_ffn_grouped_tile_boundaries(orc, batched, kernel):
+    """Many pairs per expert take the panel kernel, or, forced, the tiled one, over 64-row expert tiles: an expert with
+    exactly 64 pairs (one full tile), one with 66 (a full tile and a 2-row tile), one with none."""
+    case("moe grouped tiles", 130, kernel)
+    batched(kernel)
     rng = np.random.default_rng(130)
     E, dm, dff, rows, k = 3, 256, 256, 130, 1
     gb = [orc.quantize_q4k(normal(rng, (dff, dm), 0.05)) for _ in range(E)]
@@ -1147,8 +1166,8 @@ def test_kquant_long_rows_bit_exact(orc, fmt, rows):
 
 
 # Row counts on both sides of every threshold of the automatic kernel choice: one-row GEMV, multi-row decode kernel
-# (up to 4 rows; 8 for fused launches), small-M MFMA kernel, tiled MFMA kernel (grid >= 96 workgroups, or from 81 /
-# 97 rows), and past K = 16384 the general kernel below 32 rows.
+# (up to 4 rows; 8 for fused launches), small-M MFMA kernel (up to 16 rows of so few outputs), split kernel at each
+# height, and past K = 16384 the general kernel at 2 rows and the split kernel from 3.
 DISPATCH_ROWS = {2304: [1, 2, 3, 4, 5, 8, 9, 15, 16, 17, 31, 32, 33, 64, 65, 80, 81, 96, 97, 112, 113, 129],
                  16640: [1, 2, 4, 9, 31, 32, 33, 70]}
 
@@ -1173,11 +1192,11 @@ def test_automatic_choice_boundaries_bit_exact(orc, ctx, fmt, k):
 
 
 @pytest.mark.parametrize("kernel,rows,k", [("tiled", 48, 1024), ("small", 48, 1024), ("rows", 8, 1024),
-                                           ("auto", 1, 28672)])
+                                           ("auto", 48, 1024), ("auto", 1, 28672)])
 @pytest.mark.parametrize("fmt", ["q4k", "q6k"])
 def test_kquant_prefill_range_extremes(orc, batched, kernel, rows, k, fmt):
-    """Operand range extremes (every quant +-127, the largest scales and mins) on both MFMA kernels, the multi-row
-    decode kernel (8 rows) and its one-row use for long rows (K = 28672)."""
+    """Operand range extremes (every quant +-127, the largest scales and mins) on the tiled, small-M and split MFMA
+    kernels (48 rows), the multi-row decode kernel (8 rows) and its one-row use for long rows (K = 28672)."""
     case("prefill extremes", kernel, rows, k, fmt)
     batched(kernel)
     n = 64

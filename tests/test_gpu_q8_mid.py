@@ -101,3 +101,26 @@ def test_heads_bit_exact(orc, rows, H, hd, dm):
         torch.cuda.synchronize()
         ref = orc.q8_project_heads(x, rows, [q for q, _ in planes], [s for _, s in planes], hd, dm, b)
         _check(y, ref, f"bias={b is not None}")
+
+
+def test_scale_products_of_any_exponent(orc):
+    """One block a row, so that an output is one (wScale * aScale) * dot: the matrix unit's scale products against the
+    oracle's float multiplication for 512 x 2040 pairs of scales with random sign, exponent and fraction, subnormal,
+    infinite and NaN ones among them, and products past either end of the range."""
+    print("[case] q8 mid scale products", flush=True, file=sys.stderr)
+    rng = np.random.default_rng(31)
+    rows, k, n = 512, 32, 2040
+    bits = rng.integers(0, 1 << 32, size=n, dtype=np.uint64).astype(np.uint32)
+    bits[:64] &= np.uint32(0x807FFFFF)  # subnormal
+    s = bits.view(np.float32).reshape(n, 1)
+    s[64:68, 0] = np.inf, -np.inf, np.nan, 0.0
+    q = rng.integers(-128, 128, size=(n, k), dtype=np.int8)
+    q[:, 0] = np.where(q[:, 0] == 0, 1, q[:, 0])
+    x = np.zeros((rows, k), np.float32)  # a row's largest element gives its scale
+    exponents = rng.integers(1, 255, size=rows, dtype=np.uint32) << 23
+    x[:, 0] = (exponents | rng.integers(0, 1 << 23, size=rows, dtype=np.uint32)).view(np.float32)
+    x[:, 1:] = x[:, :1] * rng.uniform(-1, 1, size=(rows, k - 1)).astype(np.float32)
+    w = ov.Q8Weight(q.reshape(-1), s.reshape(-1), k, n)
+    y = ov.project(w, t(x).view(-1), rows=rows)
+    torch.cuda.synchronize()
+    _check(y, orc.q8_project_batched(x, rows, q, s, k, n, None), "scale products")

@@ -112,7 +112,7 @@ def test_prepared_weights_use_their_copy(rule, k, n, rows, kernel):
 
 
 def test_q8_0(rule):
-    for rows, k, n in q8_mid.PROJECT:
+    for rows, k, n in q8_mid.PROJECT + [(512, 32, 2040)]:
         assert not (rows <= 8 and rows * k <= 32768)  # the decode kernel
         assert rule.q8_mid(k, n, rows), (rows, k, n)
     # measured faster on the 64 x 64 tile kernel by 5 to 20 %, or on these by 4 to 30 %
