@@ -626,7 +626,7 @@ hipError_t launch_project_panel(int type, const ProjJob* jobs, int njobs, int in
     pa.p.b = act.bh;
     if (type == 12 && !pa.p.b) return hipErrorInvalidValue;  // the Q4_K kernel reads the bsums
     int T;
-    panel_cost(type, in, tiles, pa.p.subs, &T);
+    panel_cost(type, tiles, pa.p.subs, &T);
     pa.p.n_tiles = (pa.p.subs + T - 1) / T;
     return type == 12 ? launch_panel_t<SplitQ4K>(pa, T, st) : launch_panel_t<SplitQ6K>(pa, T, st);
 }

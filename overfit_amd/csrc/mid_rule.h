@@ -14,17 +14,18 @@ enum class MidKernel { kNone, kSplit, kPanel };  // kNone: the kernels of gemv.h
 // tile over the inputs (3.0 us at 4096). By the busiest XCD: up to one workgroup a CU, whose waits nothing hides, takes
 // 3.9 / 4.8 / 6.1 / 7.6 at T = 2 .. 5; the two that run at once take T + 0.8 each, less where not every CU has the second; so do
 // further ones (q/k/v of 4096, us at T = 2 / 3 / 4 / 5: 96 rows 21.9 / 20.0 / 22.8 / 26.4, 160 rows 23.3 / 27.0 / 30.8 / 27.5,
-// 331 rows 44.8 / 41.1 / 46.6 / 39.4, 512 rows 54.7 / 59.4 / 50.6 / 56.4; gate/up of 14336 at 65 rows 50.1 / 48.1 / 55.1 / 39.6). Even shares of at
-// most four tiles for short inputs at over 400 rows, where the estimate fails (2304x2304 at 512 rows, T = 4 / 3 21.7 / 24.9),
-// and for Q6_K, whose operand build leaves a step of five units before its first tile.
-inline double panel_cost(int type, int in, long o_tiles, long subs, int* T) {
+// 331 rows 44.8 / 41.1 / 46.6 / 39.4, 512 rows 54.7 / 59.4 / 50.6 / 56.4; gate/up of 14336 at 65 rows 50.1 / 48.1 / 55.1 / 39.6;
+// 2304x2304 at 512 rows 21.6 / 20.7 / 22.3 / 25.3, 3072x1024 17.6 / 19.8 / 22.0 / 25.0; over 1600 random shapes of 1024 to 6400 inputs
+// and 300 to 1100 rows where it differs from even shares of at most four tiles, its choice took 0.90 of their time and 1.002 of
+// the best height's). Even shares for Q6_K, whose operand build leaves a step of five units before its first tile.
+inline double panel_cost(int type, long o_tiles, long subs, int* T) {
     const auto cost = [&](int t) {
         const double w = (double)((o_tiles + 7) / 8 * ((subs + t - 1) / t)) / 32.0;
         if (w <= 1.0) return 2.6 + 0.38 * t + 0.122 * t * t;
         return (t + 0.8) * (w <= 2.0 ? 1.6 + 0.2 * w : std::ceil(w)) + (w > 2.0 ? 0.5 : 0.0);
     };
     *T = (int)((subs + (subs + 3) / 4 - 1) / ((subs + 3) / 4));
-    if (type == 12 && !(in < 4096 && subs > 25))
+    if (type == 12)
         for (int t = (int)std::min(5l, subs); t >= 2; t--)
             if (cost(t) < cost(*T)) *T = t;
     return cost(*T);
@@ -58,9 +59,10 @@ inline bool mid_over_decode(int type, int in, int rows, long tiles, int count) {
 // From 4096 inputs on: the panel kernel on tall matrices (768 16-row tiles: it then has a workgroup for nearly every CU at any
 // row count) up to 64 rows; on others the split kernel, while its work (weight tiles x activation tiles) is small. Shorter
 // inputs give the split kernel's four waves a few rounds each, the last one partly empty, beside its fixed share, so its limit
-// there is in the time of its workgroups, T + 2 units each for T activation tiles: 1536 units (256 workgroups of four tiles,
-// one a CU; two thirds more where a row is one full round), twice that for Q6_K, whose operands cost the panel kernel as much
-// again (not at one super-block a row); past that the panel kernel. The panel kernel
+// there is in the time of its workgroups, T + 2 units each for T activation tiles: 1536 units (256 workgroups of four tiles, one
+// a CU), 2560 where all rounds are full; for Q6_K, whose operands cost the panel kernel as much again, 3072 and 4608 (not at one
+// super-block a row). Past that the panel kernel (Q6_K 3735x3072 at 171 rows and Q4_K at 96 rows, panel / split, 24.4 / 22.0, 15.0 /
+// 14.2 within the limit; the shapes above past it). The panel kernel
 // in turn loses to the tiled one on Q6_K once that fills the chip (33216x512 at 327 rows 42.8 / 49.1, 13392x256 at 459 rows 20.9 /
 // 24.0, 26064x1024 at 302 rows 45.7 / 48.4) and on Q4_K of 32768 or more outputs of under 2048 inputs (33696x256 at 39 rows 10.3 / 12.1).
 // Up to 16 rows one or two short weights stay on the small-M kernel, one pass for any of these row counts, except where a row
@@ -109,15 +111,15 @@ inline MidKernel mid_choice(int type, int in, int rows, long tiles, int count, b
     const long subs = (rows + 15) / 16, work = tiles * subs, o_tiles = (tiles + 3) / 4;
     const long split_n = (subs + 3) / 4, split_t = (subs + split_n - 1) / split_n, wide_wgs = o_tiles * ((rows + 127) / 128);
     const bool is_short = spr < 16;
-    const long units = spr == 4 ? 2560 : 1536;
-    const bool split_fits = !tall && (is_short ? tiles * split_n * (split_t + 2) <= (q6 && spr > 1 ? 2 * units : units)
-                                               : work <= (q6 ? 4096 : 2880));
+    const bool rounds_full = spr % 4 == 0;
+    const long units = q6 && spr > 1 ? (rounds_full ? 4608 : 3072) : rounds_full ? 2560 : 1536;
+    const bool split_fits = !tall && (is_short ? tiles * split_n * (split_t + 2) <= units : work <= (q6 ? 4096 : 2880));
     if (prepared && rows > 128)
         return split_fits && work <= (spr < 8 ? 1536 : is_short ? 2048 : 2560) ? MidKernel::kSplit : MidKernel::kNone;
     if (!q6 && rows > 64) {
         if (is_short && split_fits) return MidKernel::kSplit;
         int T;
-        const double panel = rows <= 512 || work <= 8192 ? panel_cost(type, in, o_tiles, subs, &T) : 1e30;
+        const double panel = rows <= 512 || work <= 8192 ? panel_cost(type, o_tiles, subs, &T) : 1e30;
         const double split = split_fits ? (in < 8192 ? 0.55 : 0.48) / 256 * (double)(tiles * split_n * split_t) : 1e30;
         const long grid64 = o_tiles * ((rows + 63) / 64);
         const double other = wide_wgs >= 448 ? 4.5 + 6.3 / 256 * (double)wide_wgs : grid64 > 512 ? 6.8 + 2.5 / 256 * (double)grid64 : 1e30;

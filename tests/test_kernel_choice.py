@@ -28,9 +28,9 @@ extern "C" int over_decode(int type, int in, int rows, long tiles, int count) {
     return ovfq::mid_over_decode(type, in, rows, tiles, count);
 }
 extern "C" int q8_mid(int in, long out, int rows) { return ovfq::q8_mid_choice(in, out, rows); }
-extern "C" int panel_tiles(int type, int in, long o_tiles, long subs) {
+extern "C" int panel_tiles(int type, long o_tiles, long subs) {
     int T;
-    ovfq::panel_cost(type, in, o_tiles, subs, &T);
+    ovfq::panel_cost(type, o_tiles, subs, &T);
     return T;
 }
 """
@@ -49,7 +49,7 @@ def rule(tmp_path_factory):
     args = [ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_long, ctypes.c_int]
     lib.choice.argtypes = lib.choice_prepared.argtypes = lib.over_decode.argtypes = args
     lib.q8_mid.argtypes = [ctypes.c_int, ctypes.c_long, ctypes.c_int]
-    lib.panel_tiles.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.c_long, ctypes.c_long]
+    lib.panel_tiles.argtypes = [ctypes.c_int, ctypes.c_long, ctypes.c_long]
     return lib
 
 
@@ -73,7 +73,7 @@ def test_split_and_panel_tests_run_what_they_name(rule, fmt):
         assert choose(rule, "q4k", k, rows, ns) == "split", (rows, k, ns)
     for rows, k, n in split.PANEL_OF_FIVE:
         assert choose(rule, "q4k", k, rows, [n]) == "panel"
-        assert rule.panel_tiles(12, k, (n + 63) // 64, (rows + 15) // 16) == 5
+        assert rule.panel_tiles(12, (n + 63) // 64, (rows + 15) // 16) == 5
 
 
 # (format, inputs, rows, outputs, the kernel that measured faster), by MI355X times of every kernel on the shape: a split
@@ -111,6 +111,13 @@ def test_prepared_weights_use_their_copy(rule, k, n, rows, kernel):
         assert rule.choice_prepared(14, k, r, (n + 15) // 16, 1) != 2
 
 
+@pytest.mark.parametrize("n,rows,height", [(2304, 512, 3), (2304, 464, 3), (3456, 512, 4), (1024, 512, 2), (3072, 416, 3),
+                                           (6144, 331, 5), (6144, 512, 4)])
+def test_panel_height_is_the_fastest(rule, n, rows, height):
+    """Q4_K tile heights that measured fastest, by more than 2 %."""
+    assert rule.panel_tiles(12, (n + 63) // 64, (rows + 15) // 16) == height
+
+
 def test_q8_0(rule):
     for rows, k, n in q8_mid.PROJECT + [(512, 32, 2040)]:
         assert not (rows <= 8 and rows * k <= 32768)  # the decode kernel
@@ -130,5 +137,5 @@ def test_bounds(rule, fmt):
         for rows in (2, 5, 17, 64, 65, 513):
             assert rule.choice(FORMATS[fmt], 1 << 26, rows, tiles, 1) == 0
         for subs in range(1, 40):
-            t = rule.panel_tiles(FORMATS[fmt], 4096, tiles, subs)
+            t = rule.panel_tiles(FORMATS[fmt], tiles, subs)
             assert 1 <= t <= (5 if fmt == "q4k" else 4) and t <= subs
