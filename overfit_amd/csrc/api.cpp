@@ -1284,12 +1284,12 @@ static int heads_impl(ovfq_ctx* ctx, int H, const ovfq_weight* const* wo, const 
     for (int r = rows < ovfq::kHeadsMaxRows ? rows : ovfq::kHeadsMaxRows; r >= 1 && !R && !mfma; r--)
         if (ovfq::q8_0_heads_supported(H, hd, r)) R = r;
     // The operand-ordered kernels where they run (up to 512 rows) where the decode kernel needs a second launch, else
-    // from 6 rows of 4096 inputs and 8 rows of 512 (MI355X, us, decode launches / these: 32 x 4096x128 at 4 / 6 / 8 / 16 rows
+    // from 6 rows of 4096 inputs and 8 rows of 512, with heads of more than one block (20 x 1341x32 at 8 rows 7.6 / 9.1) (MI355X, us, decode launches / these: 32 x 4096x128 at 4 / 6 / 8 / 16 rows
     // 10.6 / 12.4 / 18.1 / 27.0, 11.7 / 11.8 / 11.8 / 11.9; 14 x 896x64 at 6 / 8 / 9 rows 7.5 / 8.7 / 12.9, 7.8 / 7.8 / 7.8;
     // 16 x 2048x128 at 6 rows, eager calls, 8.6 / 10.0;
     // 64 x 8192x128 at 4 / 5 rows, the second in two launches, 21.2 / 36.1, 25.9 / 25.9; 4 x 128x32 at 16 rows 10.7 / 5.7).
     const bool mid = ctx->batched_kernel == OVFQ_BATCHED_AUTO && ovfq::mid_enabled() && ovfq::q8_0_mid_supported(H, hd, rows) &&
-                     (mfma || (R && (rows > R || rows >= (K >= 4096 ? 6 : K >= 512 ? 8 : 9))));
+                     (mfma || (R && (rows > R || rows >= (K >= 4096 ? 6 : K >= 512 && hd > 32 ? 8 : 9))));
     if (!R && !mfma) return fail(OVFQ_ERR_SIZE, "n_heads x head_dim (%d) too large for one launch", K);
     std::lock_guard<std::mutex> lk(ctx->mu);
     HIP_TRY(hipSetDevice(ctx->device));
@@ -1440,13 +1440,17 @@ static int moe_impl(ovfq_ctx* ctx, int E, const ovfq_weight* const* gate, const 
     // Many pairs per expert: the panel kernel over expert groups (each weight read once per 64 pairs); few: the
     // expert-stream or small-M kernel (once per 16). Measured on MI355X, us, top-2 of 8 experts, stream / panel: 4096x14336
     // experts with 12 pairs each on average 204 / 239, 16 pairs 276 / 256; 2048x4096 experts with Q6_K down 12 pairs 58 /
-    // 70, 16 pairs 82 / 76 (some experts then have more than 16, and the stream reads their weights twice).
-    static const int grouped_min = [] {
+    // 70, 16 pairs 82 / 76 (some experts then have more than 16, and the stream reads their weights twice). Where a
+    // projection is on the small-M kernel (Q6_K rows off a multiple of 8 super-blocks) from 12 already: 32 experts of
+    // 1792x2816, Q6_K, 13 pairs each 272 / 205, 16 of 3072x2304, 15 pairs 191 / 154.
+    static const int grouped_env = [] {
         const char* v = getenv("OVFQ_MOE_GROUPED_MIN_PAIRS");
         return v && *v ? atoi(v) : 16;
     }();
     // the small-M kernel keeps a row's block values in LDS (d_model, d_ff <= 16384); past that, always grouped
     const bool small_ok = ovfq::mfma_small_supported(gt, dmodel) && ovfq::mfma_small_supported(dt, dff);
+    const bool streams = ovfq::experts_stream(gt, dmodel, (int)P) && ovfq::experts_stream(dt, dff, (int)P);
+    const int grouped_min = grouped_env >= 0 ? grouped_env : streams ? 16 : 12;
     const bool grouped_big = !small_ok || ctx->batched_kernel == OVFQ_BATCHED_TILED ||
                              (ctx->batched_kernel == OVFQ_BATCHED_AUTO && P >= (size_t)grouped_min * E);
     // With more than a 64-row tile of pairs each, on average, the panel kernel's 16-row steps save little and the 64-row-tiled

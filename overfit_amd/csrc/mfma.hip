@@ -1852,15 +1852,17 @@ bool stream_pair_preferred(int type, int in, int n_rows) {
     return stream_enabled() && type == 12 && mfma_small_supported(type, in) && stream_dense_ok(2, n_rows);
 }
 
-// Whether launch_mfma_small runs this launch on the expert-stream kernel.
-static bool mfma_small_streams(int type, const GroupLaunch& L) {
-    const int nmat = L.w1 ? 2 : 1;
-    const int pairs = L.expert_off ? L.pairs : L.rows;
+bool experts_stream(int type, int in, int pairs) {
     // Q6_K blocks are DMA'd from the 16-byte boundary before them, which is the same in every row when rows are whole
     // multiples of 16 bytes (super-blocks per row a multiple of 8; Mixtral's 14336 and Llama's 4096 inputs are).
-    const bool fmt = type == 12 || (type == 14 && (L.in / kQK) % 8 == 0);
-    return stream_enabled() && fmt && (L.expert_off || stream_dense_ok(nmat, L.n_rows)) && pairs > 0 &&
-           pairs <= kStreamMaxPairs;
+    const bool fmt = type == 12 || (type == 14 && (in / kQK) % 8 == 0);
+    return stream_enabled() && fmt && pairs > 0 && pairs <= kStreamMaxPairs;
+}
+
+// Whether launch_mfma_small runs this launch on the expert-stream kernel.
+static bool mfma_small_streams(int type, const GroupLaunch& L) {
+    return experts_stream(type, L.in, L.expert_off ? L.pairs : L.rows) &&
+           (L.expert_off || stream_dense_ok(L.w1 ? 2 : 1, L.n_rows));
 }
 
 hipError_t launch_mfma_small(int type, const GroupLaunch& L, hipStream_t st) {

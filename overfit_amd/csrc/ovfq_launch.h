@@ -109,6 +109,8 @@ bool mfma_small_supported(int type, int in);
 // when it takes the small-M path.
 bool stream_pair_preferred(int type, int in, int n_rows);
 hipError_t launch_mfma_small(int type, const GroupLaunch& launch, hipStream_t st);
+// Whether launch_mfma_small runs expert groups of `pairs` pairs in all on the expert-stream kernel.
+bool experts_stream(int type, int in, int pairs);
 // MFMA-ready copy of a Q4_K / Q6_K weight: its size, and the kernel that writes it from the GGUF blocks.
 size_t mfma_prepared_bytes(int in, int out);
 hipError_t launch_mfma_prepare(int type, const uint8_t* w, int in, int out, uint8_t* pre, hipStream_t st);

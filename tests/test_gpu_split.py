@@ -177,7 +177,8 @@ def test_panel_of_five_tiles_bit_exact(orc, rows, k, n):
 
 @pytest.mark.parametrize("gate,down", [("q4k", "q4k"), ("q4k", "q6k"), ("q6k", "q6k")])
 @pytest.mark.parametrize("E,k,rows,first", [
-    (3, 2, 33, 16), (8, 3, 90, 16),  # 16 to 64 pairs an expert: panel kernel both ways
+    (4, 2, 26, 8),                   # 13 pairs an expert: panel kernel where a projection cannot stream (Q6_K)
+    (3, 2, 33, 16), (8, 3, 90, 16),  # 16 to 64: panel kernel both ways
     (6, 2, 150, 90),                 # the same, expert 0 with a second, ragged 64-row tile
     (4, 1, 300, 16),                 # 75: gate/up on the tiled kernel, down on the panel kernel
     (2, 2, 130, 16),                 # 129: Q4_K down on the tiled kernel too
