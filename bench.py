@@ -411,7 +411,7 @@ def main():
                                      for h in range(n_heads)]) for hs in sets[:4]])
         us_sep = replay_us(g, 4, 8)
         del g
-        # Prefill rows (RT/CachedMultiHeadAttention.cs:689-710): the int8-MFMA kernel (automatic from 9 rows) beside
+        # Prefill rows (RT/CachedMultiHeadAttention.cs:689-710): the int8-MFMA kernels (the automatic choice) beside
         # the decode kernel's launches of 8 rows each (forced), graph-replayed over 2 weight copies.
         prefill = {}
         for m in (9, 16, 32, 64, 512):
@@ -461,7 +461,7 @@ def main():
 
     def small_batch_line(ms=(2, 4, 8)):
         """Small batches (speculative verification, batched decode): the layer's four projection launches at M
-        rows on the automatic kernel choice (multi-row decode / small-M MFMA), graph-replayed over the copies."""
+        rows on the automatic kernel choice (multi-row decode / split / panel), graph-replayed over the copies."""
         wb = sum(weight_bytes(n, k, fmt) for _, n, k, fmt in LAYER)
         out = {"what": "Llama-3-8B layer projections (4 launches) at a few activation rows", "weight_bytes": wb,
                "timing": "HIP graph replay over %d layer copies x 4, per layer" % len(copies)}

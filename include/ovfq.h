@@ -157,11 +157,11 @@ OVFQ_API int ovfq_weight_destroy(ovfq_weight* w);
  * int8 weight operands the tiled int8-MFMA kernel otherwise rebuilds from the GGUF bytes for every
  * activation tile, plus the block scale. Batches of more than 128 rows whose weights all have it skip that build;
  * smaller ones, and those of few outputs, mostly run on kernels that build each operand once for up to 64 rows and
- * are faster than the copy. Outputs are bit-identical with or without it. Costs 8704 bytes per 16 rows and super-block (~2.5x the Q6_K bytes), freed
- * with the weight; the GGUF blocks stay resident for decode. Idempotent. For a Q4_K weight the call succeeds and
- * changes nothing (its operands are cheaper to build than to stream); other types: OVFQ_ERR_TYPE. The reference's
- * counterpart is its opt-in repacked CPU layout (RT/Q4KRepack.cs, RT/Q6KRepack.cs): a load-time layout change
- * trading memory for throughput. */
+ * are faster than the copy. Outputs are bit-identical with or without it. Costs 8704 bytes per 16 rows and
+ * super-block (~2.5x the Q6_K bytes), freed with the weight; the GGUF blocks stay resident for decode. Idempotent.
+ * For a Q4_K weight the call succeeds and changes nothing (its operands are cheaper to build than to stream); other
+ * types: OVFQ_ERR_TYPE. The reference's counterpart is its opt-in repacked CPU layout (RT/Q4KRepack.cs,
+ * RT/Q6KRepack.cs): a load-time layout change trading memory for throughput. */
 OVFQ_API int ovfq_weight_prepare_mfma(ovfq_ctx* ctx, ovfq_weight* w);
 /* Shape/format query (InputSize / OutputSize / ByteCount of the weight classes). Any out pointer may be NULL.
  * `device_blocks` receives the HBM address of the resident blocks (the quant plane for Q8_0). */
@@ -204,9 +204,12 @@ OVFQ_API int ovfq_project_dev(ovfq_ctx* ctx, const ovfq_weight* w, const float* 
 
 /* ovfq_project_dev that allocates nothing. No counterpart in the reference: it is for callers that cannot
  * allocate device memory (code under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc).
- * Same arguments and bit-identical outputs as ovfq_project_dev; where that entry point quantises the
+ * Same arguments and bit-identical outputs as ovfq_project_dev. Where that entry point quantises the
  * activation into the context's growable scratch, this one uses a fixed device array of 2.5 MiB that the
- * library holds on every GPU it runs on until the process ends. rows * input_size is limited to 2^21
+ * library holds on every GPU it runs on until the process ends, in the row-major layout of
+ * ovfq_quantize_q8k: it runs the kernels of ovfq_project_prequantized_dev, not the ones that
+ * ovfq_project_dev has for batches of a few to some hundred rows (Q6_K 4096x14336 at 24 rows 41 us
+ * against 25). rows * input_size is limited to 2^21
  * (OVFQ_NOALLOC_MAX_ELEMS; e.g. 512 rows of 4096); larger calls return OVFQ_ERR_SIZE. Every call on one GPU
  * uses that GPU's one array, through any context: calls that may overlap on a GPU (two contexts, or two
  * streams) race and must be serialised by the caller. */

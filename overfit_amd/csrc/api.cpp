@@ -444,12 +444,13 @@ int launch_projection(ovfq_ctx* c, const ovfq_weight* const* ws, int count, cons
         else
             HIP_TRY(ovfq::launch_project_split(type, jobs, count, in, rows, act, c->stream));
     } else if (type == OVFQ_TYPE_Q8_0) {
-        // The int8-MFMA kernel from 8 rows; for inputs up to 8192 from 6 rows, and from 4 rows for 8192 outputs or
-        // more. Its time is flat up to 16 rows (one 16-row tile, one-wave workgroups of 16 outputs), the row
+        // Batches that q8_mid.hip does not take (a caller's quantised activation, the fixed-scratch entry point, more than 512
+        // rows, what q8_mid_choice leaves, OVFQ_SPLIT=0). The int8-MFMA kernel from 8 rows; for inputs up to 8192 from 6 rows,
+        // and from 4 rows for 8192 outputs or more. Its time is flat up to 16 rows (one 16-row tile, one-wave workgroups of 16 outputs), the row
         // kernel's grows by a pass over the weights per row (MI355X, graph replay, us, row kernel / MFMA kernel):
         // 4096x4096 at 4 rows 21.6 / 25.7, 16 rows 63.6 / 25.8, 64 rows 235 / 46.0, 512 rows - / 52.0; 14336x4096 at
         // 4 rows 43.0 / 31.6, 16 rows 149 / 31.6; 4096x14336 at 16 rows 164 / 84.3, 24 rows 234 / 122, 512 rows - /
-        // 168. OVFQ_Q8_MFMA_MIN_ROWS sets a plain row bound instead (measurements).
+        // 168. OVFQ_Q8_MFMA_MIN_ROWS sets a plain row bound here instead (measurements).
         static const int q8_mfma_min = [] {
             const char* v = getenv("OVFQ_Q8_MFMA_MIN_ROWS");
             return v && *v ? atoi(v) : 0;
@@ -1268,10 +1269,11 @@ static int heads_impl(ovfq_ctx* ctx, int H, const ovfq_weight* const* wo, const 
     if (!host && ((rc = check_dev_align(x, "input")) || (rc = check_dev_align(y, "output")) ||
                   (rc = check_dev_align(bias, "bias"))))
         return rc;
-    // Batches from 32 rows past those that q8_mid.hip takes (below): the int8-MFMA kernel streams each head's Wo once per 16-64 activation rows; fewer rows take
-    // the decode kernel, one launch per 8 rows. MI355X, Llama-3-8B Wo (32 x 4096x128), graph replay, us, MFMA / per-8
-    // launches: 9 rows 36.9 / 19.5, 16 rows 37.6 / 28.7, 32 rows 46.4 / 47.7, 64 rows 64.7 / 89.2, 512 rows 73.3 /
-    // 628.8. OVFQ_HEADS_MFMA_MIN_ROWS sets the switch (measurements).
+    // Where q8_mid.hip does not run (`mid` below: more than 512 rows, a forced kernel, OVFQ_SPLIT=0), batches from 32 rows take the
+    // int8-MFMA kernel, which streams each head's Wo once per 16-64 activation rows, and fewer the decode kernel, one launch per
+    // 8 rows. MI355X, Llama-3-8B Wo (32 x 4096x128), graph replay, us, MFMA / per-8 launches: 9 rows 36.9 / 19.5, 16 rows 37.6 /
+    // 28.7, 32 rows 46.4 / 47.7, 64 rows 64.7 / 89.2, 512 rows 73.3 / 628.8. OVFQ_HEADS_MFMA_MIN_ROWS sets that switch
+    // (measurements, with OVFQ_SPLIT=0 below 513 rows).
     static const int heads_mfma_min = [] {
         const char* v = getenv("OVFQ_HEADS_MFMA_MIN_ROWS");
         return v && *v ? atoi(v) : 32;
@@ -1445,12 +1447,12 @@ static int moe_impl(ovfq_ctx* ctx, int E, const ovfq_weight* const* gate, const 
     // 1792x2816, Q6_K, 13 pairs each 272 / 205, 16 of 3072x2304, 15 pairs 191 / 154.
     static const int grouped_env = [] {
         const char* v = getenv("OVFQ_MOE_GROUPED_MIN_PAIRS");
-        return v && *v ? atoi(v) : 16;
+        return v && *v ? atoi(v) : -1;
     }();
-    // the small-M kernel keeps a row's block values in LDS (d_model, d_ff <= 16384); past that, always grouped
-    const bool small_ok = ovfq::mfma_small_supported(gt, dmodel) && ovfq::mfma_small_supported(dt, dff);
     const bool streams = ovfq::experts_stream(gt, dmodel, (int)P) && ovfq::experts_stream(dt, dff, (int)P);
     const int grouped_min = grouped_env >= 0 ? grouped_env : streams ? 16 : 12;
+    // the small-M kernel keeps a row's block values in LDS (d_model, d_ff <= 16384); past that, always grouped
+    const bool small_ok = ovfq::mfma_small_supported(gt, dmodel) && ovfq::mfma_small_supported(dt, dff);
     const bool grouped_big = !small_ok || ctx->batched_kernel == OVFQ_BATCHED_TILED ||
                              (ctx->batched_kernel == OVFQ_BATCHED_AUTO && P >= (size_t)grouped_min * E);
     // With more than a 64-row tile of pairs each, on average, the panel kernel's 16-row steps save little and the 64-row-tiled

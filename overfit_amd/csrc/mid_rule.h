@@ -46,14 +46,14 @@ inline bool mid_over_decode(int type, int in, int rows, long tiles, int count) {
 }
 
 // Measured on MI355X (graph replay with the quantise launch, us: the kernel chosen otherwise / split / panel):
-//   Q4_K 4096x4096       16 rows  9.7 /  8.7 / 14.3   64 rows 22.8 / 13.1 / 22.3   128 rows 23.7 / 17.9 / 23.0   192 rows 24.1 / 24.3 / 23.7
-//   Q4_K 1024x14336      64 rows 59.8 / 24.1 /   -   512 rows 69.4 / 48.4 /   -
-//   Q4_K q/k/v of 4096   16 rows 24.2 / 11.3 / 14.5   64 rows 23.9 / 18.5 / 22.9    96 rows 24.0 / 21.3 / 20.2   192 rows 32.7 / 34.7 / 31.1
-//   Q4_K 8192x8192       16 rows 21.7 / 16.8 / 24.1   64 rows 41.6 / 29.0 / 38.3    96 rows 41.8 / 39.7 / 33.2   256 rows 60.3 / 84.5 / 56.0
-//   Q4_K 14336x4096       8 rows 17.6 / 17.1 / 15.6   32 rows 23.8 / 22.4 / 17.5    64 rows 25.1 / 31.5 / 23.9   192 rows 48.8 / 69.6 / 46.6
-//   gate/up of 14336     16 rows 22.8 / 24.0 / 21.0   32 rows 45.7 / 31.6 / 23.8    64 rows 47.3 / 48.2 / 32.3   128 rows 50.6 / 87.0 / 56.1
-//   Q6_K 4096x14336      24 rows 40.0 / 23.7 / 64.2   64 rows 75.1 / 30.6 / 80.1   192 rows 92.4 / 66.2 / 81.8   384 rows  106 /  115 /  119
-//   Q6_K 14336x4096       8 rows 23.8 / 21.6 / 22.0   64 rows 37.5 / 33.8 / 29.6   160 rows 64.5 / 71.9 / 58.6   512 rows  127 /  172 /  121
+//   Q4_K 4096x4096     16 rows 10.4 /  9.5 / 14.7   64 rows 23.5 / 14.1 / 17.3  128 rows 24.1 / 18.9 / 18.2  192 rows 24.6 / 25.3 / 21.8
+//   Q4_K 1024x14336    64 rows 60.6 / 25.0 / 43.1  512 rows 69.0 / 49.4 / 51.8
+//   Q4_K q/k/v of 4096 16 rows 23.5 / 10.9 / 14.9   64 rows 23.7 / 17.3 / 17.4   96 rows 24.3 / 21.2 / 20.7  192 rows 32.7 / 35.1 / 27.0
+//   Q4_K 8192x8192     16 rows 22.0 / 17.5 / 23.6   64 rows 41.5 / 29.8 / 28.1   96 rows 42.0 / 41.6 / 34.0  256 rows 60.7 / 86.4 / 56.6
+//   Q4_K 14336x4096     8 rows 17.6 / 16.0 / 15.6   32 rows 23.8 / 21.3 / 18.1   64 rows 25.3 / 29.4 / 23.2  192 rows 49.5 / 68.5 / 47.2
+//   gate/up of 14336   16 rows 24.9 / 28.8 / 22.6   32 rows 33.8 / 35.7 / 26.0   64 rows 36.8 / 50.1 / 34.3  128 rows 51.9 / 89.9 / 59.0
+//   Q6_K 4096x14336    24 rows 41.4 / 25.1 / 63.8   64 rows 76.8 / 31.9 / 78.8  192 rows 91.7 / 69.8 / 82.5  384 rows  107 /  121 /  121
+//   Q6_K 14336x4096     8 rows 23.9 / 22.6 / 22.2   64 rows 37.9 / 34.8 / 30.0  160 rows 65.9 / 72.3 / 59.6  512 rows  129 /  172 /  124
 //   Q4_K, short inputs   9136x1280 at 59 rows 13.2 / 17.7 / 12.1   7008x2816 at 18 rows 17.6 / 12.2 / 13.7   720x1024 at 529 rows 11.9 / 10.1 / 12.3
 //   Q6_K, short inputs   5408x256 at 143 rows 9.6 / 15.5 / 8.8   912x3584 at 481 rows 30.5 / 22.3 / 28.5   4096x1536 at 251 rows 17.8 / 23.7 / 16.8
 // From 4096 inputs on: the panel kernel on tall matrices (768 16-row tiles: it then has a workgroup for nearly every CU at any
@@ -75,13 +75,13 @@ inline bool mid_over_decode(int type, int in, int rows, long tiles, int count) {
 // 96 / 192 rows 14.9 / 24.3, 1024x14336 at 400 rows 42.0); and those of mfma.hip, 4.5 + 6.3 for 256 workgroups of the wide
 // kernel (gate/up of 14336 at 128 / 256 / 512 rows 52.6 / 88.7 / 154) or 6.8 + 2.5 for 256 of the 64-row kernel, which has more
 // than two for each CU (q/k/v of 4096 at 331 / 512 rows 42.8 / 47.7, of 5120 at 331 rows 52.4; with fewer it lost to the panel
-// kernel at every size). us before / now: q/k/v of 4096 at 160 / 200 / 331 rows 30.8 / 31.5 / 42.8, 23.3 / 28.0 / 39.4; 4096x4096 at
-// 128 / 160 / 300 rows 18.2 / 23.1 / 31.9, 17.1 / 20.2 / 28.3; gate/up of 14336 at 65 / 160 rows 48.5 / 79.1, 39.6 / 71.2. Q6_K takes the
+// kernel at every size). us, otherwise / so: q/k/v of 4096 at 160 / 200 / 331 rows 32.3 / 31.4 / 43.4, 23.9 / 27.3 / 39.1; 4096x4096 at
+// 300 rows 33.0 / 28.0; gate/up of 14336 at 65 / 160 rows 49.2 / 78.7, 39.7 / 70.7. Q6_K takes the
 // panel kernel where it has a workgroup for every CU and the split kernel's work has grown, except where the pair-wide kernel
 // builds each operand once for 128 rows. Past the small-M kernel's input size (16384), and below the tiled kernel's rows (32),
-// the alternative is the general kernel (8192x28672 at 2 rows 33 / 36, 3 rows 40 / 36, 16 rows 137 / 38). Very tall matrices at 5
-// to 8 rows stay on the expert-stream kernel (128256x2048 38.5, panel 39.8), and at 3 and 4 rows, where the multi-row decode
-// kernel takes 65 and 76, only a pair does.
+// the alternative is the general kernel (8192x28672, that / split, at 2 rows 36.9 / 41.5, 3 rows 43.7 / 41.5, 16 rows 141 / 43.1). Very tall matrices at 5
+// to 8 rows stay on the expert-stream kernel (128256x2048 at 6 rows 39.4, panel 42.4), and at 3 and 4 rows, where the multi-row
+// decode kernel takes 64 (3 rows, panel 41.8), only a pair does.
 // Weights that all carry their MFMA-ready copy (`prepared`, Q6_K): the tiled kernel that reads it has no operands to build. Up
 // to 128 rows the split and panel kernels are the faster all the same (us, prepared / split / panel: 4096x14336 at 64 and 128
 // rows 77.4 / 32.2 / -, 87.8 / 49.3 / -, 14336x4096 at 64 rows 39.0 / - / 30.8, 28672x8192 at 128 rows 147 / - / 134); past that the

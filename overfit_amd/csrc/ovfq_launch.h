@@ -33,7 +33,8 @@ struct ActQ {
 // bh != NULL: the bsums are also written as fp16 (exact: |bsum| <= 16 * 127), the tiled Q4_K kernels' min-term operand.
 hipError_t launch_quantize_q8k(const float* x, int64_t n_blocks, int8_t* q, float* s, int16_t* b, hipStream_t st,
                                uint16_t* bh = nullptr);
-// Q8_K quantisation into the operand-ordered planes that launch_project_split reads for weights of `type` (12 or 14):
+// Q8_K quantisation into the operand-ordered planes that launch_project_split and launch_project_panel read for weights of `type`
+// (12 or 14):
 // for every 16 rows and super-block, kTiledQ bytes of quants, kTiledB bytes of fp16 bsums and kTiledS bytes of scales.
 // Planes cover 16 * tiled_subs(rows) rows; the rows past `rows` are not written.
 constexpr size_t kTiledQ = 4096, kTiledB = 512, kTiledS = 64;
@@ -108,9 +109,9 @@ bool mfma_small_supported(int type, int in);
 // Whether a gate/up-shaped pair of Q4_K weights (n_rows outputs each, `in` inputs) runs on the expert-stream kernel
 // when it takes the small-M path.
 bool stream_pair_preferred(int type, int in, int n_rows);
-hipError_t launch_mfma_small(int type, const GroupLaunch& launch, hipStream_t st);
 // Whether launch_mfma_small runs expert groups of `pairs` pairs in all on the expert-stream kernel.
 bool experts_stream(int type, int in, int pairs);
+hipError_t launch_mfma_small(int type, const GroupLaunch& launch, hipStream_t st);
 // MFMA-ready copy of a Q4_K / Q6_K weight: its size, and the kernel that writes it from the GGUF blocks.
 size_t mfma_prepared_bytes(int in, int out);
 hipError_t launch_mfma_prepare(int type, const uint8_t* w, int in, int out, uint8_t* pre, hipStream_t st);

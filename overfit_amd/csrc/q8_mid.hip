@@ -160,8 +160,10 @@ struct Q8Cursor {
 // ------------------------------------------------------------------------------------------ panel kernel
 // 64 outputs (16 a wave) x 16 T rows a workgroup, the groups in ascending order, the sums in registers. The activation
 // (shared by the four waves) and each wave's weights are DMA'd two steps ahead; the one wait of a step leaves the next step's in
-// flight. Bound by the block values' three vector operations: of 42.8 us at 4096x4096 and 512 rows some 6 go to the quantise
-// launch and 30 are left with the DMAs taken out. Eight waves a workgroup, each with half the rows, were no faster (512 rows
+// flight. Bound by the block values' three vector operations beside the matrix work: with heads of 32 x 4096x128 at 300 rows (33.8
+// us, T = 3) vector instructions issue 65 % of the time and the matrix units work 23 %, a third of it beside them, with 1.6 waves a
+// SIMD (a conversion takes twice the issue of a multiplication or addition: 60 against 111 lanes a clock and CU). 4096x4096 at 512
+// rows, 40.3 us: 30 were left with the DMAs taken out. Eight waves a workgroup, each with half the rows, were no faster (512 rows
 // 43.4; 64 rows 20.6 instead of 19.5), nor were more groups in flight.
 // J: blocks of a group that are computed (planes of fewer than four blocks).
 template <int T, bool kHeads, int J = 4>
