@@ -444,13 +444,13 @@ int launch_projection(ovfq_ctx* c, const ovfq_weight* const* ws, int count, cons
         else
             HIP_TRY(ovfq::launch_project_split(type, jobs, count, in, rows, act, c->stream));
     } else if (type == OVFQ_TYPE_Q8_0) {
-        // Batches that q8_mid.hip does not take (a caller's quantised activation, the fixed-scratch entry point, more than 512
-        // rows, what q8_mid_choice leaves, OVFQ_SPLIT=0). The int8-MFMA kernel from 8 rows; for inputs up to 8192 from 6 rows,
-        // and from 4 rows for 8192 outputs or more. Its time is flat up to 16 rows (one 16-row tile, one-wave workgroups of 16 outputs), the row
-        // kernel's grows by a pass over the weights per row (MI355X, graph replay, us, row kernel / MFMA kernel):
-        // 4096x4096 at 4 rows 21.6 / 25.7, 16 rows 63.6 / 25.8, 64 rows 235 / 46.0, 512 rows - / 52.0; 14336x4096 at
-        // 4 rows 43.0 / 31.6, 16 rows 149 / 31.6; 4096x14336 at 16 rows 164 / 84.3, 24 rows 234 / 122, 512 rows - /
-        // 168. OVFQ_Q8_MFMA_MIN_ROWS sets a plain row bound here instead (measurements).
+        // Batches that q8_mid.hip does not take (a caller's quantised activation, the fixed-scratch entry point, more than
+        // 512 rows, what q8_mid_choice leaves, OVFQ_SPLIT=0). The int8-MFMA kernel from 8 rows; for inputs up to 8192 from 6
+        // rows, and from 4 rows for 8192 outputs or more. Its time is flat up to 16 rows (one 16-row tile, one-wave
+        // workgroups of 16 outputs), the row kernel's grows by a pass over the weights per row (MI355X, graph replay, us, row
+        // kernel / MFMA kernel): 4096x4096 at 4 rows 21.6 / 25.7, 16 rows 63.6 / 25.8, 64 rows 235 / 46.0, 512 rows - / 52.0;
+        // 14336x4096 at 4 rows 43.0 / 31.6, 16 rows 149 / 31.6; 4096x14336 at 16 rows 164 / 84.3, 24 rows 234 / 122, 512 rows
+        // - / 168. OVFQ_Q8_MFMA_MIN_ROWS sets a plain row bound here instead (measurements).
         static const int q8_mfma_min = [] {
             const char* v = getenv("OVFQ_Q8_MFMA_MIN_ROWS");
             return v && *v ? atoi(v) : 0;

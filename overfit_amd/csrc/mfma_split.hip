@@ -332,19 +332,19 @@ static hipError_t launch_split_w(int type, const PArgs& pa, int T, hipStream_t s
 }
 
 // ------------------------------------------------------------------------------------------ panel kernel
-// Tall matrices and expert groups, 16 to 80 rows a workgroup (64 in groups): there are workgroups enough without splitting the contraction, but
-// the 64-row-tiled kernel of mfma.hip waited for every load of the next super-block before the barrier of each one, so a
-// super-block took a memory latency (1.8 us a step, whatever the rows). Here a workgroup's four waves own 16 weight rows
-// each against the same 16 T activation rows and walk the super-blocks in order, the sums in registers. A step's activation
-// tile is DMA'd into LDS one step ahead, each wave's weights two steps ahead into a ring of its own (mfma_split's slots),
-// and the one wait of a step leaves the weights of the next in flight. Rows are taken 16 at a time: 45 rows cost three tiles,
-// not 64 or 128 rows.
+// Tall matrices and expert groups, 16 to 80 rows a workgroup (64 in groups): there are workgroups enough without splitting
+// the contraction, but the 64-row-tiled kernel of mfma.hip waited for every load of the next super-block before the barrier
+// of each one, so a super-block took a memory latency (1.8 us a step, whatever the rows). Here a workgroup's four waves own
+// 16 weight rows each against the same 16 T activation rows and walk the super-blocks in order, the sums in registers. A
+// step's activation tile is DMA'd into LDS one step ahead, each wave's weights two steps ahead into a ring of its own
+// (mfma_split's slots), and the one wait of a step leaves the weights of the next in flight. Rows are taken 16 at a time: 45
+// rows cost three tiles, not 64 or 128 rows.
 // At 16 rows of gate/up (2 x 14336x4096, 66 MB) it is near the weights' stream (17 us beside the quantise launch); every 16
-// rows more add 4 us. Past that it waits as much as it computes: at 45 rows (T = 3, 25.2 us) vector instructions issue 50 % of
-// the time and the matrix units work 23 %, a third of it beside them, with 1.5 waves a SIMD; q/k/v of 4096 at 331 rows (T = 5,
-// 36.8 us) 53 and 30 %; gathered expert groups of 40 pairs 54 and 24 %. us with the quantise launch, before / after: 32 rows
-// 33.8 / 26.0, 64 rows 36.8 / 34.3; Q6_K 14336x4096 at 64 rows 37.9 / 30.0; 8 experts of 48 pairs on average, 4096x7168, Q6_K, gate/up
-// 156 / 138, down 115 / 71, Q4_K 106 / 118 and 75 / 55.
+// rows more add 4 us. Past that it waits as much as it computes: at 45 rows (T = 3, 25.2 us) vector instructions issue 50 %
+// of the time and the matrix units work 23 %, a third of it beside them, with 1.5 waves a SIMD; q/k/v of 4096 at 331 rows (T
+// = 5, 36.8 us) 53 and 30 %; gathered expert groups of 40 pairs 54 and 24 %. us with the quantise launch, before / after: 32
+// rows 33.8 / 26.0, 64 rows 36.8 / 34.3; Q6_K 14336x4096 at 64 rows 37.9 / 30.0; 8 experts of 48 pairs on average, 4096x7168,
+// Q6_K, gate/up 156 / 138, down 115 / 71, Q4_K 106 / 118 and 75 / 55.
 struct PanelGroup {
     const uint8_t* w0[kMaxExperts];
     const uint8_t* w1[kMaxExperts];

@@ -114,12 +114,12 @@ def test_prepared_weight_keeps_the_kernel_that_reads_its_copy(orc):
 
 
 @pytest.mark.parametrize("down", ["q4k", "q6k"])
-def test_split_ffn_intermediate_matches_separate_calls(down):
+@pytest.mark.parametrize("d,ff,rows", [(512, 2304, 35), (8960, 1280, 59)])  # down on the split kernel, on the panel kernel
+def test_ffn_intermediate_matches_separate_calls(down, d, ff, rows):
     """The FFN's intermediate, quantised in the down kernel's operand order, against the same FFN with another kernel
-    forced, which reads it row by row: the same quants, so the same bits (35 rows, 9 super-blocks)."""
-    case("split ffn", down)
+    forced, which reads it row by row: the same quants, so the same bits."""
+    case("ffn", down, d, ff, rows)
     rng = np.random.default_rng(5)
-    d, ff, rows = 512, 2304, 35
     gate, up = _weight(rng, "q4k", ff, d)[1], _weight(rng, "q4k", ff, d)[1]
     w = _weight(rng, down, d, ff)[1]
     x = t(normal(rng, (rows, d), 0.02))
@@ -139,6 +139,7 @@ PANEL = [
     (48, 768, [6200, 6200]),     # an odd number of super-blocks, a gate/up pair
     (64, 512, [12288]),          # four full tiles
     (70, 1280, [4096, 512, 520]),  # not tall: two activation tiles of three, the last rows absent
+    (59, 1280, [9130]),          # not tall, one activation tile of four, an odd number of short super-blocks
     (150, 768, [14330]),           # three activation tiles of four, the last of two and ragged; the last weight rows absent
     (250, 1280, [4000, 520]),      # four of four, an odd number of 210-byte blocks a row
 ]
